@@ -268,9 +268,10 @@ int xt_prec_refactor_band(xt_prec pr, const int *rowptr, const int *colidx,
                           const double *vals, void *stream);
 /* xt_prec_refactor_band for a K that changed only in rows and columns >= first_row
  * (0-based; the caller guarantees it, e.g. the DOFs of deleted elements and of the nodes
- * they orphan): the factor's blocks before first_row / block are kept and the rest, with
- * the recurrence and pairing matrices that depend on them, recomputed from the kept
- * D_{j-1} and K (equal to a full refactorization up to rounding).  A factor kept in FP32
+ * they orphan).  The factor eliminates the blocks from both ends towards the middle one:
+ * of the top half the blocks before first_row / block are kept, the rest is recomputed
+ * from the kept D_{j-1} and K with the recurrence and pairing matrices that depend on it
+ * (equal to a full refactorization up to rounding).  A factor kept in FP32
  * only is refactored whole.  Plain banded factors only (no shifted or grouped factors).
  * Replaces the refactorization after element deletion, mumps_solver(job = 1),
  * main3d.f90:687. */
@@ -487,7 +488,7 @@ int xt_prof_read(int kind, double *ms, long long *launches, double *bytes, doubl
  * products of their recurrences); for the other kinds it equals xt_prof_read's. */
 int xt_prof_read_alg(int kind, double *bytes, double *flops);
 
-/* Replay the banded factor's sweeps (2 + 2 (nb - 1) launches of fixed buffers) from a
+/* Replay the banded factor's sweeps (a fixed sequence of launches on fixed buffers) from a
  * HIP graph captured on first use per column count and precision (on = 1, the
  * default), or launch them one by one (0).  No counterpart in the reference (launch
  * overhead control).  Process-wide. */
@@ -506,10 +507,8 @@ int xt_graphs_enable(int on);
  *   XT_TUNE_SPMM_LDS      node-block SpMM, several load cases: the LDS-staged kernel
  *                         (neighbour rows of X staged per slice) off 1, on 2 (where the
  *                         neighbour rows fit), built-in: off
- *   XT_TUNE_BAND_SMALLC   banded-factor sweeps with at most 16 columns: VALU rows kernel 1,
- *                         matrix-core kernels with 64-column tiles in batched passes 2,
- *                         with 16-column tiles 3; built-in: rows kernel below 1024-row
- *                         blocks (FP32) or 512-row blocks (FP64), else 3    1, 2, 3
+ *   XT_TUNE_BAND_SMALLC   banded-factor sweeps with at most 16 columns: 16 rows a workgroup
+ *                         1, 32 rows 2, by the number of workgroups 3 (built-in 3)  1, 2, 3
  *   XT_TUNE_IR_FP32_CYCLE GMRES-IR: iterations an FP32 inner cycle gets to meet its target
  *                         before the case moves to FP64 cycles              1, 2, 4, 8
  *                         (built-in 2)
@@ -523,21 +522,22 @@ int xt_graphs_enable(int on);
  *                         then again; 1: FP32 cycles first always           1, 4, 16, 64
  *                         (built-in 16)
  *   XT_TUNE_BAND_CHAIN    banded-factor sweeps, the dependent chain steps with more than
- *                         16 columns: one workgroup per 16 x 16 output tile 1, 64 x 64
- *                         tiles split over k into about 512 / 256 / 1024 workgroups with
- *                         a fixed-order sum 2 / 3 / 4 (built-in 4)          1, 2, 3, 4
+ *                         16 columns, output tile of a workgroup: 16 x 16 1, 32 rows by 32
+ *                         or 48 columns 2, 16 rows by 32 or 48 columns 3, the one that
+ *                         fills the CUs best 4 (built-in 4)                 1, 2, 3, 4
  *   XT_TUNE_BAND_LEVELS   banded factor: pairing levels of the block recurrences at most
- *                         v - 1 (read when a factor is built; built-in 4)   1, 2, 3, 5
+ *                         v - 1 (read when a factor is built; built-in: as many as pay for
+ *                         few columns, 4 at most)                           1, 2, 3, 5
  *   XT_TUNE_GMRES_REORTH  Arnoldi orthogonalisation: classical Gram-Schmidt twice always
  *                         1, the second pass only where the first lost more than half of
  *                         |w|^2 for some instance 2 (built-in 2)            1, 2
  *   XT_TUNE_GMRES_COMPACT banded-factor sweeps of a batched solve over the load cases still
  *                         iterating in the cycle only 2, over all 1 (built-in 2)   1, 2
- *   XT_TUNE_BAND_CHAIN_FEW as XT_TUNE_BAND_CHAIN for chain steps with at most 16 columns on
- *                         the matrix cores: one 16 x 16 tile per workgroup 1, split-k 64 x
- *                         64 tiles 2 (built-in 1)                            1, 2
+ *   XT_TUNE_BAND_CHAIN_FEW banded-factor sweeps, 16-row workgroups with at most 16 columns:
+ *                         the k range over 8 waves 1, 4 waves 2 (built-in 1)  1, 2
  *   XT_TUNE_BAND_PAIR     banded-factor sweeps: the factor's pairing levels never 1,
- *                         always 2 (built-in: FP32 always, FP64 up to 64 columns)   1, 2
+ *                         always 2 (built-in: the levels with the least estimated time for
+ *                         the columns)                                      1, 2
  * XT_E_ARG for a value a knob does not take. */
 #define XT_TUNE_SPMM_UNR 0
 #define XT_TUNE_SPMM_WPB 1

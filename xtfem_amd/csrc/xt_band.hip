@@ -3,25 +3,35 @@
 // The reference's live solver preconditions GMRES with the exact factor of K (MUMPS
 // LDL^T of the lower triangle, mumps.f90:22-145, applied to all q temporal blocks by
 // mpilusol, kronecker_mumps.f90:120-183).  ILUT with lfil >= n and droptol = 0 is the
-// same exact factor (ilut.f:2169-2170).  Here K (bandwidth w after the mesh numbering)
-// is cut into nb diagonal blocks of b >= w rows, so it is block tridiagonal:
+// same exact factor (ilut.f:2169-2170).  Here K (half-bandwidth w after the mesh
+// numbering) is cut into nb diagonal blocks of b >= w rows, so it is block tridiagonal,
+// and eliminated from both ends towards a middle block ("twisted" block Cholesky, FP64,
+// device): the first nt blocks top down, the last nbt blocks bottom up, the middle block
+// last.  The two eliminations are independent of each other, so every dependent step of
+// the factorization and of the sweeps works on two blocks at once and there are half as
+// many of them, with the operations of the one-sided factor.
 //
-//   K = L L^T,  L = blockbidiag(L_ii, E_i = L_{i+1,i})     (block Cholesky, FP64, device)
+// The bottom blocks are held with their rows reversed (row r of the factor's order is row
+// nb b - 1 - r of K from the last row back), which makes the bottom chain the same
+// computation as the top one: block i of a chain with its sub-diagonal block
+// E_i = K_{i+1,i} L_ii^-T, D_i = L_ii^-1 and
 //
-// With D_i = L_ii^-1 the two triangular solves become dense block recurrences
+//   forward   y_0 = D_0 x_0,   y_{i+1} = D_{i+1} x_{i+1} - G_i y_i,   G_i = D_{i+1} E_i
+//   middle    y_m = D_m x_m - G_top y_top - G_bot y_bot,   z_m = D_m^T y_m
+//   backward  z_i = D_i^T y_i - H_i z_{i+1},   H_i = (E_i D_i)^T
 //
-//   forward   y_0 = D_0 x_0,      y_{i+1} = D_{i+1} x_{i+1} - G_i y_i,   G_i = D_{i+1} E_i
-//   backward  z_nb = D^T y,       z_i     = D_i^T y_i     - H_i z_{i+1}, H_i = (E_i D_i)^T
-//
-// The D x and D^T y products of all blocks run in one batched launch.  A recurrence
-// w_v -= M_v w_{v-1} (v = 1..m, m = nb - 1; M_v = G_{v-1} forward, and H in reverse
-// block order backward) advances 2^L blocks per dependent step: pairing two steps,
+// E_i couples only the last w columns of block i with the first w rows of block i + 1, so
+// G_i has w nonzero columns (the last) and H_i too (the first): both are stored b x kw,
+// kw = w rounded up.  The D x and D^T y products of all blocks run in one batched launch.
+// A recurrence w_v -= M_v w_{v-1} (v = 1..m) advances 2^L blocks per dependent step:
+// pairing two steps,
 //   w_v -= M_v w_{v-1}  for even v            (one batched launch: the new right-hand sides)
 //   w_v -= M'_v w_{v-2} for v = 2, 4, .. in order,   M'_v = -M_v M_{v-1}
 //   w_v -= M_v w_{v-1}  for odd v             (one batched launch: the blocks between)
 // and the middle line is again such a recurrence over every second block, paired in
-// turn for L levels.  The level matrices are formed once per factorization; the
-// dependent chain shrinks from m launches to m / 2^L plus 2 L batched launches.
+// turn for L levels.  The level matrices are formed once per factorization.  Where the
+// blocks are at least twice the band (rc < b below), the chain runs on the kw rows the
+// next block reads only, and one batched launch finishes the other rows.
 // All matrix sets are stored row-major (the row of the operator a tile needs is
 // contiguous) in FP64 and FP32.
 //
@@ -41,31 +51,34 @@
 
 namespace xt {
 
-// The sweeps of one apply are a fixed sequence of 2 + 2 (nb - 1) launches on fixed
-// buffers for a given column count and precision: captured once into a HIP graph and
-// replayed, they skip the per-launch host overhead.  Keyed on every pointer the
-// launches use, so a refactorization or a grown workspace captures anew.
+// The sweeps of one apply are a fixed sequence of launches on fixed buffers for a given
+// column count and precision: captured once into a HIP graph and replayed, they skip the
+// per-launch host overhead.  Keyed on every pointer the launches use, so a
+// refactorization or a grown workspace captures anew.
 constexpr int kLevels = 4;     // pairing levels of the block recurrences, at most
-constexpr int kMinChain = 6;   // a level is added while its chain keeps this many steps
+constexpr int kMinChain = 3;   // a level is added while its chain keeps this many steps
 constexpr int kKey = 6 + 2 * kLevels;
 struct SweepGraph {
-    int c = 0, pi = -1, tile = 0, smallc = 0, nl = 0;   // columns, precision, knobs,
-    long long epoch = -1;                                // levels used, knob epoch
+    int c = 0, pi = -1, nl = 0;                          // columns, precision, levels used,
+    long long epoch = -1;                                // knob epoch
     const void *key[kKey] = {};
     hipGraphExec_t exec = nullptr;
 };
 
 struct BandPrec {
     int p = 0, b = 0, nb = 0, bw = 0;
-    // [.][0] FP64, [.][1] FP32.  Dl: D_i row-major (lower), Du: D_i^T row-major (upper),
-    // G, H: recurrence matrices (nb - 1 of each); Lv[dir][L - 1]: the level-L matrices of
-    // the forward (0) and backward (1) recurrence, (nb - 1) >> L of them in chain order.
+    int nt = 0, nbt = 0;         // blocks of the top and of the bottom chain (+ the middle)
+    int kw = 0, rc = 0;          // columns of G and H; rows the chains run on (kw or b)
+    // [.][0] FP64, [.][1] FP32.  Blocks in the factor's order (top chain, middle, bottom
+    // chain).  Dl: D_i row-major (lower), Du: D_i^T row-major (upper).  G, H: the
+    // top chain's nt, then the bottom chain's nbt.  Lv[dir][L - 1]: the level-L matrices
+    // (rc x kw) of the forward (0) and backward (1) recurrence, the top chain's
+    // steps(0, dir) >> L, then the bottom chain's (order: level_view).
     DevBuf Dl[2], Du[2], G[2], H[2];
     DevBuf Lv[2][kLevels][2];
     int nlev = 0;
     bool keep64 = true;          // false: the FP64 sets are released after the FP32 copies
     DevBuf w1, w2;
-    DevBuf part;                 // partial products of the split-k chain steps
     SweepGraph graph[4];
     int next_graph = 0;
     hipStream_t cap = nullptr;   // capture stream (non-blocking, default priority)
@@ -77,134 +90,34 @@ struct BandPrec {
             if (g.exec) (void)hipGraphExecDestroy(g.exec);
         if (cap) (void)hipStreamDestroy(cap);
     }
+    int blocks(int side) const { return side == 0 ? nt : nbt; }
+    // steps of a chain's recurrence: forward over its blocks, backward from the middle
+    int steps(int side, int dir) const {
+        const int n = blocks(side);
+        return dir == 0 ? std::max(0, n - 1) : n;
+    }
 };
 
 // ---------------------------------------------------------------------------
-// Block products of the sweeps:
-//   out_blk[r][col] = (add ? add_blk[r][col] - s : s),  s = sum_k A_blk[r][k] V_blk[k][col]
-// A_blk: b x b row-major; V, add, out: b x c row-major (c columns of one row contiguous).
+// Block products of the sweeps, batched over items z:
+//   O_z = A_z V_z   or   O_z -= A_z V_z
+// A_z: rows x kdim row-major (row stride lda); V_z, O_z: row-major with ld columns (a
+// multiple of 16; the columns past the vectors' own are never read back).  Items z < n0 are the
+// first chain's, A_z = A[0] + z as[0] and so on, the others the second chain's.
 // tri = 1: A lower triangular (k <= r), tri = 2: upper (k >= r); the stored zeros of
-// the other triangle are skipped where a whole tile lies there.  Grid z runs over the
-// blocks of a batch (a_stride, v_stride, ... between consecutive blocks).
+// the other triangle are skipped where a whole tile lies there.
 // ---------------------------------------------------------------------------
+template <typename T>
+struct Items {
+    const T *A[2], *V[2];
+    T *O[2];
+    long long as[2], vs[2], os[2];
+    int n0, n;
+    // rows dup0.. of item dupz are also written to dup (NULL: none)
+    T *dup = nullptr;
+    int dupz = 0, dup0 = 0;
+};
 
-// Few columns (c <= CM <= 16, V block in LDS): a workgroup owns RW rows.  It first
-// copies the rows k0..k1-1 of V (one contiguous span) into LDS with 16-byte loads;
-// its 256 threads then stride over k, loading the RW A rows (coalesced, every load
-// of a group of GK k issued before the products, indices clamped and out-of-range
-// terms multiplied by zero) and reading V from LDS.  The RW * CM <= 16 partial sums
-// of the 256 threads are summed through LDS: 16 threads per output add 16 partials
-// each, then a 16-lane butterfly (one value per lane).  Grid x = b / RW.
-constexpr size_t kRowsLdsMax = 96 * 1024;
-constexpr int kRowsMaxB = 1024;   // block rows from which few columns go to matrix cores
-constexpr int kRowsMaxB64 = 512;  // the same in FP64 (768-row blocks, 6-16 columns: the
-                                  // matrix-core sweeps took a plate step from 49.7 to 38 ms)
-constexpr bool kChainSplitDefault = true;    // chain steps as split-k tile products
-constexpr bool kChainSplitFewDefault = false;   // the same with at most 16 columns
-// Columns up to which the FP64 sweeps use the factor's pairing levels (the 1856-row panel
-// factor: pairing 11.6 vs 14.5 ms per apply at 48 columns, 20.7 vs 18.4 at 72, 31.0 vs
-// 27.6 at 192); FP32 sweeps use them at every width (16.1 vs 17.5 ms at 192).
-constexpr int kPairMaxC64 = 64;
-// Batched passes with at most 16 columns on 16 x 16 tiles instead of 64 x 64 ones (the
-// panel factor at one load case: FP64 apply 11.3 -> 8.0 ms, FP32 6.0 -> 4.6 ms).
-constexpr bool kSmallcMfmaBatched = true;
-
-template <typename T, int CM, int RW>
-__global__ void __launch_bounds__(256)
-band_rows_kernel(int b, int c, int tri, const T *__restrict__ A, long long a_stride,
-                 const T *__restrict__ V, long long v_stride, const T *add, long long add_stride,
-                 T *out, long long out_stride) {
-    constexpr int VEC = 16 / sizeof(T);
-    typedef T vec_t __attribute__((ext_vector_type(VEC)));
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    static_assert(RW * CM <= 16, "at most 16 outputs per workgroup");
-    T *Vsh = reinterpret_cast<T *>(smem_raw);   // [k1 - k0][c]
-    __shared__ T red[16][256];                   // [output][thread]
-    const int tid = threadIdx.x;
-    const int r0 = blockIdx.x * RW;
-    const long long z = blockIdx.z;
-    A += z * a_stride;
-    V += z * v_stride;
-    out += z * out_stride;
-    if (add) add += z * add_stride;
-    int k0 = 0, k1 = b;
-    if (tri == 1) k1 = r0 + RW;
-    if (tri == 2) k0 = r0;
-    {
-        const int n = (k1 - k0) * c;
-        const T *src = V + (size_t)k0 * c;
-        if ((((size_t)k0 * c) % VEC) == 0 && (n % VEC) == 0) {
-            for (int e = tid; e < n / VEC; e += 256)
-                *reinterpret_cast<vec_t *>(Vsh + (size_t)e * VEC) =
-                    *reinterpret_cast<const vec_t *>(src + (size_t)e * VEC);
-        } else {
-            for (int e = tid; e < n; e += 256) Vsh[e] = src[e];
-        }
-    }
-    __syncthreads();
-    T acc[RW][CM];
-#pragma unroll
-    for (int rr = 0; rr < RW; ++rr)
-#pragma unroll
-        for (int j = 0; j < CM; ++j) acc[rr][j] = T(0);
-    const T *a0 = A + (size_t)r0 * b;
-    constexpr int GK = RW >= 8 ? 2 : 4;
-    for (int kb = k0; kb < k1; kb += GK * 256) {
-        T av[GK][RW];
-#pragma unroll
-        for (int it = 0; it < GK; ++it) {
-            const int kk = min(kb + tid + 256 * it, k1 - 1);
-#pragma unroll
-            for (int rr = 0; rr < RW; ++rr) av[it][rr] = a0[(size_t)rr * b + kk];
-        }
-#pragma unroll
-        for (int it = 0; it < GK; ++it) {
-            const int k = kb + tid + 256 * it;
-            const int kk = min(k, k1 - 1);
-            const T m = (k < k1) ? T(1) : T(0);
-            T vv[CM];
-#pragma unroll
-            for (int j = 0; j < CM; ++j) vv[j] = Vsh[(kk - k0) * c + min(j, c - 1)];
-#pragma unroll
-            for (int rr = 0; rr < RW; ++rr) {
-                const T a = av[it][rr] * m;
-#pragma unroll
-                for (int j = 0; j < CM; ++j) acc[rr][j] = fma(a, vv[j], acc[rr][j]);
-            }
-        }
-    }
-#pragma unroll
-    for (int rr = 0; rr < RW; ++rr)
-#pragma unroll
-        for (int j = 0; j < CM; ++j) red[rr * CM + j][tid] = acc[rr][j];
-    __syncthreads();
-    {
-        const int o = tid >> 4, part = tid & 15;   // output o, partials part + 16 i
-        T sum = T(0);
-        if (o < RW * CM) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) sum += red[o][part + 16 * i];
-        }
-#pragma unroll
-        for (int off = 8; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 16);
-        const int rr = o / CM, j = o - rr * CM;
-        if (part == 0 && o < RW * CM && j < c) {
-            const size_t idx = (size_t)(r0 + rr) * c + j;
-            out[idx] = add ? add[idx] - sum : sum;
-        }
-    }
-}
-
-// Many columns (c > 16) on the matrix cores: a workgroup computes one 16 x 16 output
-// tile; its 4 waves split the k range into quarters (whole chunks) and each runs
-// v_mfma_*_16x16x4 steps over its quarter; the 4 partial tiles are summed through
-// LDS in a fixed order (deterministic, one launch).  Lane l = 16 g + t feeds row t of
-// A and column t of V; the k index of a step is assigned per lane group g (group g
-// holds KG consecutive k of each chunk of 4 KG, loaded as one vector), which any
-// order of the k sum allows, so A rows are read with vector loads.  Operands come
-// straight from global memory (L2), UNR chunks of loads in flight per pass.  Output
-// layout of the 4 accumulators per lane: f32 row 4 g + i, f64 row g + 4 i, column t.
-// Grid x = b / 16, y = ceil(c / 16), z = blocks of the batch.
 typedef float xt_f4m __attribute__((ext_vector_type(4)));
 typedef double xt_d4m __attribute__((ext_vector_type(4)));
 
@@ -213,7 +126,6 @@ struct Mfma;
 template <>
 struct Mfma<float> {
     typedef xt_f4m acc_t;
-    static constexpr int KG = 4, UNR = 4;
     __device__ static acc_t step(float a, float b, acc_t c) {
         return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
     }
@@ -222,97 +134,172 @@ struct Mfma<float> {
 template <>
 struct Mfma<double> {
     typedef xt_d4m acc_t;
-    static constexpr int KG = 2, UNR = 8;
     __device__ static acc_t step(double a, double b, acc_t c) {
         return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
     }
     __device__ static int row(int g, int i) { return g + 4 * i; }
 };
 
-template <typename T>
-__global__ void __launch_bounds__(256)
-band_mfma_kernel(int b, int c, int tri, const T *__restrict__ A, long long a_stride,
-                 const T *__restrict__ V, long long v_stride, const T *add, long long add_stride,
-                 T *out, long long out_stride) {
+// Tile t = (w % 8) (grid / 8) + w / 8 of workgroup w: workgroups are dealt to the 8 XCDs
+// round-robin, so each XCD gets a contiguous run of tiles (the grid is a multiple of 8).
+__device__ __forceinline__ long long xcd_tile() {
+    return (long long)(blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
+}
+
+// Dependent steps and few-column passes: a workgroup computes a (16 RT) x (16 CT) output
+// tile; its KW waves split the k range (whole chunks of 16) and their partial tiles are
+// summed through LDS in a fixed order (deterministic, one launch, no partials in
+// memory).  Each wave reads its operands straight from global memory into registers, PF
+// chunks ahead of the products and with no barrier in the loop: one FP64 matrix-core
+// step takes 64 cycles a SIMD, so RT CT of them cover the loads of a chunk; what bounds
+// a step is the latency of the first loads and of the launch.
+// Lane l = 16 g + t holds A[row t][4 g + s] and V[4 g + s][column t] in step s of a chunk
+// (any assignment of k to lane groups gives the same sum): A rows are read 32 or 16
+// bytes a lane, 128 contiguous bytes a row; column tiles go in pairs, lane t taking
+// columns 2 t and 2 t + 1 of the 32.  Output layout of the 4 accumulators per lane: f32
+// row 4 g + i, f64 row g + 4 i.
+// nseg = 2: one item whose product is A[0] V[0] + A[1] V[1], half the waves each.
+// Consecutive tiles are the column tiles of one row tile, so one XCD's L2 serves its A.
+template <typename T, int RT, int CT, int KW, int PF>
+__global__ void __launch_bounds__(64 * KW)
+band_prod_kernel(Items<T> it, int rows, int lda, int kdim, int tri, int ld, int sub, int nseg) {
     using M = Mfma<T>;
-    constexpr int KG = M::KG, CH = 4 * KG, UNR = M::UNR;
-    typedef T vec_t __attribute__((ext_vector_type(KG)));
-    __shared__ T red[3][64][4];
+    using acc_t = typename M::acc_t;
+    constexpr int AV = 16 / sizeof(T);              // elements of a 16-byte load
+    typedef T avec __attribute__((ext_vector_type(AV)));
+    typedef T vpair __attribute__((ext_vector_type(2)));
+    constexpr int CP = CT / 2;                      // column-tile pairs
+    __shared__ T red[KW][RT * CT][4][64];
+    const int ntx = rows / (16 * RT), nty = ld / (16 * CT);
+    const long long tile = xcd_tile();
+    if (tile >= (long long)ntx * nty * it.n) return;
+    const int z = (int)(tile / (ntx * nty)), rem = (int)(tile - (long long)z * ntx * nty);
+    const int r0 = rem / nty * (16 * RT), n0 = rem % nty * (16 * CT);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int g = lane >> 4, t = lane & 15;
-    const int r0 = blockIdx.x * 16, n0 = blockIdx.y * 16;
-    const long long z = blockIdx.z;
-    A += z * a_stride;
-    V += z * v_stride;
-    out += z * out_stride;
-    if (add) add += z * add_stride;
-    int k0 = 0, k1 = b;
-    if (tri == 1) k1 = r0 + 16;
+    const int sd = z < it.n0 ? 0 : 1, zi = sd ? z - it.n0 : z;
+    const int parts = KW / nseg, part = wave % parts, sg = nseg == 2 ? wave / parts : sd;
+    const T *A = it.A[sg] + (nseg == 2 ? 0 : zi * it.as[sg]);
+    const T *V = it.V[sg] + (nseg == 2 ? 0 : zi * it.vs[sg]);
+    T *O = it.O[sd] + zi * it.os[sd];
+    int k0 = 0, k1 = kdim;
+    if (tri == 1) k1 = r0 + 16 * RT;
     if (tri == 2) k0 = r0;
-    // this wave's quarter of [k0, k1), in whole chunks
-    const int per = ((k1 - k0) / CH + 3) / 4 * CH;
-    const int kw0 = k0 + wave * per, kw1 = min(k1, kw0 + per);
-    const T *arow = A + (size_t)(r0 + t) * b;
-    const int cc = min(n0 + t, c - 1);
-    typename M::acc_t acc = {T(0), T(0), T(0), T(0)};
-    for (int kc = kw0; kc < kw1; kc += CH * UNR) {
-        vec_t ra[UNR];
-        T rb[UNR][KG];
+    const int nch = (k1 - k0) >> 4;                 // chunks; this wave's: c0 .. c0 + n - 1
+    const int c0 = nch * part / parts, n = nch * (part + 1) / parts - c0;
+    const T *ap = A + (size_t)(r0 + t) * lda + k0 + 16 * c0 + 4 * g;
+    const T *vp = V + (size_t)(k0 + 16 * c0 + 4 * g) * ld + n0 + (CP ? 2 * t : t);
+    const T *vq = V + (size_t)(k0 + 16 * c0 + 4 * g) * ld + n0 + 32 * CP + t;   // odd last tile
+    // output unit u (accumulator e of 16 x 16 tile tl): summed and stored by wave u % KW,
+    // whose old values are loaded ahead of the products
+    constexpr int NU = RT * CT * 4, UW = (NU + KW - 1) / KW;
+    auto out_at = [&](int u) {
+        const int tl = u >> 2, e = u & 3, i = tl / CT, c = tl - i * CT;
+        const int col = n0 + (c < 2 * CP ? 32 * (c >> 1) + 2 * t + (c & 1) : 16 * c + t);
+        return O + (size_t)(r0 + 16 * i + M::row(g, e)) * ld + col;
+    };
+    T old[UW];
 #pragma unroll
-        for (int u = 0; u < UNR; ++u) {
-            const int kk = kc + u * CH + KG * g;
-            const bool ok = kk < kw1;
-            const int kl = ok ? kk : kw0;
-            ra[u] = *reinterpret_cast<const vec_t *>(arow + kl);
+    for (int h = 0; h < UW; ++h) {
+        old[h] = T(0);
+        const int u = wave + h * KW;
+        if (sub && u < NU) old[h] = *out_at(u);
+    }
+    acc_t acc[RT][CT];
 #pragma unroll
-            for (int s2 = 0; s2 < KG; ++s2) rb[u][s2] = V[(size_t)(kl + s2) * c + cc];
-            if (!ok) {
+    for (int i = 0; i < RT; ++i)
 #pragma unroll
-                for (int s2 = 0; s2 < KG; ++s2) ra[u][s2] = T(0);
+        for (int j = 0; j < CT; ++j) acc[i][j] = acc_t{T(0), T(0), T(0), T(0)};
+    T a[PF][RT][4], v[PF][CT][4];
+    auto load = [&](int j, int ch) {
+        const size_t ko = (size_t)16 * ch;
+#pragma unroll
+        for (int i = 0; i < RT; ++i)
+#pragma unroll
+            for (int h = 0; h < 4 / AV; ++h) {
+                const avec w = *reinterpret_cast<const avec *>(ap + (size_t)16 * i * lda + ko + AV * h);
+#pragma unroll
+                for (int e = 0; e < AV; ++e) a[j][i][AV * h + e] = w[e];
+            }
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+#pragma unroll
+            for (int cp = 0; cp < CP; ++cp) {
+                const vpair w = *reinterpret_cast<const vpair *>(vp + (ko + s) * ld + 32 * cp);
+                v[j][2 * cp][s] = w[0];
+                v[j][2 * cp + 1][s] = w[1];
+            }
+            if (CT & 1) v[j][CT - 1][s] = vq[(ko + s) * ld];
+        }
+    };
+    auto mul = [&](int j) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int i = 0; i < RT; ++i)
+#pragma unroll
+                for (int c = 0; c < CT; ++c) acc[i][c] = M::step(a[j][i][s], v[j][c][s], acc[i][c]);
+    };
+    if (n > 0) {
+#pragma unroll
+        for (int j = 0; j < PF; ++j) load(j, min(j, n - 1));
+        int i = 0;
+        for (; i + 2 * PF <= n; i += PF) {
+#pragma unroll
+            for (int j = 0; j < PF; ++j) {
+                mul(j);
+                load(j, i + PF + j);
             }
         }
+        if (n - i > PF) {
 #pragma unroll
-        for (int u = 0; u < UNR; ++u)
+            for (int j = 0; j < PF; ++j) {
+                mul(j);
+                load(j, min(i + PF + j, n - 1));
+            }
+            i += PF;
+        }
 #pragma unroll
-            for (int s2 = 0; s2 < KG; ++s2) acc = M::step(ra[u][s2], rb[u][s2], acc);
+        for (int j = 0; j < PF; ++j)
+            if (i + j < n) mul(j);
     }
-    if (wave > 0) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) red[wave - 1][lane][i] = acc[i];
-    }
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int c = 0; c < CT; ++c)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) red[wave][i * CT + c][e][lane] = acc[i][c][e];
     __syncthreads();
-    if (wave == 0 && n0 + t < c) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const T sum = ((acc[i] + red[0][lane][i]) + red[1][lane][i]) + red[2][lane][i];
-            const size_t idx = (size_t)(r0 + M::row(g, i)) * c + n0 + t;
-            out[idx] = add ? add[idx] - sum : sum;
+    for (int h = 0; h < UW; ++h) {
+        const int u = wave + h * KW;
+        if (u >= NU) break;
+        T sum = red[0][u >> 2][u & 3][lane];
+#pragma unroll
+        for (int w = 1; w < KW; ++w) sum += red[w][u >> 2][u & 3][lane];
+        T *o = out_at(u);
+        *o = sub ? old[h] - sum : sum;
+        if (it.dup && z == it.dupz) {
+            const long long at = o - (O + (size_t)it.dup0 * ld);
+            if (at >= 0) it.dup[at] = sum;
         }
     }
 }
 
-// Batched products of many blocks (the block-diagonal passes and the pairing levels'
-// passes, where parallelism is plentiful and L2 bandwidth is the limit of the tile
-// kernel above): a workgroup computes a TM x 64 output tile of one block.  TM = 64: each
-// of its 4 waves a 32 x 32 quadrant as 2 x 2 matrix-core tiles; TM = 128 (large
-// batches): each wave a 32 x 64 strip as 2 x 4 tiles, fewer operand reads per product.
-// k advances in chunks of 16 staged through LDS, double-buffered (the next chunk's
-// global loads are in flight while the current chunk is multiplied), so every operand
-// element fetched feeds TM or 64 outputs instead of 16.  In MFMA step s of a chunk,
-// lane group g takes k = 4 g + s for both operands.  Columns past c read a clamped
-// column and are not stored.  One-dimensional grid, a multiple of 8 covering the
-// nblk (b / TM) ceil(c / 64) tiles: workgroups are dealt to the 8 XCDs round-robin
-// (workgroup w runs on XCD w % 8), so tile t = (w % 8) (grid / 8) + w / 8 gives each XCD
-// a contiguous run of whole blocks and one L2 serves all tiles of a block (the A row
-// tiles and V column tiles each tile shares with its neighbours); surplus workgroups
-// return at once.  ksplit > 0 (one product split over k, tri = 0, A and V strides 0):
-// "block" z covers k in [z ksplit, (z+1) ksplit) and writes its partial product to
-// out + z out_stride, summed afterwards by chain_reduce_kernel.
+// Batched products of many blocks with more than 16 columns (the block-diagonal passes and
+// the pairing levels' passes, where parallelism is plentiful and L2 bandwidth is the
+// limit of the tile kernel above): a workgroup computes a TM x 64 output tile of one
+// block.  TM = 64: each of its 4 waves a 32 x 32 quadrant as 2 x 2 matrix-core tiles;
+// TM = 128 (large batches): each wave a 32 x 64 strip as 2 x 4 tiles, fewer operand reads
+// per product.  k advances in chunks of 16 staged through LDS, double-buffered (the next
+// chunk's global loads are in flight while the current chunk is multiplied), so every
+// operand element fetched feeds TM or 64 outputs instead of 16.  In MFMA step s of a
+// chunk, lane group g takes k = 4 g + s for both operands.  Columns past ld read a
+// clamped column and are not stored.  The XCD mapping gives one L2 all tiles of a block
+// (the A row tiles and V column tiles each tile shares with its neighbours).
 template <typename T, int TM>
 __global__ void __launch_bounds__(256)
-band_tile_kernel(int b, int c, int tri, int nblk, const T *__restrict__ A, long long a_stride,
-                 const T *__restrict__ V, long long v_stride, const T *add,
-                 long long add_stride, T *out, long long out_stride, int ksplit) {
+band_tile_kernel(Items<T> it, int rows, int lda, int kdim, int tri, int ld, int sub) {
     using M = Mfma<T>;
     constexpr int KC = 16, AP = KC + 4, VP = 64 + 4;
     constexpr int AV = TM / 64;                    // A vec4 loads per thread per chunk
@@ -320,32 +307,26 @@ band_tile_kernel(int b, int c, int tri, int nblk, const T *__restrict__ A, long 
     typedef T vec4_t __attribute__((ext_vector_type(4)));
     __shared__ T As[2][TM][AP];
     __shared__ T Vs[2][KC][VP];
-    const int ntx = b / TM;
-    const long long per_blk = (long long)ntx * ((c + 63) / 64);
-    const long long tile = (long long)(blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
-    if (tile >= per_blk * nblk) return;
-    const long long z = tile / per_blk;
+    const int ntx = rows / TM;
+    const long long per_blk = (long long)ntx * ((ld + 63) / 64);
+    const long long tile = xcd_tile();
+    if (tile >= per_blk * it.n) return;
+    const int z = (int)(tile / per_blk);
     const int rem = (int)(tile - z * per_blk);
     const int R0 = (rem % ntx) * TM, N0 = (rem / ntx) * 64;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int g = lane >> 4, t = lane & 15;
-    A += z * a_stride;
-    V += z * v_stride;
-    out += z * out_stride;
-    if (add) add += z * add_stride;
-    int k0 = 0, k1 = b;
+    const int sd = z < it.n0 ? 0 : 1, zi = sd ? z - it.n0 : z;
+    const T *A = it.A[sd] + zi * it.as[sd];
+    const T *V = it.V[sd] + zi * it.vs[sd];
+    T *O = it.O[sd] + zi * it.os[sd];
+    int k0 = 0, k1 = kdim;
     if (tri == 1) k1 = R0 + TM;
     if (tri == 2) k0 = R0;
-    if (ksplit > 0) {   // split-k product: "block" z is the k range [z ksplit, (z+1) ksplit)
-        k0 = (int)z * ksplit;
-        k1 = min(b, k0 + ksplit);
-    }
     const int ar = tid >> 2, ac = (tid & 3) * 4;   // A chunk: rows ar + 64 u, k ac..ac+3
     const int vr = tid >> 4, vc = (tid & 15) * 4;  // V chunk: k row vr, columns vc..vc+3
-    const T *ap = A + (size_t)(R0 + ar) * b + ac;  // 4-element aligned: b % 64 == 0
-    int vcol[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) vcol[e] = min(N0 + vc + e, c - 1);
+    const T *ap = A + (size_t)(R0 + ar) * lda + ac;  // 4-element aligned: lda % 16 == 0
+    const T *vp = V + (size_t)vr * ld + min(N0 + vc, ld - 4);
     const int wr = TM == 64 ? (wave >> 1) * 32 : wave * 32;
     const int wc = TM == 64 ? (wave & 1) * 32 : 0;
     typename M::acc_t acc[RT][CT];
@@ -356,10 +337,8 @@ band_tile_kernel(int b, int c, int tri, int nblk, const T *__restrict__ A, long 
     vec4_t ga[AV];
 #pragma unroll
     for (int u = 0; u < AV; ++u)
-        ga[u] = *reinterpret_cast<const vec4_t *>(ap + (size_t)64 * u * b + k0);
-    T gv[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) gv[e] = V[(size_t)(k0 + vr) * c + vcol[e]];
+        ga[u] = *reinterpret_cast<const vec4_t *>(ap + (size_t)64 * u * lda + k0);
+    vec4_t gv = *reinterpret_cast<const vec4_t *>(vp + (size_t)k0 * ld);
     int buf = 0;
     for (int kc = k0; kc < k1; kc += KC) {
 #pragma unroll
@@ -372,9 +351,8 @@ band_tile_kernel(int b, int c, int tri, int nblk, const T *__restrict__ A, long 
         if (kc + KC < k1) {
 #pragma unroll
             for (int u = 0; u < AV; ++u)
-                ga[u] = *reinterpret_cast<const vec4_t *>(ap + (size_t)64 * u * b + kc + KC);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) gv[e] = V[(size_t)(kc + KC + vr) * c + vcol[e]];
+                ga[u] = *reinterpret_cast<const vec4_t *>(ap + (size_t)64 * u * lda + kc + KC);
+            gv = *reinterpret_cast<const vec4_t *>(vp + (size_t)(kc + KC) * ld);
         }
         T a[RT][4], bv[CT][4];
 #pragma unroll
@@ -395,145 +373,105 @@ band_tile_kernel(int b, int c, int tri, int nblk, const T *__restrict__ A, long 
 #pragma unroll
     for (int j = 0; j < CT; ++j) {
         const int col = N0 + wc + 16 * j + t;
-        if (col >= c) continue;
+        if (col >= ld) continue;
 #pragma unroll
         for (int i = 0; i < RT; ++i)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const size_t idx = (size_t)(R0 + wr + 16 * i + M::row(g, e)) * c + col;
-                out[idx] = add ? add[idx] - acc[i][j][e] : acc[i][j][e];
+                T *o = O + (size_t)(R0 + wr + 16 * i + M::row(g, e)) * ld + col;
+                *o = sub ? *o - acc[i][j][e] : acc[i][j][e];
+                if (it.dup && z == it.dupz) {
+                    const long long at = o - (O + (size_t)it.dup0 * ld);
+                    if (at >= 0) it.dup[at] = acc[i][j][e];
+                }
             }
     }
 }
 
-// out = add - (part_0 + part_1 + ... ) (or the sum when add is null), the partials of a
-// split-k product summed in a fixed order (the result does not depend on scheduling).
-template <typename T>
-__global__ void __launch_bounds__(256)
-chain_reduce_kernel(long long n, int ns, const T *__restrict__ part, const T *add, T *out) {
-    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    T sum = part[i];
-    for (int z = 1; z < ns; ++z) sum += part[(long long)z * n + i];
-    out[i] = add ? add[i] - sum : sum;
-}
-
-// Split of one chain-step product b x b times b x c over k so that the 64 x 64 tiles of
-// all splits give about four workgroups per CU: ns splits of ks rows (a multiple of the
-// 16-row k chunk); XT_TUNE_BAND_CHAIN 2 / 3 aim at 512 / 256 workgroups instead (1024
-// measured fastest on a 1856-row, 192-column chain, 512 within 2%).
-static void chain_split(int b, int c, int *ks, int *ns) {
-    const int kn = tune_knob(XT_TUNE_BAND_CHAIN);
-    const long long target = kn == 3 ? 256 : kn == 2 ? 512 : 1024;   // workgroups
-    const long long tiles = (long long)(b / 64) * ceil_div(c, 64);
-    int want = (int)std::min<long long>(b / 64, std::max<long long>(1, ceil_div(target, tiles)));
-    int k = (int)ceil_div(ceil_div(b, want), 16) * 16;
-    *ks = k;
-    *ns = (int)ceil_div(b, k);
-}
-// The chain steps use the split-k tile products (else one workgroup per 16 x 16 output
-// tile with its 4 waves splitting k): XT_TUNE_BAND_CHAIN 2-4 / 1, built-in: split.
-static bool chain_split_on(int c) {
-    const int k = tune_knob(XT_TUNE_BAND_CHAIN);
-    if (c <= 16) {   // few columns (XT_TUNE_BAND_CHAIN_FEW): split-k tiles 2, one 16 x 16
-        const int kf = tune_knob(XT_TUNE_BAND_CHAIN_FEW);   // tile per workgroup 1
-        return kf == 2 || (kf == 0 && kChainSplitFewDefault);
-    }
-    return k >= 2 || (k == 0 && kChainSplitDefault);
-}
-
-// Algorithmic bytes and flops of one sweep kernel launch: the matrix elements of the
-// stored operator (triangular: the lower or upper half and the diagonal), V read and
-// out_elems elements written or read besides, per block of the batch.
 // Profile kind of the sweeps in precision T.
 template <typename T>
 constexpr int band_kind() { return sizeof(T) == 8 ? XT_PROF_BAND64 : XT_PROF_BAND; }
 
-template <typename T>
-static void band_prof_end(int b, int c, int tri, int nblk, double out_elems, hipStream_t s) {
-    const double mat = tri ? (double)b * (b + 1) / 2 : (double)b * b;
-    const double bytes = sizeof(T) * nblk * (mat + (double)b * c + out_elems);
-    prof_end(band_kind<T>(), s, bytes, 2.0 * nblk * mat * c, false);
+// Columns of the workspace for c columns: a multiple of 16 up to 16, else the least
+// multiple of 32 or of 48 (two or three 16-column tiles a workgroup).
+static int pad_cols(int c) {
+    if (c <= 16) return 16;
+    return std::min((c + 31) / 32 * 32, (c + 47) / 48 * 48);
 }
 
-// Matrix-core launch for many columns.
+// Workgroups from which a pass with more than 16 columns takes the LDS-staged tiles.
+constexpr long long kBatchedTiles = 1536;
+
 template <typename T>
-static int launch_tile(const BandPrec &bp, int c, int tri, const T *A, long long as,
-                       const T *V, long long vs, const T *add, long long ads, T *out,
-                       long long os, int nblk, hipStream_t s) {
-    const int b = bp.b;
+static int launch_prod(const Items<T> &it, int rows, int lda, int kdim, int tri, int c, int ld,
+                       bool sub, int nseg, hipStream_t s) {
+    if (it.n <= 0 || rows <= 0) return XT_OK;
     const bool prof = prof_on(band_kind<T>());
     if (prof) prof_begin(band_kind<T>(), s);
-    const int skn = tune_knob(XT_TUNE_BAND_SMALLC);
-    if (nblk > 1 && c <= 16 && (skn == 3 || (skn == 0 && kSmallcMfmaBatched))) {
-        // few columns, many blocks: 16 x 16 output tiles (k split over the 4 waves), a
-        // quarter of the 64-column tiles' padded products
-        hipLaunchKernelGGL(band_mfma_kernel<T>, dim3(b / 16, ceil_div(c, 16), nblk), dim3(256),
-                           0, s, b, c, tri, A, as, V, vs, add, ads, out, os);
-    } else if (nblk > 1) {   // batched pass: 128-row tiles for large FP32 batches, else 64 (the
-                      // FP64 128-row tile holds 2 waves a SIMD and measured slower)
+    auto grid = [&](int tr, int tc) {
+        return dim3((unsigned)(ceil_div((long long)(rows / tr) * ceil_div(ld, tc) * it.n, 8) * 8));
+    };
+#define XT_PROD(RT, CT, KW, PF)                                                              \
+    hipLaunchKernelGGL((band_prod_kernel<T, RT, CT, KW, PF>), grid(16 * RT, 16 * CT),         \
+                       dim3(64 * KW), 0, s, it, rows, lda, kdim, tri, ld, (int)sub, nseg)
+    if (ld == 16) {
+        // few columns: the matrix is streamed once; two row tiles share V's loads where
+        // that leaves enough workgroups (4.3 TB/s in the passes over 92 768-row blocks)
+        const int sk = tune_knob(XT_TUNE_BAND_SMALLC);
+        const bool rt2 = sk == 2 || (sk != 1 && (long long)rows / 32 * it.n >= 512);
+        if (rt2 && rows % 32 == 0) XT_PROD(2, 1, 4, 4);
+        else if (tune_knob(XT_TUNE_BAND_CHAIN_FEW) == 2) XT_PROD(1, 1, 4, 4);
+        else XT_PROD(1, 1, 8, 2);
+    } else if (const long long tiles = (long long)(rows / 64) * ceil_div(ld, 64) * it.n;
+               rows % 64 == 0 && nseg == 1 && tiles >= kBatchedTiles) {
         const int tk = tune_knob(XT_TUNE_BAND_TILE);
-        const bool can128 = sizeof(T) == 4 && b % 128 == 0;
-        const int tm = (can128 && (tk == 128 || (tk == 0 && nblk >= 23))) ? 128 : 64;
-        const long long tiles = (long long)(b / tm) * ceil_div(c, 64) * nblk;
-        const dim3 grid((unsigned)(ceil_div(tiles, 8) * 8));
-        if (tm == 128)
-            hipLaunchKernelGGL((band_tile_kernel<T, 128>), grid, dim3(256), 0, s, b, c, tri, nblk,
-                               A, as, V, vs, add, ads, out, os, 0);
+        const bool can128 = sizeof(T) == 4 && rows % 128 == 0;
+        if (can128 && (tk == 128 || (tk == 0 && it.n >= 23)))
+            hipLaunchKernelGGL((band_tile_kernel<T, 128>), grid(128, 64), dim3(256), 0, s, it, rows,
+                               lda, kdim, tri, ld, (int)sub);
         else
-            hipLaunchKernelGGL((band_tile_kernel<T, 64>), grid, dim3(256), 0, s, b, c, tri, nblk,
-                               A, as, V, vs, add, ads, out, os, 0);
-    } else if (tri == 0 && chain_split_on(c) && bp.part.ptr &&
-               [&] { int ks = 0, ns = 1; chain_split(b, c, &ks, &ns);
-                     return sizeof(T) * (size_t)ns * b * c <= bp.part.bytes; }()) {
-        // one product split over k: the partials of all splits, then their fixed-order sum
-        int ks = 0, ns = 1;
-        chain_split(b, c, &ks, &ns);
-        const long long tiles = (long long)(b / 64) * ceil_div(c, 64) * ns;
-        const long long n = (long long)b * c;
-        T *part = bp.part.as<T>();
-        hipLaunchKernelGGL((band_tile_kernel<T, 64>), dim3((unsigned)(ceil_div(tiles, 8) * 8)),
-                           dim3(256), 0, s, b, c, 0, ns, A, 0LL, V, 0LL, (const T *)nullptr, 0LL,
-                           part, n, ks);
-        hipLaunchKernelGGL(chain_reduce_kernel<T>, dim3((unsigned)ceil_div(n, 256)), dim3(256), 0,
-                           s, n, ns, (const T *)part, add, out);
-    } else
-        hipLaunchKernelGGL(band_mfma_kernel<T>, dim3(b / 16, ceil_div(c, 16), nblk), dim3(256), 0,
-                           s, b, c, tri, A, as, V, vs, add, ads, out, os);
-    if (prof) band_prof_end<T>(b, c, tri, nblk, (double)b * c * (add ? 2 : 1), s);
-    return XT_OK;
-}
-
-template <typename T>
-static int launch_gemm(const BandPrec &bp, int c, int tri, const T *A, long long as,
-                       const T *V, long long vs, const T *add, long long ads, T *out,
-                       long long os, int nblk, hipStream_t s) {
-    const int b = bp.b;
-    const bool prof = prof_on(band_kind<T>());
-    const size_t vlds = sizeof(T) * (size_t)b * c;
-    // few columns: the VALU rows kernel stages V once per RW rows, which for large blocks
-    // re-reads V from L2 b / RW times per block; the matrix-core kernels read it once per
-    // tile and win there (the knob overrides)
-    const int sk = tune_knob(XT_TUNE_BAND_SMALLC);
-#define XT_ROWS(CM, RW)                                                                        \
-    do {                                                                                       \
-        if (prof) prof_begin(band_kind<T>(), s);                                               \
-        hipLaunchKernelGGL((band_rows_kernel<T, CM, RW>), dim3(b / RW, 1, nblk), dim3(256),    \
-                           vlds, s, b, c, tri, A, as, V, vs, add, ads, out, os);               \
-        if (prof) band_prof_end<T>(b, c, tri, nblk, (double)b * c * (add ? 2 : 1), s);         \
-    } while (0)
-    if (vlds > kRowsLdsMax) {
-        XT_TRY(launch_tile<T>(bp, c, tri, A, as, V, vs, add, ads, out, os, nblk, s));
-    } else if (c <= 16 && (sk == 1 || (sk == 0 && b < (sizeof(T) == 8 ? kRowsMaxB64 : kRowsMaxB)))) {
-        if (c <= 8) {
-            XT_ROWS(8, 2);
-        } else {
-            XT_ROWS(16, 1);
-        }
+            hipLaunchKernelGGL((band_tile_kernel<T, 64>), grid(64, 64), dim3(256), 0, s, it, rows,
+                               lda, kdim, tri, ld, (int)sub);
     } else {
-        XT_TRY(launch_tile<T>(bp, c, tri, A, as, V, vs, add, ads, out, os, nblk, s));
+        // dependent steps: the tile with the least work on the fullest of the 256 CUs.  FP64 steps of two b x b blocks, us: b 768,
+        // 192 columns 16.1 with 2 x 3 tiles (192 workgroups), 18.6 with 1 x 3, 19.2 with 2 x 2;
+        // b 1856, 96 columns 31.0 with 2 x 3, 40.4 with 1 x 3; b 256, 192 columns 5.7 with
+        // 1 x 2 (192 workgroups), 6.5 with 1 x 3, 8.6 with 2 x 3.
+        // The second factor weighs the operand reads per product: with b 768 and 192 columns
+        // 16 x 16 tiles would leave the CUs fuller (5 against 6 tiles each) but take 24.8 us.
+        const int cm = ld % 48 == 0 ? 3 : 2;
+        const int ck = tune_knob(XT_TUNE_BAND_CHAIN);
+        int rt = 1, ct = 1;
+        double best = 1e300;
+        for (int r = 1; r <= 2; ++r)
+            for (int k : {1, 2, 3}) {
+                if (rows % (16 * r) || ld % (16 * k) || (r == 2 && k == 1)) continue;
+                if ((ck == 1 && (r != 1 || k != 1)) || (ck == 2 && (r != 2 || k != cm)) ||
+                    (ck == 3 && (r != 1 || k != cm)))
+                    continue;
+                const long long n = (long long)(rows / (16 * r)) * (ld / (16 * k)) * it.n;
+                const double w = ceil_div(n, 256) * (r * k) * (1.0 + 0.25 / r + 0.25 / k);
+                if (w < best) {
+                    best = w;
+                    rt = r;
+                    ct = k;
+                }
+            }
+        const bool one = (long long)(rows / (16 * rt)) * (ld / (16 * ct)) * it.n <= 256;
+        // (a workgroup alone on its CU: 8 waves, two a SIMD, hide more of the loads)
+        if (rt == 2 && ct == 3 && one) XT_PROD(2, 3, 8, 2);
+        else if (rt == 2 && ct == 3) XT_PROD(2, 3, 4, 2);
+        else if (rt == 2) XT_PROD(2, 2, 4, 2);
+        else if (ct == 3) XT_PROD(1, 3, 4, 3);
+        else if (ct == 2) XT_PROD(1, 2, 4, 3);
+        else XT_PROD(1, 1, 4, 4);
     }
-#undef XT_ROWS
+#undef XT_PROD
+    if (prof) {
+        const double mat = tri ? (double)rows * (rows + 1) / 2 : (double)rows * kdim * nseg;
+        const double vec = (double)kdim * c * nseg + (double)rows * c * (sub ? 2 : 1);
+        prof_end(band_kind<T>(), s, sizeof(T) * it.n * (mat + vec), 2.0 * it.n * mat * c, false);
+    }
     return XT_OK;
 }
 
@@ -568,6 +506,15 @@ zero_upper_kernel(int b, double *L) {   // strict upper triangle of each col-maj
 // ---------------------------------------------------------------------------
 constexpr int kCT = 64;   // panel width and tile size
 
+// One elimination's operands; a launch works on one or two of them (grid y).
+struct CholSide {
+    double *L, *E, *Kn, *W;   // diagonal block, sub-diagonal block, next diagonal block, scratch
+    int *info;
+};
+struct CholSides {
+    CholSide s[2];
+};
+
 __device__ inline const double *tall_tile(const double *L, const double *E, int b, int nt,
                                           int rt, int ct) {
     const double *base = rt < nt ? L + (size_t)rt * kCT : E + (size_t)(rt - nt) * kCT;
@@ -585,8 +532,10 @@ __device__ inline double lane_bcast(double v, int src) {
 typedef double xt_d4c __attribute__((ext_vector_type(4)));
 
 __global__ void __launch_bounds__(256)
-chol_panel_kernel(int b, int nt, int k, const double *__restrict__ L,
-                  const double *__restrict__ E, double *__restrict__ W, int *__restrict__ info) {
+chol_panel_kernel(int b, int nt, int k, CholSides cs) {
+    const double *L = cs.s[blockIdx.y].L, *E = cs.s[blockIdx.y].E;
+    double *W = cs.s[blockIdx.y].W;
+    int *info = cs.s[blockIdx.y].info;
     // The 64 x 64 diagonal tile (sA) and this workgroup's row tile (sX) in LDS, factored
     // and solved in four 16-column steps: the 16 x 16 diagonal block by one wave in
     // registers, the rows below it (and the row tile's) by forward substitution, one
@@ -753,8 +702,9 @@ __device__ inline void tile_update(double *C, int b, const double *P, const doub
 // (i, j), k < j <= i < nt, of L_i; then (if E) the nt x (nt - 1 - k) tiles right of the
 // panel in E_i; then the nt (nt + 1) / 2 lower tiles of Knext.
 __global__ void __launch_bounds__(256)
-chol_update_kernel(int b, int nt, int k, double *L, double *E, double *Knext,
-                   const double *__restrict__ W) {
+chol_update_kernel(int b, int nt, int k, CholSides cs) {
+    double *L = cs.s[blockIdx.y].L, *E = cs.s[blockIdx.y].E, *Knext = cs.s[blockIdx.y].Kn;
+    const double *W = cs.s[blockIdx.y].W;
     __shared__ double sP[kCT][kCT], sQ[kCT][kCT];
     const int ntot = E ? 2 * nt : nt;
     const int ncp = ntot - k, T = nt - 1 - k;
@@ -823,35 +773,57 @@ fill_zero_kernel(long long n, T *d) {
         d[i] = T(0);
 }
 
-// Lower triangle of the 1-based CSR K, rows of blocks fb.. on, into the column-major
-// b x b diagonal blocks kd (block fb first) and sub-diagonal blocks ko (row block i+1,
-// column block i; the first is column block fb - 1 when fb > 0, else 0), one lane per
-// row in entry order (a repeated entry: the last one stays).  The rows of the last block
-// beyond p get a unit diagonal.  The blocks are zero on entry.
+// Lower triangle of the 1-based CSR K into column-major b x b blocks in the factor's order:
+// diagonal blocks from block f0 on (kd) and sub-diagonal blocks from index e0 on (ko; top
+// chain's block i at index i, bottom chain's block j at nt + j).  One lane per row in entry
+// order (a repeated entry: the last one stays).  A row i past the middle block is row
+// split + total - 1 - i of the factor's order, where the roles of an entry's row and column
+// change places; the last bottom block's couplings to the middle block keep the middle's
+// row order.  The rows of the last block beyond p get a unit diagonal.  The blocks are zero
+// on entry.  flags[0] set: an entry outside the blocks; flags[1]: the largest i - j.
 __global__ void __launch_bounds__(256)
-band_scatter_kernel(int p, int b, int nb, int fb, const int *__restrict__ ia,
+band_scatter_kernel(int p, int b, int nb, int nt, int f0, int e0, const int *__restrict__ ia,
                     const int *__restrict__ ja, const double *__restrict__ a, double *kd,
-                    double *ko, int *outside) {
-    const int i = fb * b + blockIdx.x * 256 + threadIdx.x;
+                    double *ko, int *flags) {
+    const int i = f0 * b + blockIdx.x * 256 + threadIdx.x;
     const long long bb = (long long)b * b;
-    if (i >= nb * b) return;
-    const int bi = i / b, li = i - bi * b, ko0 = fb > 0 ? fb - 1 : 0;
+    const int total = nb * b, split = (nt + 1) * b;
+    if (i >= total) return;
+    const int pi = i < split ? i : split + total - 1 - i;
+    const int bi = pi / b, li = pi - bi * b;
     if (i >= p) {
-        kd[(bi - fb) * bb + (long long)li * b + li] = 1.0;
+        kd[(bi - f0) * bb + (long long)li * b + li] = 1.0;
         return;
     }
+    int wide = 0;
     for (int k = ia[i] - 1; k < ia[i + 1] - 1; ++k) {
         const int j = ja[k] - 1;
         if (j > i) continue;
-        if (j < 0 || i - j > b) {   // not in the band this factor was sized for
-            outside[0] = 1;
+        if (j < 0 || i - j > b) {   // not in the blocks this factor was sized for
+            flags[0] = 1;
             continue;
         }
-        const int bj = j / b, lj = j - bj * b;
-        // bi == bj + 1 otherwise
-        double *dst = bi == bj ? kd + (bi - fb) * bb : ko + (bj - ko0) * bb;
-        dst[(long long)lj * b + li] = a[k];
+        wide = max(wide, i - j);
+        const int pj = j < split ? j : split + total - 1 - j;
+        const int bj = pj / b, lj = pj - bj * b;
+        int row = li, col = lj, e = bj;      // off-diagonal block: index, row, column in it
+        if (i >= split) {                    // (j in the middle block or past it)
+            row = lj;
+            col = li;
+            e = bi - 1;
+        }
+        if (bi == bj) kd[(bi - f0) * bb + (long long)col * b + row] = a[k];
+        else if (e >= e0) ko[(e - e0) * bb + (long long)col * b + row] = a[k];
     }
+    if (wide > 0) atomicMax(flags + 1, wide);
+}
+
+// dst += src (n elements)
+__global__ void __launch_bounds__(256)
+add_block_kernel(long long n, const double *__restrict__ src, double *__restrict__ dst) {
+    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n;
+         i += (long long)gridDim.x * 256)
+        dst[i] += src[i];
 }
 
 #define XT_RB(...)                                                                      \
@@ -876,48 +848,73 @@ static int zero_fill(double *d, long long n, hipStream_t s) {
     return XT_OK;
 }
 
-// Level-L matrices t0 <= t < t1 of direction dir: M^L_t = -(M^{L-1}_{2t+1} M^{L-1}_{2t}),
-// M^0_t = G_t forward and H_{m-1-t} backward.  Row-major X is column-major X^T, so the
-// row-major product is the column-major product of the stored blocks in the order
-// M_{2t}, M_{2t+1}.
-static int level_products(rocblas_handle h, int b, int m, int dir, int L, int t0, int t1,
-                          const double *G, const double *H, double *const lv[2][kLevels]) {
+// Where the matrices of one chain's recurrence (dir 0 forward, 1 backward) sit in a level's
+// array: cnt of them, es elements apart.  They are stored in ascending block order, which
+// for the backward recurrence is the reverse of its steps: step v (1, 2, ..) uses entry
+// v - 1 forward and cnt - v backward.  vrow / crow: first of the kw rows the next step
+// reads and of the rc rows the chain runs on, in an entry of rows rows.
+struct LevelView {
+    long long base, es;
+    int cnt, vrow, crow;
+};
+static LevelView level_view(const BandPrec &bp, int side, int dir, int L) {
+    LevelView v;
+    const int rows = L == 0 ? bp.b : bp.rc;
+    v.es = (long long)rows * bp.kw;
+    v.cnt = bp.steps(side, dir) >> L;
+    v.base = side == 0 ? 0 : v.es * (L == 0 ? bp.nt : bp.steps(0, dir) >> L);
+    v.vrow = dir == 0 ? rows - bp.kw : 0;
+    v.crow = dir == 0 ? rows - bp.rc : 0;
+    return v;
+}
+
+// Level-L matrices of direction dir of one chain, stored entries t0 <= t < t1:
+// M^L_t = -(M^{L-1}_{2t+1} M^{L-1}_{2t}) in step order, M^0 = G forward and H backward.
+// Row-major X is column-major X^T, so the row-major product is the column-major product
+// of the stored blocks in the order M_{2t}, M_{2t+1}.
+static int level_products(rocblas_handle h, const BandPrec &bp, int side, int dir, int L, int t0,
+                          int t1, const double *below, double *out) {
     if (t1 <= t0) return XT_OK;
-    const long long bb = (long long)b * b;
+    const LevelView f = level_view(bp, side, dir, L - 1), v = level_view(bp, side, dir, L);
     const double minus = -1.0, zero = 0.0;
-    double *out = lv[dir][L - 1];
-    if (L == 1 && dir == 1) {   // level 0 backward runs through H in reverse
-        for (int t = t0; t < t1; ++t) {
-            const double *A = H + (long long)(m - 1 - 2 * t) * bb;
-            XT_RB(rocblas_dgemm(h, rocblas_operation_none, rocblas_operation_none, b, b, b,
-                                &minus, A, b, A - bb, b, &zero, out + (long long)t * bb, b));
-        }
-        return XT_OK;
-    }
-    // consecutive pairs of a contiguous set: one batched call
-    const double *A = (L == 1 ? G : lv[dir][L - 2]) + (long long)(2 * t0) * bb;
-    XT_RB(rocblas_dgemm_strided_batched(h, rocblas_operation_none, rocblas_operation_none, b, b,
-                                        b, &minus, A, b, 2 * bb, A + bb, b, 2 * bb, &zero,
-                                        out + (long long)t0 * bb, b, bb, t1 - t0));
+    // stored entries of M_{2t} and M_{2t+1} for the first t
+    const long long lo = dir == 0 ? 2LL * t0 : f.cnt - 2LL * v.cnt + 2LL * t0 + 1;
+    const long long hi = dir == 0 ? lo + 1 : lo - 1;
+    const double *A = below + f.base + lo * f.es + (long long)f.vrow * bp.kw;
+    const double *B = below + f.base + hi * f.es + (long long)f.crow * bp.kw;
+    XT_RB(rocblas_dgemm_strided_batched(h, rocblas_operation_none, rocblas_operation_none, bp.kw,
+                                        bp.rc, bp.kw, &minus, A, bp.kw, 2 * f.es, B, bp.kw,
+                                        2 * f.es, &zero, out + v.base + t0 * v.es, bp.kw, v.es,
+                                        t1 - t0));
     return XT_OK;
 }
 
-// G_i = (D_{i+1} E_i)^T column-major, i.e. row-major D_{i+1} E_i, for n consecutive i
-// (E_i, D_{i+1} column-major with stride bb); H_i = E_i D_i column-major, row-major
-// (E_i D_i)^T.
-static int recurrence_products(rocblas_handle h, int b, const double *E, const double *Dnext,
-                               double *G, int ng, const double *Dsame, const double *Eh,
-                               double *Hout, int nh) {
+// G_i (row-major D_{i+1} E_i, its last kw columns) for n consecutive i: E the first E_i,
+// Dn the first D_{i+1}, both column-major b x b, G the first G_i.  E_i's nonzero rows start
+// at e0 (0 within a chain).
+static int g_products(rocblas_handle h, const BandPrec &bp, const double *E, int e0,
+                      const double *Dn, double *G, int n) {
+    if (n <= 0) return XT_OK;
+    const int b = bp.b, kw = bp.kw;
     const long long bb = (long long)b * b;
     const double one = 1.0, zero = 0.0;
-    if (ng > 0)
-        XT_RB(rocblas_dgemm_strided_batched(h, rocblas_operation_transpose,
-                                            rocblas_operation_transpose, b, b, b, &one, E, b, bb,
-                                            Dnext, b, bb, &zero, G, b, bb, ng));
-    if (nh > 0)
-        XT_RB(rocblas_dgemm_strided_batched(h, rocblas_operation_none, rocblas_operation_none, b,
-                                            b, b, &one, Eh, b, bb, Dsame, b, bb, &zero, Hout, b,
-                                            bb, nh));
+    XT_RB(rocblas_dgemm_strided_batched(
+        h, rocblas_operation_transpose, rocblas_operation_transpose, kw, b, kw, &one,
+        E + e0 + (long long)(b - kw) * b, b, bb, Dn + (long long)e0 * b, b, bb, &zero, G, kw,
+        (long long)b * kw, n));
+    return XT_OK;
+}
+// H_i (row-major (E_i D_i)^T, the kw columns from E_i's row e0 on) for n consecutive i.
+static int h_products(rocblas_handle h, const BandPrec &bp, const double *E, int e0,
+                      const double *D, double *H, int n) {
+    if (n <= 0) return XT_OK;
+    const int b = bp.b, kw = bp.kw;
+    const long long bb = (long long)b * b;
+    const double one = 1.0, zero = 0.0;
+    XT_RB(rocblas_dgemm_strided_batched(
+        h, rocblas_operation_none, rocblas_operation_none, kw, b, kw, &one,
+        E + e0 + (long long)(b - kw) * b, b, bb, D + (b - kw), b, bb, &zero, H, kw,
+        (long long)b * kw, n));
     return XT_OK;
 }
 
@@ -930,87 +927,158 @@ static int to_f32_range(DevBuf *set, long long off, long long n, hipStream_t s) 
     return XT_OK;
 }
 
+// Column-panel factorization of the blocks st of one or two eliminations.
+static int factor_blocks(int b, int nsides, const CholSides &cs, hipStream_t s) {
+    const int nt = b / kCT;
+    const bool E = cs.s[0].E != nullptr;
+    const int ntot = E ? 2 * nt : nt;
+    for (int k = 0; k < nt; ++k) {
+        const int T = nt - 1 - k;
+        hipLaunchKernelGGL(chol_panel_kernel, dim3(ntot - k, nsides), dim3(256), 0, s, b, nt, k, cs);
+        const int nwork = (ntot - k) + T * (T + 1) / 2 + (E ? nt * T + nt * (nt + 1) / 2 : 0);
+        hipLaunchKernelGGL(chol_update_kernel, dim3(nwork, nsides), dim3(256), 0, s, b, nt, k, cs);
+    }
+    XT_HIP(hipGetLastError());
+    return XT_OK;
+}
+
+// Estimated time (us) of one chain pair's forward or backward recurrence with nl pairing
+// levels: every launch costs a latency (the boundary and the first loads: 4.6 us for two
+// 256-row blocks) plus the larger of streaming its matrices and its products, at the rates
+// the sweeps reach (4.4 TB/s; 45 TFLOP/s in FP64, the products of the dependent steps and
+// of the batched passes alike).  Levels halve the number of dependent steps and add a pass
+// over half the blocks each way.
+static double chain_cost(int rows, int kw, int m0, int m1, int nl, int ld, size_t sv) {
+    auto launch = [&](double n) {
+        const double e = n * rows * kw;
+        return 4.6 + std::max(e * sv / 4.4e6, 2.0 * e * ld / (sv == 8 ? 45e6 : 90e6));
+    };
+    double t = 0.0;
+    for (int L = 0; L < nl; ++L)
+        t += launch((m0 >> L) / 2 + (m1 >> L) / 2) +
+             launch(((m0 >> L) + 1) / 2 + ((m1 >> L) + 1) / 2);
+    return t + std::max(m0 >> nl, m1 >> nl) * launch(2);
+}
+// Pairing levels, of at most most, with the least estimated time for ld columns.
+static int chain_levels(const BandPrec &bp, int most, int ld, size_t sv) {
+    int best = 0;
+    double tb = 1e300;
+    for (int nl = 0; nl <= most; ++nl) {
+        const double t = chain_cost(bp.rc, bp.kw, bp.steps(0, 1), bp.steps(1, 1), nl, ld, sv);
+        if (t < tb) {
+            tb = t;
+            best = nl;
+        }
+    }
+    return best;
+}
+
+// Columns of G and H and rows of the chains for a half-bandwidth of bw.
+static void set_band(BandPrec &bp, int bw) {
+    bp.kw = std::min(bp.b, std::max(64, (bw + 63) / 64 * 64));
+    bp.rc = 2 * bp.kw <= bp.b ? bp.kw : bp.b;
+}
+
 // Block Cholesky of K given as a 1-based CSR in device memory (lower triangle read).
 // fb > 0 (a factor with its FP64 sets, K changed only in rows and columns of blocks fb..):
-// blocks before fb are kept and the factor is recomputed from block fb on, starting from
-// E_{fb-1} = K_{fb,fb-1} D_{fb-1}^T and the Schur complement K_{fb,fb} - E E^T; the
-// pairing levels are recomputed where they depend on a changed block.  The result equals
-// a full factorization up to rounding.
+// the top chain's blocks before fb are kept and the factor is recomputed from there on,
+// starting from E_{ft-1} = K_{ft,ft-1} D_{ft-1}^T and the Schur complement K_{ft,ft} - E E^T
+// (ft = fb, or the middle block when fb is past it: the bottom chain, which starts at the
+// last row, is always recomputed); the pairing levels are recomputed where they depend on
+// a changed block.  The result equals a full factorization up to rounding.
 static int factor_dev(BandPrec &bp, const int *dia, const int *dja, const double *da,
                       hipStream_t s, int fb = 0) {
-    const int b = bp.b, nb = bp.nb, p = bp.p;
+    const int b = bp.b, nb = bp.nb, p = bp.p, nt = bp.nt, nbt = bp.nbt;
     const long long bb = (long long)b * b;
-    if (fb > 0 && (fb >= nb || !band_has_fp64(&bp) || !bp.Dl[0].ptr)) fb = 0;
-    const int nr = nb - fb;                       // blocks factored here
-    DevBuf L, E, Dl, G, H, info, E0;
+    if (fb >= nb || !band_has_fp64(&bp) || !bp.Dl[0].ptr) fb = 0;
+    const int ft = std::min(fb, nt);              // first block factored here
+    const int nr = nb - ft, e0 = std::max(0, ft - 1), ne = nb - 1 - e0;
+    DevBuf L, E, Dl, G, H, info, E0, Km;
     XT_TRY(L.reserve(sizeof(double) * bb * nr));
     XT_TRY(zero_fill(L.as<double>(), bb * nr, s));
-    const int ne = fb > 0 ? nr : nb - 1;          // sub-diagonal blocks held
     if (ne > 0) {
         XT_TRY(E.reserve(sizeof(double) * bb * ne));
         XT_TRY(zero_fill(E.as<double>(), bb * ne, s));
     }
-    XT_TRY(info.reserve(sizeof(int) * (nb + 1)));
-    XT_HIP(hipMemsetAsync(info.ptr, 0, sizeof(int) * (nb + 1), s));
-    hipLaunchKernelGGL(band_scatter_kernel, dim3(ceil_div((long long)nr * b, 256)), dim3(256), 0,
-                       s, p, b, nb, fb, dia, dja, da, L.as<double>(),
+    XT_TRY(info.reserve(sizeof(int) * (nb + 2)));
+    XT_HIP(hipMemsetAsync(info.ptr, 0, sizeof(int) * (nb + 2), s));
+    hipLaunchKernelGGL(band_scatter_kernel, dim3(ceil_div((long long)(nb - ft) * b, 256)), dim3(256),
+                       0, s, p, b, nb, nt, ft, e0, dia, dja, da, L.as<double>(),
                        ne > 0 ? E.as<double>() : nullptr, info.as<int>() + nb);
     XT_HIP(hipGetLastError());
     {
-        int outside = 0;
-        XT_HIP(hipMemcpyAsync(&outside, info.as<int>() + nb, sizeof(int), hipMemcpyDeviceToHost, s));
+        int flags[2] = {0, 0};
+        XT_HIP(hipMemcpyAsync(flags, info.as<int>() + nb, 2 * sizeof(int), hipMemcpyDeviceToHost, s));
         XT_HIP(hipStreamSynchronize(s));
-        if (outside) {
+        if (flags[0]) {
             set_error("K has entries outside the band of width %d the factor was built for", b);
             return XT_E_ARG;
         }
+        if (flags[1] > bp.kw) {   // a wider band than the factor had, within its blocks
+            set_band(bp, flags[1]);
+            if (ft > 0) return factor_dev(bp, dia, dja, da, s, 0);
+        }
     }
-    XT_HIP(hipMemsetAsync(info.ptr, 0, sizeof(int) * (nb + 1), s));
+    XT_HIP(hipMemsetAsync(info.ptr, 0, sizeof(int) * (nb + 2), s));
+    const int kw = bp.kw, rc = bp.rc;
+    const long long bk = (long long)b * kw;
     double *Lp = L.as<double>(), *Ep = E.as<double>();
+    auto Lat = [&](int beta) { return Lp + (beta - ft) * bb; };   // diagonal block beta
+    auto Eat = [&](int e) { return Ep + (e - e0) * bb; };         // sub-diagonal block e
     RbHandle rb;
     XT_RB(rocblas_create_handle(&rb.h));
     XT_RB(rocblas_set_stream(rb.h, s));
     XT_RB(rocblas_set_pointer_mode(rb.h, rocblas_pointer_mode_host));
-    // Ep + e(i) bb holds E_i (first K_{i+1,i}): e(i) = i for the full factorization, and
-    // i - fb + 1 (E_{fb-1} at 0) for the partial one
-    const int eo = fb > 0 ? 1 - fb : 0;
-    if (fb > 0) {
-        // E_{fb-1} = K_{fb,fb-1} L_{fb-1}^-T = K_{fb,fb-1} D_{fb-1}^T (column-major, D kept
+    if (ft > 0) {
+        // E_{ft-1} = K_{ft,ft-1} L_{ft-1}^-T = K_{ft,ft-1} D_{ft-1}^T (column-major, D kept
         // column-major in the backward set), in place of the K block; then the Schur
-        // complement K_{fb,fb} -= E E^T (lower triangle)
+        // complement K_{ft,ft} -= E E^T (lower triangle)
         const double one = 1.0, zero = 0.0, minus = -1.0;
         XT_TRY(E0.reserve(sizeof(double) * bb));
         XT_RB(rocblas_dgemm(rb.h, rocblas_operation_none, rocblas_operation_transpose, b, b, b,
-                            &one, Ep, b, bp.Du[0].as<double>() + (long long)(fb - 1) * bb, b,
-                            &zero, E0.as<double>(), b));
-        XT_HIP(hipMemcpyAsync(Ep, E0.ptr, sizeof(double) * bb, hipMemcpyDeviceToDevice, s));
-        XT_RB(rocblas_dsyrk(rb.h, rocblas_fill_lower, rocblas_operation_none, b, b, &minus, Ep,
-                            b, &one, Lp, b));
+                            &one, Eat(ft - 1), b, bp.Du[0].as<double>() + (ft - 1) * bb, b, &zero,
+                            E0.as<double>(), b));
+        XT_HIP(hipMemcpyAsync(Eat(ft - 1), E0.ptr, sizeof(double) * bb, hipMemcpyDeviceToDevice, s));
+        XT_RB(rocblas_dsyrk(rb.h, rocblas_fill_lower, rocblas_operation_none, b, b, &minus,
+                            Eat(ft - 1), b, &one, Lat(ft), b));
     }
+    // L_ii, E_i = K_{i+1,i} L_ii^-T and K_{i+1,i+1} -= E_i E_i^T, panel by panel, block st
+    // of both chains at once; the last bottom block's update of the middle block goes to Km
+    // (both chains may end in the same launch)
     int *ip = info.as<int>();
-    // L_ii, E_i = K_{i+1,i} L_ii^-T and K_{i+1,i+1} -= E_i E_i^T, panel by panel
-    const int nt = b / kCT;
     DevBuf Wb;
-    XT_TRY(Wb.reserve(sizeof(double) * 2 * nt * kCT * kCT));
-    for (int i = fb; i < nb; ++i) {
-        double *Li = Lp + (long long)(i - fb) * bb;
-        double *Ei = i + 1 < nb ? Ep + (long long)(i + eo) * bb : nullptr;
-        double *Kn = i + 1 < nb ? Li + bb : nullptr;
-        const int ntot = Ei ? 2 * nt : nt;
-        for (int k = 0; k < nt; ++k) {
-            const int T = nt - 1 - k;
-            hipLaunchKernelGGL(chol_panel_kernel, dim3(ntot - k), dim3(256), 0, s, b, nt, k, Li,
-                               Ei, Wb.as<double>(), ip + i);
-            const int nwork = (ntot - k) + T * (T + 1) / 2 + (Ei ? nt * T + nt * (nt + 1) / 2 : 0);
-            hipLaunchKernelGGL(chol_update_kernel, dim3(nwork), dim3(256), 0, s, b, nt, k, Li, Ei,
-                               Kn, Wb.as<const double>());
-        }
+    const long long wsize = 2LL * (b / kCT) * kCT * kCT;
+    XT_TRY(Wb.reserve(sizeof(double) * 2 * wsize));
+    if (nbt > 0) {
+        XT_TRY(Km.reserve(sizeof(double) * bb));
+        XT_TRY(zero_fill(Km.as<double>(), bb, s));
     }
-    XT_HIP(hipGetLastError());
+    for (int st = 0; st < std::max(nt - ft, nbt); ++st) {
+        CholSides cs;
+        int n = 0;
+        if (ft + st < nt)
+            cs.s[n++] = {Lat(ft + st), Eat(ft + st), Lat(ft + st + 1), Wb.as<double>(), ip + ft + st};
+        if (st < nbt) {
+            const int beta = nt + 1 + st;
+            cs.s[n] = {Lat(beta), Eat(nt + st), st + 1 < nbt ? Lat(beta + 1) : Km.as<double>(),
+                       Wb.as<double>() + n * wsize, ip + beta};
+            ++n;
+        }
+        if (n == 1) cs.s[1] = cs.s[0];
+        XT_TRY(factor_blocks(b, n, cs, s));
+    }
+    if (nbt > 0)
+        hipLaunchKernelGGL(add_block_kernel, dim3(std::min<long long>(ceil_div(bb, 256), 4096)),
+                           dim3(256), 0, s, bb, Km.as<const double>(), Lat(nt));
+    {
+        CholSides cs;
+        cs.s[0] = cs.s[1] = {Lat(nt), nullptr, nullptr, Wb.as<double>(), ip + nt};
+        XT_TRY(factor_blocks(b, 1, cs, s));
+    }
     std::vector<int> hinfo(nb + 1);
     XT_HIP(hipMemcpyAsync(hinfo.data(), ip, sizeof(int) * nb, hipMemcpyDeviceToHost, s));
     XT_HIP(hipStreamSynchronize(s));
-    for (int i = fb; i < nb; ++i)
+    for (int i = ft; i < nb; ++i)
         if (hinfo[i] != 0) {
             set_error("K is not positive definite (block %d, minor %d)", i, hinfo[i]);
             return XT_E_SINGULAR;
@@ -1019,86 +1087,91 @@ static int factor_dev(BandPrec &bp, const int *dia, const int *dja, const double
     XT_HIP(hipGetLastError());
     // D_i = L_ii^-1 in place (column-major lower = D_i^T row-major: the backward set)
     XT_RB(rocsolver_dtrtri_strided_batched(rb.h, rocblas_fill_lower, rocblas_diagonal_non_unit,
-                                           b, Lp, b, bb, ip + fb, nr));
+                                           b, Lp, b, bb, ip + ft, nr));
     XT_HIP(hipMemcpyAsync(hinfo.data(), ip, sizeof(int) * nb, hipMemcpyDeviceToHost, s));
     XT_HIP(hipStreamSynchronize(s));
-    for (int i = fb; i < nb; ++i)
+    for (int i = ft; i < nb; ++i)
         if (hinfo[i] != 0) {
             set_error("singular diagonal factor block %d", i);
             return XT_E_SINGULAR;
         }
-    const int m = nb - 1;
-    if (fb > 0) {
-        // nothing can fail numerically from here on: the new blocks go into the kept sets
-        double *Du = bp.Du[0].as<double>(), *Dlp = bp.Dl[0].as<double>();
-        double *Gp = bp.G[0].as<double>(), *Hp = bp.H[0].as<double>();
-        XT_HIP(hipMemcpyAsync(Du + (long long)fb * bb, Lp, sizeof(double) * bb * nr,
-                              hipMemcpyDeviceToDevice, s));
-        hipLaunchKernelGGL(transpose_kernel, dim3(b / 32, b / 32, nr), dim3(256), 0, s, b,
-                           (const double *)Lp, Dlp + (long long)fb * bb);
-        XT_HIP(hipGetLastError());
-        // G_i for i = fb-1..nb-2 (E_{fb-1} with the new D_fb on), H_i for i = fb..nb-2
-        XT_TRY(recurrence_products(rb.h, b, Ep, Lp, Gp + (long long)(fb - 1) * bb, nr, Lp,
-                                   Ep + bb, Hp + (long long)fb * bb, nr - 1));
-        // levels: forward entries whose G range reaches index fb - 1, backward entries
-        // whose H range (H_{m-1-t}) reaches index fb
-        double *lvp[2][kLevels] = {};
+    // nothing can fail numerically from here on: a partial factorization writes the new
+    // blocks into the kept sets, a full one into new ones
+    const bool full = ft == 0;
+    int nlev = bp.nlev;
+    DevBuf lv[2][kLevels];
+    if (full) {
+        // the levels that pay for the fewest columns (more columns use fewer of them);
+        // XT_TUNE_BAND_LEVELS v: v - 1 levels (set before the factor is built)
+        const int kn = tune_knob(XT_TUNE_BAND_LEVELS), maxlev = kn ? kn - 1 : kLevels;
+        nlev = 0;
+        while (nlev < maxlev && (nt >> (nlev + 1)) >= kMinChain) ++nlev;
+        if (!kn) nlev = std::max(chain_levels(bp, nlev, 16, 8), chain_levels(bp, nlev, 16, 4));
+        XT_TRY(Dl.reserve(sizeof(double) * bb * nb));
+        if (nb > 1) {
+            XT_TRY(G.reserve(sizeof(double) * bk * (nb - 1)));
+            XT_TRY(H.reserve(sizeof(double) * bk * (nb - 1)));
+        }
         for (int dir = 0; dir < 2; ++dir)
-            for (int L = 0; L < bp.nlev; ++L) lvp[dir][L] = bp.Lv[dir][L][0].as<double>();
-        for (int L = 1; L <= bp.nlev; ++L) {
-            const int cnt = m >> L;
-            XT_TRY(level_products(rb.h, b, m, 0, L, (fb - 1) >> L, cnt, Gp, Hp, lvp));
-            if (m - 1 - fb >= 0)
-                XT_TRY(level_products(rb.h, b, m, 1, L, 0,
-                                      std::min(cnt, ((m - 1 - fb) >> L) + 1), Gp, Hp, lvp));
+            for (int l = 1; l <= nlev; ++l)
+                XT_TRY(lv[dir][l - 1].reserve(sizeof(double) * rc * (size_t)kw *
+                                              ((bp.steps(0, dir) >> l) + (bp.steps(1, dir) >> l))));
+    } else {
+        XT_HIP(hipMemcpyAsync(bp.Du[0].as<double>() + ft * bb, Lp, sizeof(double) * bb * nr,
+                              hipMemcpyDeviceToDevice, s));
+    }
+    double *Dlp = full ? Dl.as<double>() : bp.Dl[0].as<double>();
+    double *Gp = full ? G.as<double>() : bp.G[0].as<double>();
+    double *Hp = full ? H.as<double>() : bp.H[0].as<double>();
+    hipLaunchKernelGGL(transpose_kernel, dim3(b / 32, b / 32, nr), dim3(256), 0, s, b,
+                       (const double *)Lp, Dlp + ft * bb);
+    XT_HIP(hipGetLastError());
+    // top chain: G_i from E_{ft-1} (with the new D_ft) on, H_i from block ft on; bottom chain:
+    // all, its last block coupled to the middle block by the middle's last rows
+    XT_TRY(g_products(rb.h, bp, Eat(e0), 0, Lat(e0 + 1), Gp + e0 * bk, nt - e0));
+    XT_TRY(h_products(rb.h, bp, Eat(ft), 0, Lat(ft), Hp + ft * bk, nt - ft));
+    XT_TRY(g_products(rb.h, bp, Eat(nt), 0, Lat(nt + 2), Gp + nt * bk, nbt - 1));
+    XT_TRY(h_products(rb.h, bp, Eat(nt), 0, Lat(nt + 1), Hp + nt * bk, nbt - 1));
+    if (nbt > 0) {
+        XT_TRY(g_products(rb.h, bp, Eat(nb - 2), b - kw, Lat(nt), Gp + (nb - 2) * bk, 1));
+        XT_TRY(h_products(rb.h, bp, Eat(nb - 2), b - kw, Lat(nb - 1), Hp + (nb - 2) * bk, 1));
+    }
+    // first changed stored entry of the top chain's levels: forward entries whose G range
+    // reaches index ft - 1, backward entries whose H range reaches block ft
+    int first[2][kLevels + 1] = {};
+    for (int dir = 0; dir < 2; ++dir)
+        for (int l = 1; l <= nlev; ++l) {
+            const int cnt = bp.steps(0, dir) >> l;
+            if (ft > 0)
+                first[dir][l] = dir == 0 ? std::min(cnt, (ft - 1) >> l)
+                                         : std::max(0, cnt - 1 - ((nt - 1 - ft) >> l));
+            if (ft > 0 && dir == 1 && ft >= nt) first[dir][l] = cnt;   // no changed H
+            const double *below = l == 1 ? (dir == 0 ? Gp : Hp)
+                                  : full ? lv[dir][l - 2].as<double>() : bp.Lv[dir][l - 2][0].as<double>();
+            double *out = full ? lv[dir][l - 1].as<double>() : bp.Lv[dir][l - 1][0].as<double>();
+            XT_TRY(level_products(rb.h, bp, 0, dir, l, first[dir][l], cnt, below, out));
+            XT_TRY(level_products(rb.h, bp, 1, dir, l, 0, bp.steps(1, dir) >> l, below, out));
         }
-        XT_TRY(to_f32_range(bp.Du, (long long)fb * bb, bb * nr, s));
-        XT_TRY(to_f32_range(bp.Dl, (long long)fb * bb, bb * nr, s));
-        XT_TRY(to_f32_range(bp.G, (long long)(fb - 1) * bb, bb * nr, s));
-        XT_TRY(to_f32_range(bp.H, (long long)fb * bb, bb * (nr - 1), s));
-        for (int L = 1; L <= bp.nlev; ++L) {
-            const int cnt = m >> L, f0 = (fb - 1) >> L;
-            XT_TRY(to_f32_range(bp.Lv[0][L - 1], (long long)f0 * bb, bb * (cnt - f0), s));
-            if (m - 1 - fb >= 0)
-                XT_TRY(to_f32_range(bp.Lv[1][L - 1], 0,
-                                    bb * std::min(cnt, ((m - 1 - fb) >> L) + 1), s));
-        }
+    if (!full) {
+        XT_TRY(to_f32_range(bp.Du, ft * bb, bb * nr, s));
+        XT_TRY(to_f32_range(bp.Dl, ft * bb, bb * nr, s));
+        XT_TRY(to_f32_range(bp.G, e0 * bk, bk * (nb - 1 - e0), s));
+        XT_TRY(to_f32_range(bp.H, ft * bk, bk * (nb - 1 - ft), s));
+        for (int dir = 0; dir < 2; ++dir)
+            for (int l = 1; l <= nlev; ++l) {
+                const long long es = (long long)rc * kw, off = first[dir][l] * es;
+                const long long n = es * ((bp.steps(0, dir) >> l) + (bp.steps(1, dir) >> l));
+                XT_TRY(to_f32_range(bp.Lv[dir][l - 1], off, n - off, s));
+            }
         XT_HIP(hipStreamSynchronize(s));
         return XT_OK;
     }
-    XT_TRY(Dl.reserve(sizeof(double) * bb * nb));
-    hipLaunchKernelGGL(transpose_kernel, dim3(b / 32, b / 32, nb), dim3(256), 0, s, b, Lp,
-                       Dl.as<double>());
-    XT_HIP(hipGetLastError());
-    if (nb > 1) {
-        XT_TRY(G.reserve(sizeof(double) * bb * (nb - 1)));
-        XT_TRY(H.reserve(sizeof(double) * bb * (nb - 1)));
-        XT_TRY(recurrence_products(rb.h, b, Ep, Lp + bb, G.as<double>(), nb - 1, Lp, Ep,
-                                   H.as<double>(), nb - 1));
-    }
-    // Level matrices: M^L_t = -(M^{L-1}_{2t+1} M^{L-1}_{2t}), t < m >> L, where
-    // M^0_t = G_t forward and H_{m-1-t} backward.
-    int nlev = 0;
-    // XT_TUNE_BAND_LEVELS v caps the pairing levels at v - 1 (set before the factor is built)
-    const int maxlev = tune_knob(XT_TUNE_BAND_LEVELS) ? tune_knob(XT_TUNE_BAND_LEVELS) - 1 : kLevels;
-    while (nlev < maxlev && (m >> (nlev + 1)) >= kMinChain) ++nlev;
-    DevBuf lv[2][kLevels];
-    double *lvp[2][kLevels] = {};
-    for (int dir = 0; dir < 2; ++dir)
-        for (int L = 1; L <= nlev; ++L) {
-            XT_TRY(lv[dir][L - 1].reserve(sizeof(double) * bb * (m >> L)));
-            lvp[dir][L - 1] = lv[dir][L - 1].as<double>();
-        }
-    for (int dir = 0; dir < 2; ++dir)
-        for (int L = 1; L <= nlev; ++L)
-            XT_TRY(level_products(rb.h, b, m, dir, L, 0, m >> L, G.as<double>(), H.as<double>(),
-                                  lvp));
     bp.Du[0] = std::move(L);
     bp.Dl[0] = std::move(Dl);
     bp.G[0] = std::move(G);
     bp.H[0] = std::move(H);
     for (int dir = 0; dir < 2; ++dir)
-        for (int L = 0; L < kLevels; ++L) bp.Lv[dir][L][0] = std::move(lv[dir][L]);
+        for (int l = 0; l < kLevels; ++l) bp.Lv[dir][l][0] = std::move(lv[dir][l]);
     bp.nlev = nlev;
     for (int k = 0; k < 4 + 2 * kLevels; ++k) {
         DevBuf *src = k == 0 ? bp.Dl : k == 1 ? bp.Du : k == 2 ? bp.G : k == 3 ? bp.H
@@ -1141,12 +1214,6 @@ int band_refactor(BandPrec *bp, const int *dia, const int *dja, const double *da
 int band_build(int p, const int *ia, const int *ja, const double *a, int block, BandPrec **out,
                bool keep64) {
     XT_ARG(p > 0 && ia && ja && a && out, "band prec arguments");
-#define XT_ROWS_ATTR(T, CM, RW)                                                                \
-    XT_HIP(hipFuncSetAttribute((const void *)band_rows_kernel<T, CM, RW>,                      \
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)kRowsLdsMax))
-    XT_ROWS_ATTR(double, 8, 2); XT_ROWS_ATTR(double, 16, 1);
-    XT_ROWS_ATTR(float, 8, 2); XT_ROWS_ATTR(float, 16, 1);
-#undef XT_ROWS_ATTR
     XT_ARG(ia[0] == 1, "CSR must be 1-based");
     int bw = 0;
     for (int i = 0; i < p; ++i) XT_ARG(ia[i + 1] >= ia[i], "CSR row pointers must not decrease");
@@ -1171,6 +1238,9 @@ int band_build(int p, const int *ia, const int *ja, const double *a, int block, 
     bp->b = b;
     bp->nb = nb;
     bp->bw = bw;
+    bp->nt = nb / 2;
+    bp->nbt = (nb - 1) / 2;
+    set_band(*bp, bw);
     bp->keep64 = keep64;
     hipStream_t s = nullptr;
     int rc = factor(*bp, ia, ja, a, s);
@@ -1189,37 +1259,90 @@ void band_dims(const BandPrec *bp, int *b, int *nb, int *bw) {
 
 bool band_has_fp64(const BandPrec *bp) { return bp->keep64; }
 
-// Columns of the active load cases, gathered (out[row][a q + j] = in[row][cols[a] q + j],
-// a < Ra) or scattered back (out[row][cols[a] q + j] = in[row][a q + j] for a < Ra, zero
-// for the inactive cases a >= Ra), rows < p.
-template <typename T>
+// x into the sweeps' workspace w (rows in the factor's order, ld columns): the temporal mix
+// with minv (NULL: none) of the active cases a < Ra (case cols[a], NULL: a), slot a's q
+// columns at a q; the rows past p zero.  One thread per row and slot.  Q: the q that is
+// unrolled, 0 for any.  The sums run
+// in the order of temporal_mix.
+template <typename T, int Q>
 __global__ void __launch_bounds__(256)
-gather_cols_kernel(long long n, int q, int R, int Ra, const int *__restrict__ cols,
-                   const T *__restrict__ in, T *__restrict__ out) {
-    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;   // over p * Ra q
-    if (i >= n) return;
-    const int ca = Ra * q;
-    const long long row = i / ca;
-    const int e = (int)(i - row * ca), a = e / q, j = e - a * q;
-    out[i] = in[row * (long long)R * q + (long long)cols[a] * q + j];
+band_load_kernel(unsigned n, int p, int split, int total, int R, int q, int Ra,
+                 const int *__restrict__ cols, int ld, const T *__restrict__ minv,
+                 const T *__restrict__ x, T *__restrict__ w) {
+    constexpr int LM = Q ? 256 * Q : 1;
+    __shared__ T Ms[LM];                      // the R q x q matrices, R q <= 256
+    const bool staged = Q && minv && R * Q <= 256;
+    if (staged) {
+        for (int e = threadIdx.x; e < R * Q * Q; e += 256) Ms[e] = minv[e];
+        __syncthreads();
+    }
+    const unsigned idx = blockIdx.x * 256u + threadIdx.x;
+    if (idx >= n) return;
+    const unsigned row = idx / (unsigned)Ra;
+    const int a = (int)(idx - row * (unsigned)Ra);
+    T *o = w + (size_t)row * ld + a * q;
+    const int dof = (int)row < split ? (int)row : split + total - 1 - (int)row;
+    if (dof >= p) {
+        for (int j = 0; j < q; ++j) o[j] = T(0);
+        return;
+    }
+    const int r = cols ? cols[a] : a;
+    const T *xr = x + ((size_t)dof * R + r) * q;
+    if (!minv) {
+        for (int j = 0; j < q; ++j) o[j] = xr[j];
+        return;
+    }
+    if (Q) {
+        T v[Q ? Q : 1];
+#pragma unroll
+        for (int j = 0; j < Q; ++j) v[j] = xr[j];
+        const T *m = staged ? Ms + r * Q * Q : minv + (size_t)r * Q * Q;
+#pragma unroll
+        for (int i = 0; i < Q; ++i) {
+            T sum = T(0);
+#pragma unroll
+            for (int j = 0; j < Q; ++j) sum += m[i * Q + j] * v[j];
+            o[i] = sum;
+        }
+    } else {
+        for (int i = 0; i < q; ++i) {
+            const T *m = minv + ((size_t)r * q + i) * q;
+            T sum = T(0);
+            for (int j = 0; j < q; ++j) sum += m[j] * xr[j];
+            o[i] = sum;
+        }
+    }
 }
-template <typename T>
+
+// The workspace's columns back to y: slot a's to case cols[a], zero for the cases listed
+// from Ra on (inactive).  One thread per DOF and case.
+template <typename T, int Q>
 __global__ void __launch_bounds__(256)
-scatter_cols_kernel(long long n, int q, int R, int Ra, const int *__restrict__ cols,
-                    const T *__restrict__ in, T *__restrict__ out) {
-    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;   // over p * R q
-    if (i >= n) return;
-    const int c = R * q;
-    const long long row = i / c;
-    const int e = (int)(i - row * c), a = e / q, j = e - a * q;
-    out[row * c + (long long)cols[a] * q + j] =
-        a < Ra ? in[row * (long long)Ra * q + (long long)a * q + j] : T(0);
+band_store_kernel(unsigned n, int split, int total, int R, int q, int Ra,
+                  const int *__restrict__ cols, int ld, const T *__restrict__ w,
+                  T *__restrict__ y) {
+    const unsigned idx = blockIdx.x * 256u + threadIdx.x;
+    if (idx >= n) return;
+    const unsigned dof = idx / (unsigned)R;
+    const int a = (int)(idx - dof * (unsigned)R);
+    const int row = (int)dof < split ? (int)dof : split + total - 1 - (int)dof;
+    T *o = y + ((size_t)dof * R + (cols ? cols[a] : a)) * q;
+    const T *v = w + (size_t)row * ld + a * q;
+    if (Q) {
+        T u[Q ? Q : 1];
+#pragma unroll
+        for (int j = 0; j < Q; ++j) u[j] = a < Ra ? v[j] : T(0);
+#pragma unroll
+        for (int j = 0; j < Q; ++j) o[j] = u[j];
+    } else {
+        for (int j = 0; j < q; ++j) o[j] = a < Ra ? v[j] : T(0);
+    }
 }
 
 template <typename T>
 int band_apply(BandPrec *bp, int R, int q, const T *minv, const T *x, T *y, hipStream_t s,
                int Ra, const int *dcols) {
-    const int b = bp->b, nb = bp->nb;
+    const int b = bp->b, nb = bp->nb, nt = bp->nt, nbt = bp->nbt, kw = bp->kw, rc = bp->rc;
     const int pi = sizeof(T) == 4 ? 1 : 0;
     if (pi == 0 && !bp->keep64) {
         set_error("band factor kept in FP32 only: no FP64 sweeps");
@@ -1232,86 +1355,123 @@ int band_apply(BandPrec *bp, int R, int q, const T *minv, const T *x, T *y, hipS
         XT_HIP(hipGetLastError());
         return XT_OK;
     }
-    const int c = q * (compact ? Ra : R), cfull = q * R;
-    const long long npad = (long long)nb * b * c, nreal = (long long)bp->p * c;
+    if (!compact) {
+        Ra = R;
+        dcols = nullptr;
+    }
+    const int c = q * Ra, ld = pad_cols(c);
     // sized for FP64 sweeps when the factor has them, and for all cases, so switching
-    // precision or the active set does not reallocate (captured graphs hold these pointers)
+    // precision or the active set does not reallocate (captured graphs hold these
+    // pointers); one block more than the factor's (the bottom chain's view of the middle)
     const size_t es = bp->keep64 ? sizeof(double) : sizeof(T);
-    XT_TRY(bp->w1.reserve(es * (size_t)nb * b * cfull));
-    XT_TRY(bp->w2.reserve(es * (size_t)nb * b * cfull));
-    if (chain_split_on(cfull)) {   // the largest ns x c over the column counts up to cfull
-        size_t most = 0;
-        for (int cc = q; cc <= cfull; cc += q) {
-            if (!chain_split_on(cc)) continue;
-            int ks = 0, ns = 1;
-            chain_split(b, cc, &ks, &ns);
-            most = std::max(most, (size_t)ns * cc);
-        }
-        XT_TRY(bp->part.reserve(es * most * b));
-    }
+    XT_TRY(bp->w1.reserve(es * (size_t)(nb + 1) * b * pad_cols(q * R)));
+    XT_TRY(bp->w2.reserve(es * (size_t)(nb + 1) * b * pad_cols(q * R)));
     T *w1 = bp->w1.as<T>(), *w2 = bp->w2.as<T>();
-    if (compact) {   // temporal mix of every case into w2, the active columns into w1
-        const T *src = x;
-        if (minv) {
-            XT_TRY(temporal_mix<T, T>(bp->p, q, R, minv, x, w2, s));
-            src = w2;
-        }
-        hipLaunchKernelGGL(gather_cols_kernel<T>, dim3(ceil_div(nreal, 256)), dim3(256), 0, s,
-                           nreal, q, R, Ra, dcols, src, w1);
-    } else if (minv) {
-        XT_TRY(temporal_mix<T, T>(bp->p, q, R, minv, x, w1, s));
-    } else {
-        XT_HIP(hipMemcpyAsync(w1, x, sizeof(T) * nreal, hipMemcpyDeviceToDevice, s));
-    }
-    if (npad > nreal)
-        hipLaunchKernelGGL(fill_zero_kernel<T>, dim3(ceil_div(npad - nreal, 256)), dim3(256), 0,
-                           s, npad - nreal, w1 + nreal);
-    const long long bb = (long long)b * b, bc = (long long)b * c;
+    const int total = nb * b, split = (nt + 1) * b;
+    const long long nload = (long long)total * Ra, nstore = (long long)bp->p * R;
+    XT_ARG(nload < (1LL << 32) - 256 && nstore < (1LL << 32) - 256, "band_apply: too many columns");
+#define XT_LOAD(Q)                                                                             \
+    hipLaunchKernelGGL((band_load_kernel<T, Q>), dim3(ceil_div(nload, 256)), dim3(256), 0, s,   \
+                       (unsigned)nload, bp->p, split, total, R, q, Ra, dcols, ld, minv, x, w1)
+    if (q == 6) XT_LOAD(6);
+    else if (q == 3) XT_LOAD(3);
+    else XT_LOAD(0);
+#undef XT_LOAD
+    XT_HIP(hipGetLastError());
+    const long long bb = (long long)b * b, bk = (long long)b * kw, bc = (long long)b * ld;
     const T *Dl = bp->Dl[pi].as<T>(), *Du = bp->Du[pi].as<T>();
     const T *G = bp->G[pi].as<T>(), *H = bp->H[pi].as<T>();
-    // pairing levels used by this apply: the factor's, or none when the columns alone
-    // give the chain steps enough work (XT_TUNE_BAND_PAIR: 1 never, 2 always; built-in:
-    // FP32 always, FP64 up to kPairMaxC64 columns)
+    // pairing levels used by this apply (XT_TUNE_BAND_PAIR: 1 none, 2 all of the factor's)
     const int pk = tune_knob(XT_TUNE_BAND_PAIR);
-    const int m = nb - 1,
-              nlev = (pk == 2 || (pk == 0 && (sizeof(T) == 4 || c <= kPairMaxC64))) ? bp->nlev : 0;
-    // One recurrence in chain coordinates: block v (0..m) at W + v S, level-L matrix of
-    // step v at Mb[L] + (v - 1) MS[L] (level 0: G forward, H in reverse backward).
+    const int nlev = pk == 1 ? 0 : pk == 2 ? bp->nlev : chain_levels(*bp, bp->nlev, ld, sizeof(T));
+    // Both chains' recurrences in step coordinates: block v of side sd at W0 + v S, its
+    // step's level-L matrix at Mb[L] + (v - 1) MS[L].
     auto chain = [&](int dir, T *w, const T *M0, hipStream_t st) -> int {
-        if (m < 1) return XT_OK;
-        T *W = dir == 0 ? w : w + (long long)m * bc;
-        const long long S = dir == 0 ? bc : -bc;
-        const T *Mb[kLevels + 1];
+        T *W0[2];
+        long long S;
+        const T *Mb[2][kLevels + 1];
         long long MS[kLevels + 1];
-        Mb[0] = dir == 0 ? M0 : M0 + (long long)(m - 1) * bb;
-        MS[0] = dir == 0 ? bb : -bb;
-        for (int L = 1; L <= nlev; ++L) {
-            Mb[L] = bp->Lv[dir][L - 1][pi].as<T>();
-            MS[L] = bb;
+        int m[2];
+        const LevelView v0 = level_view(*bp, 0, dir, 0);
+        const long long vo = (long long)v0.vrow * ld, oo = (long long)v0.crow * ld;
+        S = dir == 0 ? bc : -bc;
+        for (int sd = 0; sd < 2; ++sd) {
+            m[sd] = bp->steps(sd, dir);
+            W0[sd] = w + (dir == 0 ? (sd == 0 ? 0 : nt + 1) : (sd == 0 ? nt : nb)) * bc;
+            for (int L = 0; L <= nlev; ++L) {
+                const LevelView v = level_view(*bp, sd, dir, L);
+                // (a chain without forward steps has one stored G, for the middle block)
+                const T *arr = L == 0 ? M0 : bp->Lv[dir][L - 1][pi].as<T>();
+                Mb[sd][L] = arr + v.base + (dir == 0 ? 0 : (v.cnt - 1) * v.es) + (long long)v.crow * kw;
+                MS[L] = dir == 0 ? v.es : -v.es;
+            }
         }
+        // items of both chains: a0 + i as, V = block v0 + i vs, O = block o0 + i vs
+        auto launch = [&](int L, long long a0, long long as, long long vb, long long ob,
+                          long long str, int cnt0, int cnt1) -> int {
+            Items<T> it;
+            const int cn[2] = {std::max(0, cnt0), std::max(0, cnt1)};
+            for (int sd = 0; sd < 2; ++sd) {
+                it.A[sd] = Mb[sd][L] + a0 * MS[L];
+                it.as[sd] = as * MS[L];
+                it.V[sd] = W0[sd] + vb * S + vo;
+                it.O[sd] = W0[sd] + ob * S + oo;
+                it.vs[sd] = it.os[sd] = str * S;
+            }
+            it.n0 = cn[0];
+            it.n = cn[0] + cn[1];
+            return launch_prod<T>(it, rc, kw, kw, 0, c, ld, true, 1, st);
+        };
         for (int L = 0; L < nlev; ++L) {   // even steps of level L: the next level's rhs
             const long long d = 1LL << L;
-            XT_TRY(launch_gemm<T>(*bp, c, 0, Mb[L] + MS[L], 2 * MS[L], W + d * S, 2 * d * S,
-                                  W + 2 * d * S, 2 * d * S, W + 2 * d * S, 2 * d * S,
-                                  (m >> L) / 2, st));
+            XT_TRY(launch(L, 1, 2, d, 2 * d, 2 * d, (m[0] >> L) / 2, (m[1] >> L) / 2));
         }
         const long long D = 1LL << nlev;   // the dependent chain of the top level
-        for (int v = 1; v <= (m >> nlev); ++v)
-            XT_TRY(launch_gemm<T>(*bp, c, 0, Mb[nlev] + (v - 1) * MS[nlev], 0, W + (v - 1) * D * S,
-                                  0, W + v * D * S, 0, W + v * D * S, 0, 1, st));
+        for (int v = 1; v <= (std::max(m[0], m[1]) >> nlev); ++v)
+            XT_TRY(launch(nlev, v - 1, 0, (v - 1) * D, v * D, 0, v <= (m[0] >> nlev),
+                          v <= (m[1] >> nlev)));
         for (int L = nlev - 1; L >= 0; --L) {   // odd steps of level L, from the finished ones
             const long long d = 1LL << L;
-            XT_TRY(launch_gemm<T>(*bp, c, 0, Mb[L], 2 * MS[L], W, 2 * d * S, W + d * S,
-                                  2 * d * S, W + d * S, 2 * d * S, ((m >> L) + 1) / 2, st));
+            XT_TRY(launch(L, 0, 2, 0, d, 2 * d, ((m[0] >> L) + 1) / 2, ((m[1] >> L) + 1) / 2));
+        }
+        if (rc < b) {   // the rows no step reads
+            Items<T> it;
+            const int r0 = dir == 0 ? 0 : rc;
+            for (int sd = 0; sd < 2; ++sd) {
+                it.A[sd] = Mb[sd][0] + (long long)(r0 - v0.crow) * kw;
+                it.as[sd] = MS[0];
+                it.V[sd] = W0[sd] + vo;
+                it.O[sd] = W0[sd] + S + (long long)r0 * ld;
+                it.vs[sd] = it.os[sd] = S;
+            }
+            it.n0 = m[0];
+            it.n = m[0] + m[1];
+            XT_TRY(launch_prod<T>(it, b - rc, kw, kw, 0, c, ld, true, 1, st));
         }
         return XT_OK;
     };
+    auto diagonal = [&](int tri, const T *D, const T *v, T *o, hipStream_t st) -> int {
+        Items<T> it = {{D, D}, {v, v}, {o, o}, {bb, bb}, {bc, bc}, {bc, bc}, nb, nb};
+        if (tri == 2 && nbt > 0) {   // the bottom chain starts from the middle block's last rows
+            it.dup = o + nb * bc;
+            it.dupz = nt;
+            it.dup0 = b - kw;
+        }
+        return launch_prod<T>(it, b, b, b, tri, c, ld, false, 1, st);
+    };
     auto sweeps = [&](hipStream_t st) -> int {
-        // forward: w2 = D w1 (all blocks), then w2_{i+1} -= G_i w2_i
-        XT_TRY(launch_gemm<T>(*bp, c, 1, Dl, bb, w1, bc, nullptr, 0, w2, bc, nb, st));
+        // forward: w2 = D w1 (all blocks), the chains, then the middle block from both
+        XT_TRY(diagonal(1, Dl, w1, w2, st));
         XT_TRY(chain(0, w2, G, st));
-        // backward: w1 = D^T w2 (all blocks), then w1_i -= H_i w1_{i+1}
-        XT_TRY(launch_gemm<T>(*bp, c, 2, Du, bb, w2, bc, nullptr, 0, w1, bc, nb, st));
+        if (nt > 0) {
+            const long long vo = (long long)(b - kw) * ld;
+            Items<T> it = {{G + (nt - 1) * bk, G + (nb - 2) * bk},
+                           {w2 + (nt - 1) * bc + vo, w2 + (nb - 1) * bc + vo},
+                           {w2 + nt * bc, w2 + nt * bc}, {0, 0}, {0, 0}, {0, 0}, 1, 1};
+            XT_TRY(launch_prod<T>(it, b, kw, kw, 0, c, ld, true, nbt > 0 ? 2 : 1, st));
+        }
+        // backward: w1 = D^T w2 (all blocks), then the chains from the middle block
+        XT_TRY(diagonal(2, Du, w2, w1, st));
         XT_TRY(chain(1, w1, H, st));
         return XT_OK;
     };
@@ -1325,8 +1485,6 @@ int band_apply(BandPrec *bp, int R, int q, const T *minv, const T *x, T *y, hipS
         SweepGraph *g = nullptr;
         for (SweepGraph &cand : bp->graph)
             if (cand.exec && cand.c == c && cand.pi == pi &&
-                cand.tile == tune_knob(XT_TUNE_BAND_TILE) &&
-                cand.smallc == tune_knob(XT_TUNE_BAND_SMALLC) &&
                 cand.epoch == tune_epoch() &&
                 cand.nl == nlev &&
                 std::equal(key, key + kKey, cand.key)) {
@@ -1356,8 +1514,6 @@ int band_apply(BandPrec *bp, int R, int q, const T *minv, const T *x, T *y, hipS
             XT_HIP(ei);
             g->c = c;
             g->pi = pi;
-            g->tile = tune_knob(XT_TUNE_BAND_TILE);
-            g->smallc = tune_knob(XT_TUNE_BAND_SMALLC);
             g->epoch = tune_epoch();
             g->nl = nlev;
             std::copy(key, key + kKey, g->key);
@@ -1374,14 +1530,14 @@ int band_apply(BandPrec *bp, int R, int q, const T *minv, const T *x, T *y, hipS
                  2.0 * (2.0 * nb * tri * c + 2.0 * (nb - 1) * full * c));
     }
     XT_HIP(hipGetLastError());
-    if (compact) {
-        const long long nfull = (long long)bp->p * cfull;
-        hipLaunchKernelGGL(scatter_cols_kernel<T>, dim3(ceil_div(nfull, 256)), dim3(256), 0, s,
-                           nfull, q, R, Ra, dcols, (const T *)w1, y);
-        XT_HIP(hipGetLastError());
-    } else {
-        XT_HIP(hipMemcpyAsync(y, w1, sizeof(T) * nreal, hipMemcpyDeviceToDevice, s));
-    }
+#define XT_STORE(Q)                                                                            \
+    hipLaunchKernelGGL((band_store_kernel<T, Q>), dim3(ceil_div(nstore, 256)), dim3(256), 0, s, \
+                       (unsigned)nstore, split, total, R, q, Ra, dcols, ld, (const T *)w1, y)
+    if (q == 6) XT_STORE(6);
+    else if (q == 3) XT_STORE(3);
+    else XT_STORE(0);
+#undef XT_STORE
+    XT_HIP(hipGetLastError());
     return XT_OK;
 }
 template int band_apply<double>(BandPrec *, int, int, const double *, const double *, double *,

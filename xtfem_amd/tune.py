@@ -8,8 +8,7 @@ the launching stream (the library's per-launch profiler), the candidates of
   (1, 2, 4), for one load case lanes per node row (4, 8), for several the kernel that
   stages each slice's neighbour rows of X in LDS (off, on);
 * the banded-factor sweeps: the tile rows of the batched passes (64, 128 in FP32), and
-  for a few columns the VALU rows kernel or the matrix-core kernels (64- or 16-column
-  tiles in the batched passes);
+  for a few columns the rows of a workgroup (16, 32, or by the number of workgroups);
 * the slab solve, timed on whole solves when a solve is given: the least residual
   reduction an FP32 refinement step of GMRES-IR must reach for a case to stay in FP32
   (2, 8, 32, 128), the iterations an FP32 inner cycle gets before a case moves to FP64
@@ -146,7 +145,7 @@ def autotune(op, pr, R, fp32=True, reps=7, solve=None):
         best, res = _pick("band_tile", cands, kb, sweep, max(3, reps // 2))
         out["picks"]["band_tile"] = best
         out["timings_ms"]["band_tile"] = res
-        # few columns (a shifted factor's group, one load case): rows kernel or matrix cores
+        # few columns (a shifted factor's group, one load case): rows of a workgroup
         xs = x[:p * q].contiguous()                 # one load case: q columns
         ys = torch.empty_like(xs)
         sweep_small = lambda: pr.apply(None, xs, ys, 1, q=q, fp32=fp32)
