@@ -494,30 +494,58 @@ zero_upper_kernel(int b, double *L) {   // strict upper triangle of each col-maj
 //
 // Block i's column of the band is the tall panel [L_i; E_i] (diagonal block K_ii, then
 // the sub-diagonal block K_{i+1,i}), both column-major b x b with leading dimension b.
-// Panel k (columns 64k..64k+63) takes two launches:
-//   chol_panel_kernel: every workgroup factors the 64 x 64 diagonal tile (identical
-//     arithmetic in each workgroup, so identical results) and workgroup t > 0 solves
-//     row tile k + t of the tall panel, P = A_t L_kk^-T, alongside.  Results go to the
-//     scratch W; the matrix is only read.
-//   chol_update_kernel: copies W back into the panel's tiles and applies the rank-64
-//     update to every tile to the right: the lower tiles of L_i, all tiles of E_i, and
-//     the lower tiles of the next diagonal block (K_{i+1,i+1} -= E_i E_i^T, a piece per
-//     panel).
+// One launch per panel k (columns 64k..64k+63) of one or two eliminations (grid y), its
+// workgroups independent of each other:
+//   panel tiles t: the diagonal tile (k, k) and row tile k + t take the rank-64 update of
+//     panel k - 1, the diagonal tile is factored (identical arithmetic in each workgroup,
+//     so identical results) and the row tile solved against it, P = A_t L_kk^-T, alongside.
+//     Results go to the scratch W; the matrix is only read.
+//   trailing tiles: the rank-64 update of panel k - 1 on every tile right of column k: the
+//     lower tiles of L_i, all tiles of E_i, and the lower tiles of the next diagonal
+//     block (K_{i+1,i+1} -= E_i E_i^T, a piece per panel).
+//   copies: panel k - 1's results from the other scratch Wp into its tiles of the matrix.
+// Panel 0 of a block applies and copies the last panel of the block before it (pL, pE); a
+// launch with k = nt only applies and copies the block's own last panel.
+// What bounds it is the chain of panels, each the path through one workgroup: the launch,
+// the tile loads, the two rank-64 updates (6,700 cycles of FP64 matrix-core time on a CU)
+// and four 16-column steps (9,500 cycles each, 5,900 of them the 16 x 16 Cholesky's chain):
+// 28 us a panel on 768-row blocks, where a panel kernel (31.4 us) and an update kernel
+// (18.9 us) followed each other before.
 // ---------------------------------------------------------------------------
 constexpr int kCT = 64;   // panel width and tile size
+constexpr int kCW = 8;    // waves of a workgroup
 
 // One elimination's operands; a launch works on one or two of them (grid y).
 struct CholSide {
-    double *L, *E, *Kn, *W;   // diagonal block, sub-diagonal block, next diagonal block, scratch
-    int *info;
+    double *L = nullptr, *E = nullptr;     // diagonal and sub-diagonal block (E: NULL, none)
+    double *Kn = nullptr;                  // next diagonal block (with E)
+    double *pL = nullptr, *pE = nullptr;   // panel 0: the previous block
+    const double *Wp = nullptr;            // tiles of the panel before this one (NULL: none)
+    double *W = nullptr;                   // this panel's tiles
+    int *info = nullptr;
 };
 struct CholSides {
     CholSide s[2];
 };
 
-__device__ inline const double *tall_tile(const double *L, const double *E, int b, int nt,
-                                          int rt, int ct) {
-    const double *base = rt < nt ? L + (size_t)rt * kCT : E + (size_t)(rt - nt) * kCT;
+// Work items of one launch: panel tiles, trailing tiles of L, E and Kn, copies.
+struct CholItems {
+    int np, nl, ne, nk, nc;
+    __host__ __device__ int total() const { return np + nl + ne + nk + nc; }
+};
+__host__ __device__ inline CholItems chol_items(int nt, int k, bool E, bool Wp) {
+    const int ntot = E ? 2 * nt : nt, T = nt - 1 - k;
+    CholItems c;
+    c.np = k < nt ? ntot - k : 0;
+    c.nl = k < nt && Wp ? T * (T + 1) / 2 : 0;
+    c.ne = k >= 1 && k < nt && E ? nt * T : 0;
+    c.nk = k >= 1 && E ? nt * (nt + 1) / 2 : 0;
+    c.nc = !Wp ? 0 : k == 0 ? nt + 1 : ntot - k + 1;
+    return c;
+}
+
+__device__ inline double *tall_tile(double *L, double *E, int b, int nt, int rt, int ct) {
+    double *base = rt < nt ? L + (size_t)rt * kCT : E + (size_t)(rt - nt) * kCT;
     return base + (size_t)ct * kCT * b;
 }
 
@@ -531,219 +559,302 @@ __device__ inline double lane_bcast(double v, int src) {
 
 typedef double xt_d4c __attribute__((ext_vector_type(4)));
 
-__global__ void __launch_bounds__(256)
-chol_panel_kernel(int b, int nt, int k, CholSides cs) {
-    const double *L = cs.s[blockIdx.y].L, *E = cs.s[blockIdx.y].E;
-    double *W = cs.s[blockIdx.y].W;
-    int *info = cs.s[blockIdx.y].info;
-    // The 64 x 64 diagonal tile (sA) and this workgroup's row tile (sX) in LDS, factored
-    // and solved in four 16-column steps: the 16 x 16 diagonal block by one wave in
-    // registers, the rows below it (and the row tile's) by forward substitution, one
-    // row per thread, then the rank-16 update of the columns to the right on the matrix
-    // cores (v_mfma_f64_16x16x4f64, one 16 x 16 block per wave at a time).
-    __shared__ double sA[kCT][kCT + 1], sX[kCT][kCT + 1];
-    __shared__ double rdiag[16], colb[16];
-    __shared__ int sbad;
-    const int tid = threadIdx.x, t = blockIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
-    const double *D = tall_tile(L, E, b, nt, k, k);
-    for (int e = tid; e < kCT * kCT; e += 256) {
-        const int c = e >> 6, r = e & 63;
-        sA[r][c] = D[(size_t)c * b + r];
+// Block (16 I.., 16 J..) of P Q^T, P and Q 64 x 64 column-major tiles: accumulator i of
+// lane (g, q) is element (16 I + q, 16 J + g + 4 i).
+__device__ inline xt_d4c block_product(const double *P, const double *Q, int I, int J, int g,
+                                       int q) {
+    double pv[kCT / 4], qv[kCT / 4];
+#pragma unroll
+    for (int k4 = 0; k4 < kCT / 4; ++k4) {
+        pv[k4] = P[(4 * k4 + g) * kCT + 16 * I + q];
+        qv[k4] = Q[(4 * k4 + g) * kCT + 16 * J + q];
     }
-    if (t > 0) {
-        const double *At = tall_tile(L, E, b, nt, k + t, k);
-        for (int e = tid; e < kCT * kCT; e += 256) {
-            const int c = e >> 6, r = e & 63;
-            sX[r][c] = At[(size_t)c * b + r];
+    xt_d4c acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int k4 = 0; k4 < kCT / 4; ++k4)
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(qv[k4], pv[k4], acc, 0, 0, 0);
+    return acc;
+}
+
+// value of v in lane G of this lane's quad
+template <int G>
+__device__ inline double quad_bcast(double v) {
+    constexpr int ctrl = G * 0x55;
+    const long long bits = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_mov_dpp((int)bits, ctrl, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(bits >> 32), ctrl, 0xF, 0xF, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+__device__ inline double quad_bcast(double v, int g) {   // g: known when unrolled
+    return g == 0 ? quad_bcast<0>(v) : g == 1 ? quad_bcast<1>(v)
+         : g == 2 ? quad_bcast<2>(v) : quad_bcast<3>(v);
+}
+
+// 16 x 16 Cholesky in place at columns c0 of the tile, by one wave: lane 4 r + h holds
+// columns 4 h .. 4 h + 3 of row r.  rdiag: 1 / L_jj; Ls[j][m]: L_mj below the diagonal, else
+// zero.  Returns the first non-positive pivot (1-based, 0: none).
+// Bound by the dependent chain pivot -> 1 / sqrt -> column -> next pivot: the next two
+// columns are updated by the one just scaled with lane broadcasts of their coefficients,
+// so the next pivot's root starts at once; the other columns' updates go through LDS, a
+// column behind.
+__device__ inline int chol16(double (*sA)[kCT + 1], int c0, int lane, double *rdiag,
+                             double (*Ls)[16], double (*colb)[16]) {
+    const int r = lane >> 2, h = lane & 3;
+    double a[4], prev = 0.0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) a[e] = sA[c0 + r][c0 + 4 * h + e];
+    int bad = 0;
+    double pj = lane_bcast(a[0], 0);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+        const int hj = j >> 2, ej = j & 3;
+        bad = (!(pj > 0.0) && !bad) ? j + 1 : bad;
+        // y = 1 / sqrt(pj): the hardware estimate (relative error e ~ 2^-24) and one step of
+        // third order, y (1 + e/2 + 3 e^2/8) with e = 1 - pj y^2: error 0.3 e^3
+        double rd = __builtin_amdgcn_rsq(pj), cl[4];
+        if (j > 0) {   // column j - 1 for its update at the end of this step
+#pragma unroll
+            for (int e = 0; e < 4; ++e) cl[e] = colb[(j - 1) & 1][4 * h + e];
         }
+        const double er = fma(-pj * rd, rd, 1.0);
+        rd = fma(rd * er, fma(0.375, er, 0.5), rd);
+        const double col = r > j ? a[ej] * rd : (r == j ? pj * rd : 0.0);
+        a[ej] = h == hj ? col : a[ej];
+        const double cq = quad_bcast(col, hj);
+        if (j < 15) {
+            const int h1 = (j + 1) >> 2, e1 = (j + 1) & 3;
+            const double c1 = lane_bcast(cq, 4 * (j + 1));
+            a[e1] = fma(-cq, h == h1 ? c1 : 0.0, a[e1]);
+            pj = lane_bcast(a[e1], 4 * (j + 1) + h1);
+        }
+        if (j < 14) {
+            const int h2 = (j + 2) >> 2, e2 = (j + 2) & 3;
+            const double c2 = lane_bcast(cq, 4 * (j + 2));
+            a[e2] = fma(-cq, h == h2 ? c2 : 0.0, a[e2]);
+        }
+        if (j > 0 && j < 15) {   // columns past j + 1 (rows 0..j + 1 of cl are zero)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) a[e] = fma(-prev, cl[e], a[e]);
+        }
+        if (h == 0) colb[j & 1][r] = r > j + 2 ? cq : 0.0;
+        __builtin_amdgcn_wave_barrier();
+        prev = cq;
+        if (lane == 0) rdiag[j] = rd;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        sA[c0 + r][c0 + 4 * h + e] = a[e];
+        Ls[4 * h + e][r] = r > 4 * h + e ? a[e] : 0.0;
+    }
+    return bad;
+}
+
+__global__ void __launch_bounds__(64 * kCW)
+chol_step_kernel(int b, int nt, int k, CholSides cs) {
+    // panel: the diagonal tile and this workgroup's row tile, [row][column]; trailing: P, Q
+    __shared__ double lds[2][kCT][kCT + 1];
+    __shared__ double rdiag[16], colb[2][16];
+    __shared__ __align__(16) double Ls[16][16];
+    __shared__ int sbad;
+    const CholSide &S = cs.s[blockIdx.y];
+    double *L = S.L, *E = S.E;
+    const double *Wp = S.Wp;
+    const CholItems ci = chol_items(nt, k, E != nullptr, Wp != nullptr);
+    int id = blockIdx.x;
+    if (id >= ci.total()) return;      // (the two eliminations' counts can differ)
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, q = lane & 15;
+    constexpr size_t TS = (size_t)kCT * kCT;
+    // tile of Wp that holds row tile rt of the panel before (panel 0: row i of the next block)
+    auto wp = [&](int rt) { return Wp + TS * (k == 0 ? 1 + rt : rt - (k - 1)); };
+    if (id >= ci.np) {                 // trailing tile or copy
+        id -= ci.np;
+        const int T = nt - 1 - k;
+        double *C;
+        const double *P, *Q;
+        if (id < ci.nl) {              // lower tile (i, j) of L, k < j <= i
+            int jj = 0, rem = id;
+            while (rem >= T - jj) { rem -= T - jj; ++jj; }
+            const int j = k + 1 + jj, i = j + rem;
+            C = tall_tile(L, E, b, nt, i, j);
+            P = wp(i);
+            Q = wp(j);
+        } else if ((id -= ci.nl) < ci.ne) {   // E tile (i, j), j > k
+            const int i = id / T, j = k + 1 + (id - i * T);
+            C = tall_tile(L, E, b, nt, nt + i, j);
+            P = wp(nt + i);
+            Q = wp(j);
+        } else if ((id -= ci.ne) < ci.nk) {   // Kn lower tile (i, j): E's row tiles i, j
+            int j = 0, rem = id;
+            while (rem >= nt - j) { rem -= nt - j; ++j; }
+            const int i = j + rem;
+            C = S.Kn + (size_t)j * kCT * b + (size_t)i * kCT;
+            P = wp(nt + i);
+            Q = wp(nt + j);
+        } else {                       // copy of the panel before: its tile id
+            id -= ci.nk;
+            double *dst = k == 0 ? tall_tile(S.pL, S.pE, b, nt, nt - 1 + id, nt - 1)
+                                 : tall_tile(L, E, b, nt, k - 1 + id, k - 1);
+            const double *src = Wp + TS * id;
+            for (int e = tid; e < kCT * kCT; e += 64 * kCW)
+                dst[(size_t)(e >> 6) * b + (e & 63)] = src[e];
+            return;
+        }
+        double *sP = &lds[0][0][0], *sQ = &lds[1][0][0];
+        for (int e = tid; e < kCT * kCT; e += 64 * kCW) {
+            sP[e] = P[e];
+            sQ[e] = Q[e];
+        }
+        // 16 x 16 blocks (I, J0) and (I, J0 + 2) by each wave; the lanes of a quarter wave hold
+        // 16 consecutive rows of one column
+        const int I = wave & 3, J0 = wave >> 2;
+        double old[2][4];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                old[h][i] = C[(size_t)(16 * (J0 + 2 * h) + g + 4 * i) * b + 16 * I + q];
+        __syncthreads();
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const xt_d4c acc = block_product(sP, sQ, I, J0 + 2 * h, g, q);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                C[(size_t)(16 * (J0 + 2 * h) + g + 4 * i) * b + 16 * I + q] = old[h][i] - acc[i];
+        }
+        return;
+    }
+    const int t = id;
+    double (*sA)[kCT + 1] = lds[0], (*sX)[kCT + 1] = lds[1];
+    const double *D = tall_tile(L, E, b, nt, k, k);
+    const double *At = tall_tile(L, E, b, nt, k + t, k);
+    // the two tiles into registers and the panel before's tiles k and k + t into LDS (every
+    // wave needs most of them: 16 loads of one wave's column instead of 64)
+    constexpr int NE = kCT / kCW;     // columns of a tile each wave loads
+    double dv[NE], xv[NE];
+#pragma unroll
+    for (int e = 0; e < NE; ++e) {
+        dv[e] = D[(size_t)(wave + kCW * e) * b + lane];
+        xv[e] = t > 0 ? At[(size_t)(wave + kCW * e) * b + lane] : 0.0;
+    }
+    // rank-64 update of the panel before: the diagonal tile's lower blocks and the row
+    // tile's (panel 0 leaves the rows of E alone); wave (I, H): blocks (I, 2 H), (I, 2 H + 1)
+    const bool upx = t > 0 && (k > 0 || t < nt);
+    const int I = wave & 3, J0 = 2 * (wave >> 2);
+    xt_d4c ax[2], ad[2];
+    if (Wp) {
+        double *sk = &lds[0][0][0], *st = &lds[1][0][0];
+        const double *Pk = wp(k), *Pt = wp(k + t);
+        double pk[NE], pt[NE];
+#pragma unroll
+        for (int e = 0; e < NE; ++e) {
+            pk[e] = Pk[tid + 64 * kCW * e];
+            pt[e] = upx ? Pt[tid + 64 * kCW * e] : 0.0;
+        }
+#pragma unroll
+        for (int e = 0; e < NE; ++e) {
+            sk[tid + 64 * kCW * e] = pk[e];
+            st[tid + 64 * kCW * e] = pt[e];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            if (J0 + h <= I) ad[h] = block_product(sk, sk, I, J0 + h, g, q);
+            if (upx) ax[h] = block_product(st, sk, I, J0 + h, g, q);
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int e = 0; e < NE; ++e) {
+        sA[lane][wave + kCW * e] = dv[e];
+        sX[lane][wave + kCW * e] = xv[e];
     }
     if (tid == 0) sbad = 0;
     __syncthreads();
-    for (int s = 0; s < 4; ++s) {
-        const int c0 = 16 * s;
-        if (tid < 16) {   // (1) 16 x 16 Cholesky, lane r holds row r
-            const int r = tid;
-            double a[16];
+    if (Wp) {
 #pragma unroll
-            for (int c = 0; c < 16; ++c) a[c] = sA[c0 + r][c0 + c];
-            int bad = 0;
-#pragma unroll
-            for (int j = 0; j < 16; ++j) {
-                const double pj = lane_bcast(a[j], j);
-                bad = (!(pj > 0.0) && !bad) ? j + 1 : bad;
-                // 1 / sqrt(pj): the hardware estimate refined by two Newton steps
-                // (y <- y + y (1 - pj y^2) / 2, full FP64 precision), then sqrt(pj) = pj y
-                double rd = __builtin_amdgcn_rsq(pj);
-#pragma unroll
-                for (int it = 0; it < 2; ++it) rd = fma(0.5 * rd, fma(-pj * rd, rd, 1.0), rd);
-                const double d = pj * rd;
-                const double col = r > j ? a[j] * rd : (r == j ? d : 0.0);
-                a[j] = r >= j ? col : a[j];
-                if (r == j) rdiag[j] = rd;
-                // the column to every lane through LDS (one write, broadcast reads: the
-                // lanes are one wave, whose LDS accesses complete in order)
-                colb[r] = col;
-                __builtin_amdgcn_wave_barrier();
-#pragma unroll
-                for (int l = j + 1; l < 16; ++l) {
-                    const double cl = colb[l];
-                    a[l] = l <= r ? a[l] - col * cl : a[l];
-                }
-                __builtin_amdgcn_wave_barrier();
-            }
-#pragma unroll
-            for (int c = 0; c < 16; ++c) sA[c0 + r][c0 + c] = a[c];
-            if (r == 0 && bad && !sbad) sbad = c0 + bad;
-        }
-        __syncthreads();
-        // (2) rows below the block in the tile, then the row tile's rows: x L_s^T = a
-        const int nd = kCT - c0 - 16;
-        double *row = nullptr;
-        if (tid < nd) row = &sA[c0 + 16 + tid][0];
-        else if (t > 0 && tid < nd + kCT) row = &sX[tid - nd][0];
-        if (row) {
-            double x[16];
-#pragma unroll
-            for (int c = 0; c < 16; ++c) x[c] = row[c0 + c];
-#pragma unroll
-            for (int j = 0; j < 16; ++j) {
-                double v = x[j];
-#pragma unroll
-                for (int m = 0; m < j; ++m) v = v - x[m] * sA[c0 + j][c0 + m];
-                x[j] = v * rdiag[j];
-            }
-#pragma unroll
-            for (int c = 0; c < 16; ++c) row[c0 + c] = x[c];
-        }
-        __syncthreads();
-        // (3) C -= P Q^T over the 16-column step: lower blocks (I, J), s < J <= I, of the
-        // tile, and blocks (R, J), J > s, of the row tile; P from the block row, Q from
-        // block row J of the tile, both at columns c0..c0+15
-        const int nrem = 3 - s;
-        const int n1 = nrem * (nrem + 1) / 2, n2 = t > 0 ? 4 * nrem : 0;
-        const int g = lane >> 4, q = lane & 15;
-        for (int blk = wave; blk < n1 + n2; blk += 4) {
-            int I, J;
-            double (*Cm)[kCT + 1];
-            if (blk < n1) {
-                int jj = 0, rem = blk;
-                while (rem >= nrem - jj) { rem -= nrem - jj; ++jj; }
-                J = s + 1 + jj;
-                I = J + rem;
-                Cm = sA;
-            } else {
-                const int e = blk - n1;
-                I = e / nrem;
-                J = s + 1 + (e - I * nrem);
-                Cm = sX;
-            }
-            xt_d4c acc = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-            for (int k4 = 0; k4 < 4; ++k4) {
-                const double pa = Cm[16 * I + q][c0 + 4 * k4 + g];
-                const double qb = sA[16 * J + q][c0 + 4 * k4 + g];
-                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(pa, qb, acc, 0, 0, 0);
-            }
+        for (int h = 0; h < 2; ++h)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                double &cv = Cm[16 * I + g + 4 * i][16 * J + q];
-                cv = cv - acc[i];
+                const int c = 16 * (J0 + h) + g + 4 * i;
+                if (J0 + h <= I) sA[16 * I + q][c] -= ad[h][i];
+                if (upx) sX[16 * I + q][c] -= ax[h][i];
+            }
+        __syncthreads();
+    }
+    // rank-16 update of block (Ib, J) of the tile (or of the row tile) by step s's columns
+    auto rank16 = [&](double (*Cm)[kCT + 1], int Ib, int J, int c0) {
+        xt_d4c a4 = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int k4 = 0; k4 < 4; ++k4) {
+            const double pa = Cm[16 * Ib + q][c0 + 4 * k4 + g];
+            const double qb = sA[16 * J + q][c0 + 4 * k4 + g];
+            a4 = __builtin_amdgcn_mfma_f64_16x16x4f64(pa, qb, a4, 0, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) Cm[16 * Ib + g + 4 * i][16 * J + q] -= a4[i];
+    };
+    // four 16-column steps: the 16 x 16 diagonal block by wave 0 in registers while the other
+    // waves finish the step before (the rank-16 updates past the next 16 columns); the rows
+    // below it (and the row tile's) by forward substitution, four lanes a row; the rank-16
+    // update of the next 16 columns on the matrix cores
+    for (int s = 0; s < 4; ++s) {
+        const int c0 = 16 * s;
+        if (wave == 0) {
+            const int bad = chol16(sA, c0, lane, rdiag, Ls, colb);
+            if (tid == 0 && bad && !sbad) sbad = c0 + bad;
+        } else if (s > 0) {
+            // blocks (Ib, J) of the tile with s < J <= Ib, then (0..3, J) of the row tile
+            const int nj = 3 - s, n1 = nj * (nj + 1) / 2, n2 = t > 0 ? 4 * nj : 0;
+            for (int u = wave - 1; u < n1 + n2; u += kCW - 1) {
+                if (u < n1) {
+                    const int J = u < nj ? s + 1 : s + 2, Ib = u < nj ? s + 1 + u : 3;
+                    rank16(sA, Ib, J, c0 - 16);
+                } else {
+                    rank16(sX, (u - n1) & 3, s + 1 + ((u - n1) >> 2), c0 - 16);
+                }
             }
         }
         __syncthreads();
-    }
-    if (t == 0) {
-        if (tid == 0 && sbad) info[0] = k * kCT + sbad;
-        for (int e = tid; e < kCT * kCT; e += 256) {
-            const int c = e >> 6, r = e & 63;
-            W[e] = c <= r ? sA[r][c] : 0.0;
+        // x L_s^T = a for the rows below the block in the tile, then the row tile's rows
+        const int nd = kCT - c0 - 16, rw = tid >> 2, h = tid & 3;
+        double *row = nullptr;
+        if (rw < nd) row = &sA[c0 + 16 + rw][c0 + 4 * h];
+        else if (t > 0 && rw < nd + kCT) row = &sX[rw - nd][c0 + 4 * h];
+        if (row) {
+            double x[4], l[16][4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] = row[e];
+#pragma unroll
+            for (int j = 0; j < 15; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) l[j][e] = Ls[j][4 * h + e];
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+                const double c = x[j & 3] * rdiag[j];
+                x[j & 3] = h == (j >> 2) ? c : x[j & 3];
+                const double cq = quad_bcast(c, j >> 2);
+                if (j < 15) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) x[e] = fma(-cq, l[j][e], x[e]);
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) row[e] = x[e];
         }
-        return;
+        __syncthreads();
+        if (s < 3) {   // the next 16 columns: blocks (s + 1..3, s + 1), the row tile's (0..3, s + 1)
+            const int n1 = 3 - s;
+            if (wave < n1) rank16(sA, s + 1 + wave, s + 1, c0);
+            else if (t > 0 && wave < n1 + 4) rank16(sX, wave - n1, s + 1, c0);
+            __syncthreads();
+        }
     }
-    double *wt = W + (size_t)t * kCT * kCT;
-    for (int e = tid; e < kCT * kCT; e += 256) {
+    if (t == 0 && tid == 0 && sbad) S.info[0] = k * kCT + sbad;
+    double *wt = S.W + TS * t;
+    for (int e = tid; e < kCT * kCT; e += 64 * kCW) {
         const int c = e >> 6, r = e & 63;
-        wt[e] = sX[r][c];
+        wt[e] = t > 0 ? sX[r][c] : c <= r ? sA[r][c] : 0.0;
     }
-}
-
-// C (64 x 64 at C, leading dimension b) -= P Q^T with P, Q 64 x 64 column-major in W, on
-// the matrix cores: wave w takes the 16-row band 16w of C, four 16 x 16 blocks, k = 64.
-__device__ inline void tile_update(double *C, int b, const double *P, const double *Q,
-                                   double (*sP)[kCT], double (*sQ)[kCT]) {
-    const int tid = threadIdx.x;
-    for (int e = tid; e < kCT * kCT; e += 256) {
-        (&sP[0][0])[e] = P[e];   // sP[m][r] = P(r, m)
-        (&sQ[0][0])[e] = Q[e];
-    }
-    __syncthreads();
-    const int lane = tid & 63, w = tid >> 6, g = lane >> 4, q = lane & 15;
-    xt_d4c acc[4];
-#pragma unroll
-    for (int n = 0; n < 4; ++n) acc[n] = xt_d4c{0.0, 0.0, 0.0, 0.0};
-    for (int k4 = 0; k4 < kCT / 4; ++k4) {
-        const int m = 4 * k4 + g;
-        const double pa = sP[m][16 * w + q];
-#pragma unroll
-        for (int n = 0; n < 4; ++n)
-            acc[n] = __builtin_amdgcn_mfma_f64_16x16x4f64(pa, sQ[m][16 * n + q], acc[n], 0, 0, 0);
-    }
-#pragma unroll
-    for (int n = 0; n < 4; ++n)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            double &c = C[(size_t)(16 * n + q) * b + 16 * w + g + 4 * i];
-            c = c - acc[n][i];
-        }
-}
-
-// Work items: [0, ncp) copy W tile t to tall-panel tile (k + t, k); then the lower tiles
-// (i, j), k < j <= i < nt, of L_i; then (if E) the nt x (nt - 1 - k) tiles right of the
-// panel in E_i; then the nt (nt + 1) / 2 lower tiles of Knext.
-__global__ void __launch_bounds__(256)
-chol_update_kernel(int b, int nt, int k, CholSides cs) {
-    double *L = cs.s[blockIdx.y].L, *E = cs.s[blockIdx.y].E, *Knext = cs.s[blockIdx.y].Kn;
-    const double *W = cs.s[blockIdx.y].W;
-    __shared__ double sP[kCT][kCT], sQ[kCT][kCT];
-    const int ntot = E ? 2 * nt : nt;
-    const int ncp = ntot - k, T = nt - 1 - k;
-    int id = blockIdx.x;
-    if (id < ncp) {
-        const int rt = k + id;
-        double *dst = (double *)tall_tile(L, E, b, nt, rt, k);
-        const double *src = W + (size_t)id * kCT * kCT;
-        for (int e = threadIdx.x; e < kCT * kCT; e += 256) {
-            const int c = e >> 6, r = e & 63;
-            dst[(size_t)c * b + r] = src[e];
-        }
-        return;
-    }
-    id -= ncp;
-    const int nl = T * (T + 1) / 2;
-    if (id < nl) {   // lower tile (i, j) of L_i right of the panel: j = k+1+jj, i = j + ii
-        int jj = 0, rem = id;
-        while (rem >= T - jj) { rem -= T - jj; ++jj; }
-        const int j = k + 1 + jj, i = j + rem;
-        tile_update((double *)tall_tile(L, E, b, nt, i, j), b, W + (size_t)(i - k) * kCT * kCT,
-                    W + (size_t)(j - k) * kCT * kCT, sP, sQ);
-        return;
-    }
-    id -= nl;
-    if (!E) return;
-    if (id < nt * T) {   // E_i tile (i, j), j > k
-        const int i = id / T, j = k + 1 + (id - (id / T) * T);
-        tile_update((double *)tall_tile(L, E, b, nt, nt + i, j), b,
-                    W + (size_t)(nt + i - k) * kCT * kCT, W + (size_t)(j - k) * kCT * kCT, sP, sQ);
-        return;
-    }
-    id -= nt * T;
-    // Knext lower tile (i, j), j <= i: -= E_i(row tile i, panel) E_i(row tile j, panel)^T
-    int j = 0, rem = id;
-    while (rem >= nt - j) { rem -= nt - j; ++j; }
-    const int i = j + rem;
-    tile_update(Knext + (size_t)j * kCT * b + (size_t)i * kCT, b,
-                W + (size_t)(nt + i - k) * kCT * kCT, W + (size_t)(nt + j - k) * kCT * kCT, sP, sQ);
 }
 
 // dst_blk = src_blk^T (b x b blocks), 32 x 32 tiles through LDS.
@@ -927,19 +1038,62 @@ static int to_f32_range(DevBuf *set, long long off, long long n, hipStream_t s) 
     return XT_OK;
 }
 
-// Column-panel factorization of the blocks st of one or two eliminations.
-static int factor_blocks(int b, int nsides, const CholSides &cs, hipStream_t s) {
-    const int nt = b / kCT;
-    const bool E = cs.s[0].E != nullptr;
-    const int ntot = E ? 2 * nt : nt;
-    for (int k = 0; k < nt; ++k) {
-        const int T = nt - 1 - k;
-        hipLaunchKernelGGL(chol_panel_kernel, dim3(ntot - k, nsides), dim3(256), 0, s, b, nt, k, cs);
-        const int nwork = (ntot - k) + T * (T + 1) / 2 + (E ? nt * T + nt * (nt + 1) / 2 : 0);
-        hipLaunchKernelGGL(chol_update_kernel, dim3(nwork, nsides), dim3(256), 0, s, b, nt, k, cs);
+// One elimination in progress: its two scratch panels (of 2 nt tiles each) and the panel
+// that the next launch applies.
+struct CholRun {
+    double *W[2] = {nullptr, nullptr};
+    int cur = 0;                      // W[cur]: the next panel's tiles
+    bool have = false;                // W[1 - cur] holds a panel not yet applied
+    double *pL = nullptr, *pE = nullptr;   // the block it belongs to, when it is that block's last
+    CholSide side(double *L, double *E, double *Kn, int *info) const {
+        CholSide c;
+        c.L = L;
+        c.E = E;
+        c.Kn = Kn;
+        c.pL = pL;
+        c.pE = pE;
+        c.Wp = have ? W[1 - cur] : nullptr;
+        c.W = W[cur];
+        c.info = info;
+        return c;
     }
+};
+
+static int chol_launch(int b, int nt, int k, const CholSide *sides, int n, hipStream_t s) {
+    CholSides cs;
+    int total = 0;
+    for (int i = 0; i < 2; ++i) {
+        cs.s[i] = sides[std::min(i, n - 1)];
+        total = std::max(total, chol_items(nt, k, cs.s[i].E != nullptr, cs.s[i].Wp != nullptr).total());
+    }
+    if (total > 0)
+        hipLaunchKernelGGL(chol_step_kernel, dim3(total, n), dim3(64 * kCW), 0, s, b, nt, k, cs);
     XT_HIP(hipGetLastError());
     return XT_OK;
+}
+
+// The panels of one block of each of n eliminations (side i: block blk[i], run *run[i]).
+static int factor_blocks(int b, const CholSide *blk, CholRun *const *run, int n, hipStream_t s) {
+    const int nt = b / kCT;
+    for (int k = 0; k < nt; ++k) {
+        CholSide sd[2];
+        for (int i = 0; i < n; ++i) {
+            sd[i] = run[i]->side(blk[i].L, blk[i].E, blk[i].Kn, blk[i].info);
+            run[i]->cur ^= 1;
+            run[i]->have = true;
+        }
+        XT_TRY(chol_launch(b, nt, k, sd, n, s));
+    }
+    for (int i = 0; i < n; ++i) {
+        run[i]->pL = blk[i].L;
+        run[i]->pE = blk[i].E;
+    }
+    return XT_OK;
+}
+// Apply and store the last panel of an elimination's last block.
+static int factor_flush(int b, const CholSide &blk, const CholRun &run, hipStream_t s) {
+    const CholSide sd = run.side(blk.L, blk.E, blk.Kn, blk.info);
+    return chol_launch(b, b / kCT, b / kCT, &sd, 1, s);
 }
 
 // Estimated time (us) of one chain pair's forward or backward recurrence with nl pairing
@@ -1048,32 +1202,49 @@ static int factor_dev(BandPrec &bp, const int *dia, const int *dja, const double
     int *ip = info.as<int>();
     DevBuf Wb;
     const long long wsize = 2LL * (b / kCT) * kCT * kCT;
-    XT_TRY(Wb.reserve(sizeof(double) * 2 * wsize));
+    XT_TRY(Wb.reserve(sizeof(double) * 4 * wsize));
+    CholRun run[2];
+    for (int sd = 0; sd < 2; ++sd)
+        for (int h = 0; h < 2; ++h) run[sd].W[h] = Wb.as<double>() + (2 * sd + h) * wsize;
     if (nbt > 0) {
         XT_TRY(Km.reserve(sizeof(double) * bb));
         XT_TRY(zero_fill(Km.as<double>(), bb, s));
     }
+    CholSide last;
     for (int st = 0; st < std::max(nt - ft, nbt); ++st) {
-        CholSides cs;
+        CholSide blk[2];
+        CholRun *rn[2];
         int n = 0;
-        if (ft + st < nt)
-            cs.s[n++] = {Lat(ft + st), Eat(ft + st), Lat(ft + st + 1), Wb.as<double>(), ip + ft + st};
+        if (ft + st < nt) {
+            blk[n].L = Lat(ft + st);
+            blk[n].E = Eat(ft + st);
+            blk[n].Kn = Lat(ft + st + 1);
+            blk[n].info = ip + ft + st;
+            rn[n++] = &run[0];
+        }
         if (st < nbt) {
             const int beta = nt + 1 + st;
-            cs.s[n] = {Lat(beta), Eat(nt + st), st + 1 < nbt ? Lat(beta + 1) : Km.as<double>(),
-                       Wb.as<double>() + n * wsize, ip + beta};
-            ++n;
+            blk[n].L = Lat(beta);
+            blk[n].E = Eat(nt + st);
+            blk[n].Kn = st + 1 < nbt ? Lat(beta + 1) : Km.as<double>();
+            blk[n].info = ip + beta;
+            last = blk[n];
+            rn[n++] = &run[1];
         }
-        if (n == 1) cs.s[1] = cs.s[0];
-        XT_TRY(factor_blocks(b, n, cs, s));
+        XT_TRY(factor_blocks(b, blk, rn, n, s));
     }
-    if (nbt > 0)
+    if (nbt > 0) {
+        XT_TRY(factor_flush(b, last, run[1], s));
         hipLaunchKernelGGL(add_block_kernel, dim3(std::min<long long>(ceil_div(bb, 256), 4096)),
                            dim3(256), 0, s, bb, Km.as<const double>(), Lat(nt));
+    }
     {
-        CholSides cs;
-        cs.s[0] = cs.s[1] = {Lat(nt), nullptr, nullptr, Wb.as<double>(), ip + nt};
-        XT_TRY(factor_blocks(b, 1, cs, s));
+        CholSide mid;
+        mid.L = Lat(nt);
+        mid.info = ip + nt;
+        CholRun *rn[1] = {&run[0]};
+        XT_TRY(factor_blocks(b, &mid, rn, 1, s));
+        XT_TRY(factor_flush(b, mid, run[0], s));
     }
     std::vector<int> hinfo(nb + 1);
     XT_HIP(hipMemcpyAsync(hinfo.data(), ip, sizeof(int) * nb, hipMemcpyDeviceToHost, s));
