@@ -101,3 +101,25 @@ def test_refactor_with_a_wider_band(dev):
         pr = dev.BandPreconditioner(K, block=b)
         pr.refactor(*(t(v) for v in K2), first_row=first)
         check(dev, pr, K2, (3, 60), first)
+
+
+def test_failed_refactor_keeps_the_factor(dev):
+    """An indefinite K of a wider band is refused and the factor still solves with the old one;
+    a good K afterwards refactors in place, several times."""
+    import torch
+    from xtfem_amd.api import XtError
+    K = strip(60)
+    ia, ja, a = (np.asarray(v) for v in K)
+    t = lambda v, d: torch.as_tensor(np.ascontiguousarray(v, dtype=d), device="cuda")
+    pr = dev.BandPreconditioner(K, block=256)
+    p = len(ia) - 1
+    bad = (np.arange(1, p + 2), np.arange(1, p + 1), np.full(p, -1.0))
+    bad[0][p] += 1                       # last row: also couples 200 columns back
+    bad = (bad[0], np.concatenate([bad[1][:-1], [p - 200, p]]), np.full(p + 1, -1.0))
+    with pytest.raises(XtError, match="code -3"):
+        pr.refactor(t(bad[0], np.int32), t(bad[1], np.int32), t(bad[2], np.float64))
+    check(dev, pr, K, (6, 60), 1)
+    for scale in (1.5, 0.7, 1.1):
+        K2 = (ia, ja, a * scale)
+        pr.refactor(t(ia, np.int32), t(ja, np.int32), t(K2[2], np.float64))
+        check(dev, pr, K2, (6, 60), 2)

@@ -22,8 +22,8 @@ ARCH = os.environ.get("XTFEM_OFFLOAD_ARCH", "gfx950")
 SOURCES = ["xt_kron.hip", "xt_bsr.hip", "xt_prec.hip", "xt_band.hip", "xt_gmres.hip",
            "xt_damage.hip", "xt_capi.hip", "xt_prof.hip", "xt_ilut.cpp",
            "xt_delete.cpp", "xt_asm.hip"]
-# rocSOLVER / rocBLAS: dense block factorization of the banded preconditioner (setup only).
-LIBS = ["-L/opt/rocm/lib", "-lrocsolver", "-lrocblas"]
+# rocBLAS: the dense block products of the banded preconditioner's factorization (setup only).
+LIBS = ["-L/opt/rocm/lib", "-lrocblas"]
 
 # Packed FP32 instructions are disabled for all device code (-packed-fp32-ops).
 COMMON = ["-O3", "-fPIC", "-std=c++17", f"--offload-arch={ARCH}",

@@ -38,10 +38,9 @@
 // The factorization runs on the device once per K, and again at every refactorization
 // (xt_prec_refactor_band: per slab when K follows the temperature; from the first
 // changed block on after an element deletion): this file's panel kernels for the block
-// Cholesky, rocSOLVER trtri for D_i and rocBLAS gemm for G_i, H_i and the level matrices
+// Cholesky and the inverses D_i, rocBLAS gemm for G_i, H_i and the level matrices
 // (b^3 products near the FP64 matrix-core peak).  None of it is on the per-iteration path.
 #include <rocblas/rocblas.h>
-#include <rocsolver/rocsolver.h>
 
 #include <algorithm>
 #include <cstring>
@@ -65,6 +64,23 @@ struct SweepGraph {
     hipGraphExec_t exec = nullptr;
 };
 
+#define XT_RB(...)                                                                      \
+    do {                                                                                \
+        rocblas_status st_ = (__VA_ARGS__);                                             \
+        if (st_ != rocblas_status_success) {                                            \
+            ::xt::set_error("%s:%d %s -> rocblas status %d", __FILE__, __LINE__,        \
+                            #__VA_ARGS__, (int)st_);                                    \
+            return XT_E_HIP;                                                            \
+        }                                                                               \
+    } while (0)
+
+struct RbHandle {
+    rocblas_handle h = nullptr;
+    ~RbHandle() { if (h) rocblas_destroy_handle(h); }
+};
+
+constexpr size_t kKeepScratch = 8ull << 30;
+
 struct BandPrec {
     int p = 0, b = 0, nb = 0, bw = 0;
     int nt = 0, nbt = 0;         // blocks of the top and of the bottom chain (+ the middle)
@@ -79,6 +95,12 @@ struct BandPrec {
     int nlev = 0;
     bool keep64 = true;          // false: the FP64 sets are released after the FP32 copies
     DevBuf w1, w2;
+    // scratch of the factorization, kept from the first refactorization on while it is at
+    // most kKeepScratch bytes (a refactorization per slab would spend 5 ms of 30 on its
+    // allocations and frees), and the rocBLAS handle with it
+    DevBuf sL, sE, sW, sK, sinfo;
+    bool built = false;
+    RbHandle *rb = nullptr;
     SweepGraph graph[4];
     int next_graph = 0;
     hipStream_t cap = nullptr;   // capture stream (non-blocking, default priority)
@@ -89,6 +111,7 @@ struct BandPrec {
         for (SweepGraph &g : graph)
             if (g.exec) (void)hipGraphExecDestroy(g.exec);
         if (cap) (void)hipStreamDestroy(cap);
+        delete rb;
     }
     int blocks(int side) const { return side == 0 ? nt : nbt; }
     // steps of a chain's recurrence: forward over its blocks, backward from the middle
@@ -478,17 +501,6 @@ static int launch_prod(const Items<T> &it, int rows, int lda, int kdim, int tri,
 // ---------------------------------------------------------------------------
 // Setup kernels
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256)
-zero_upper_kernel(int b, double *L) {   // strict upper triangle of each col-major block
-    const long long blk = blockIdx.y;
-    double *a = L + blk * (long long)b * b;
-    for (long long e = (long long)blockIdx.x * 256 + threadIdx.x; e < (long long)b * b;
-         e += (long long)gridDim.x * 256) {
-        const int j = (int)(e / b), i = (int)(e - (long long)j * b);
-        if (i < j) a[e] = 0.0;
-    }
-}
-
 // ---------------------------------------------------------------------------
 // Blocked Cholesky of the band, 64-column panels (replaces potrf + trsm + syrk per block)
 //
@@ -499,7 +511,8 @@ zero_upper_kernel(int b, double *L) {   // strict upper triangle of each col-maj
 //   panel tiles t: the diagonal tile (k, k) and row tile k + t take the rank-64 update of
 //     panel k - 1, the diagonal tile is factored (identical arithmetic in each workgroup,
 //     so identical results) and the row tile solved against it, P = A_t L_kk^-T, alongside.
-//     Results go to the scratch W; the matrix is only read.
+//     Workgroup 0 solves the identity instead, which gives D_kk = L_kk^-1 (nothing reads
+//     L_kk again).  Results go to the scratch W; the matrix is only read.
 //   trailing tiles: the rank-64 update of panel k - 1 on every tile right of column k: the
 //     lower tiles of L_i, all tiles of E_i, and the lower tiles of the next diagonal
 //     block (K_{i+1,i+1} -= E_i E_i^T, a piece per panel).
@@ -734,7 +747,8 @@ chol_step_kernel(int b, int nt, int k, CholSides cs) {
 #pragma unroll
     for (int e = 0; e < NE; ++e) {
         dv[e] = D[(size_t)(wave + kCW * e) * b + lane];
-        xv[e] = t > 0 ? At[(size_t)(wave + kCW * e) * b + lane] : 0.0;
+        xv[e] = t > 0 ? At[(size_t)(wave + kCW * e) * b + lane]
+                      : lane == wave + kCW * e ? 1.0 : 0.0;
     }
     // rank-64 update of the panel before: the diagonal tile's lower blocks and the row
     // tile's (panel 0 leaves the rows of E alone); wave (I, H): blocks (I, 2 H), (I, 2 H + 1)
@@ -804,7 +818,7 @@ chol_step_kernel(int b, int nt, int k, CholSides cs) {
             if (tid == 0 && bad && !sbad) sbad = c0 + bad;
         } else if (s > 0) {
             // blocks (Ib, J) of the tile with s < J <= Ib, then (0..3, J) of the row tile
-            const int nj = 3 - s, n1 = nj * (nj + 1) / 2, n2 = t > 0 ? 4 * nj : 0;
+            const int nj = 3 - s, n1 = nj * (nj + 1) / 2, n2 = 4 * nj;
             for (int u = wave - 1; u < n1 + n2; u += kCW - 1) {
                 if (u < n1) {
                     const int J = u < nj ? s + 1 : s + 2, Ib = u < nj ? s + 1 + u : 3;
@@ -819,7 +833,7 @@ chol_step_kernel(int b, int nt, int k, CholSides cs) {
         const int nd = kCT - c0 - 16, rw = tid >> 2, h = tid & 3;
         double *row = nullptr;
         if (rw < nd) row = &sA[c0 + 16 + rw][c0 + 4 * h];
-        else if (t > 0 && rw < nd + kCT) row = &sX[rw - nd][c0 + 4 * h];
+        else if (rw < nd + kCT) row = &sX[rw - nd][c0 + 4 * h];
         if (row) {
             double x[4], l[16][4];
 #pragma unroll
@@ -845,7 +859,7 @@ chol_step_kernel(int b, int nt, int k, CholSides cs) {
         if (s < 3) {   // the next 16 columns: blocks (s + 1..3, s + 1), the row tile's (0..3, s + 1)
             const int n1 = 3 - s;
             if (wave < n1) rank16(sA, s + 1 + wave, s + 1, c0);
-            else if (t > 0 && wave < n1 + 4) rank16(sX, wave - n1, s + 1, c0);
+            else if (wave < n1 + 4) rank16(sX, wave - n1, s + 1, c0);
             __syncthreads();
         }
     }
@@ -853,20 +867,101 @@ chol_step_kernel(int b, int nt, int k, CholSides cs) {
     double *wt = S.W + TS * t;
     for (int e = tid; e < kCT * kCT; e += 64 * kCW) {
         const int c = e >> 6, r = e & 63;
-        wt[e] = t > 0 ? sX[r][c] : c <= r ? sA[r][c] : 0.0;
+        wt[e] = t > 0 ? sX[r][c] : sX[c][r];
     }
 }
 
-// dst_blk = src_blk^T (b x b blocks), 32 x 32 tiles through LDS.
+// D = L^-1 of column-major lower b x b blocks whose diagonal tiles already hold D_kk, in
+// both layouts (du column-major, dl row-major), one 64 x 64 tile a workgroup: the tiles at
+// distance d below the diagonal from those nearer to it,
+//   D_ij = -D_ii (L_ij D_jj + ... + L_i,i-1 D_i-1,j),   j = i - d,
+// the inner products accumulated in registers (operands straight from memory: L
+// column-major gives the rows of A, dl row-major the columns of B as 128-byte runs), the
+// sum and the result turned through LDS.  d = 0 copies the diagonal tiles and zeroes the
+// others above.  nt - 1 launches over all blocks; matrix-core bound where there are many
+// (93 blocks of 768 rows: 0.9 ms, the library's batched trtri and two transposing passes
+// 5.2 ms).
 __global__ void __launch_bounds__(256)
-transpose_kernel(int b, const double *__restrict__ src, double *__restrict__ dst) {
-    __shared__ double tile[32][33];
-    const long long off = (long long)blockIdx.z * b * b;
-    const int i0 = blockIdx.x * 32, j0 = blockIdx.y * 32;
-    const int tx = threadIdx.x % 32, ty = threadIdx.x / 32;
-    for (int j = ty; j < 32; j += 8) tile[j][tx] = src[off + (size_t)(j0 + j) * b + i0 + tx];
+tri_inverse_kernel(int b, int nt, int d, const double *__restrict__ Lb, double *du, double *dl) {
+    __shared__ double sm[kCT][kCT + 1];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, q = lane & 15;
+    const long long off = (long long)blockIdx.y * b * b;
+    Lb += off;
+    du += off;
+    dl += off;
+    if (d == 0) {   // tiles (i, j), j >= i
+        int i = 0, rem = blockIdx.x;
+        while (rem >= nt - i) { rem -= nt - i; ++i; }
+        const int j = i + rem;
+        for (int e = tid; e < kCT * kCT; e += 256) {
+            const int c = e >> 6, r = e & 63;
+            const double v = i == j ? Lb[(size_t)(j * kCT + c) * b + i * kCT + r] : 0.0;
+            du[(size_t)(j * kCT + c) * b + i * kCT + r] = v;
+            if (i == j) sm[r][c] = v;
+        }
+        __syncthreads();
+        for (int e = tid; e < kCT * kCT; e += 256) {
+            const int r = e >> 6, c = e & 63;
+            dl[(size_t)(i * kCT + r) * b + j * kCT + c] = i == j ? sm[r][c] : 0.0;
+        }
+        return;
+    }
+    const int i = d + blockIdx.x, j = blockIdx.x;
+    const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;   // this wave's quadrant
+    xt_d4c acc[2][2];
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y) acc[x][y] = xt_d4c{0.0, 0.0, 0.0, 0.0};
+    // one 64-deep product: A(row, m) = a[m b + row], B(m, column) from the functor
+    auto product = [&](const double *a, auto bval) {
+#pragma unroll
+        for (int m0 = 0; m0 < kCT / 4; m0 += 8) {
+            double av[8][2], bv[8][2];
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+#pragma unroll
+                for (int x = 0; x < 2; ++x) {
+                    const int m = 4 * (m0 + u) + g;
+                    av[u][x] = a[(size_t)m * b + wr + 16 * x + q];
+                    bv[u][x] = bval(m, wc + 16 * x + q);
+                }
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+#pragma unroll
+                for (int x = 0; x < 2; ++x)
+#pragma unroll
+                    for (int y = 0; y < 2; ++y)
+                        acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[u][x], bv[u][y],
+                                                                         acc[x][y], 0, 0, 0);
+        }
+    };
+    for (int k = j; k < i; ++k) {
+        const double *B = dl + (size_t)k * kCT * b + j * kCT;
+        product(Lb + (size_t)k * kCT * b + i * kCT,
+                [&](int m, int c) { return B[(size_t)m * b + c]; });
+    }
+    auto to_lds = [&]() {
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int y = 0; y < 2; ++y)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    sm[wr + 16 * x + g + 4 * e][wc + 16 * y + q] = acc[x][y][e];
+                    acc[x][y][e] = 0.0;
+                }
+        __syncthreads();
+    };
+    to_lds();
+    product(Lb + (size_t)i * kCT * b + i * kCT, [&](int m, int c) { return sm[m][c]; });
     __syncthreads();
-    for (int i = ty; i < 32; i += 8) dst[off + (size_t)(i0 + i) * b + j0 + tx] = tile[tx][i];
+    to_lds();
+    for (int e = tid; e < kCT * kCT; e += 256) {
+        const int c = e >> 6, r = e & 63;
+        dl[(size_t)(i * kCT + c) * b + j * kCT + r] = -sm[c][r];
+        du[(size_t)(j * kCT + c) * b + i * kCT + r] = -sm[r][c];
+    }
 }
 
 __global__ void __launch_bounds__(256)
@@ -936,21 +1031,6 @@ add_block_kernel(long long n, const double *__restrict__ src, double *__restrict
          i += (long long)gridDim.x * 256)
         dst[i] += src[i];
 }
-
-#define XT_RB(...)                                                                      \
-    do {                                                                                \
-        rocblas_status st_ = (__VA_ARGS__);                                             \
-        if (st_ != rocblas_status_success) {                                            \
-            ::xt::set_error("%s:%d %s -> rocblas status %d", __FILE__, __LINE__,        \
-                            #__VA_ARGS__, (int)st_);                                    \
-            return XT_E_HIP;                                                            \
-        }                                                                               \
-    } while (0)
-
-struct RbHandle {
-    rocblas_handle h = nullptr;
-    ~RbHandle() { if (h) rocblas_destroy_handle(h); }
-};
 
 static int zero_fill(double *d, long long n, hipStream_t s) {
     if (n <= 0) return XT_OK;
@@ -1147,7 +1227,31 @@ static int factor_dev(BandPrec &bp, const int *dia, const int *dja, const double
     if (fb >= nb || !band_has_fp64(&bp) || !bp.Dl[0].ptr) fb = 0;
     const int ft = std::min(fb, nt);              // first block factored here
     const int nr = nb - ft, e0 = std::max(0, ft - 1), ne = nb - 1 - e0;
-    DevBuf L, E, Dl, G, H, info, E0, Km;
+    DevBuf &L = bp.sL, &E = bp.sE, &Wb = bp.sW, &Km = bp.sK, &info = bp.sinfo;
+    struct Release {   // the scratch is freed on every way out unless it is kept
+        BandPrec &bp;
+        ~Release() {
+            DevBuf *b[5] = {&bp.sL, &bp.sE, &bp.sW, &bp.sK, &bp.sinfo};
+            size_t sum = 0;
+            for (DevBuf *d : b) sum += d->bytes;
+            if (bp.built && bp.keep64 && sum <= kKeepScratch) return;
+            for (DevBuf *d : b) d->release();
+            delete bp.rb;
+            bp.rb = nullptr;
+        }
+    } release{bp};
+    struct Band {      // a failed factorization leaves the old factor's layout
+        BandPrec &bp;
+        const int kw, rc;
+        bool ok = false;
+        ~Band() {
+            if (!ok) {
+                bp.kw = kw;
+                bp.rc = rc;
+            }
+        }
+    } band{bp, bp.kw, bp.rc};
+    DevBuf E0;
     XT_TRY(L.reserve(sizeof(double) * bb * nr));
     XT_TRY(zero_fill(L.as<double>(), bb * nr, s));
     if (ne > 0) {
@@ -1170,7 +1274,11 @@ static int factor_dev(BandPrec &bp, const int *dia, const int *dja, const double
         }
         if (flags[1] > bp.kw) {   // a wider band than the factor had, within its blocks
             set_band(bp, flags[1]);
-            if (ft > 0) return factor_dev(bp, dia, dja, da, s, 0);
+            if (ft > 0) {
+                const int rc0 = factor_dev(bp, dia, dja, da, s, 0);
+                band.ok = rc0 == XT_OK;
+                return rc0;
+            }
         }
     }
     XT_HIP(hipMemsetAsync(info.ptr, 0, sizeof(int) * (nb + 2), s));
@@ -1179,8 +1287,10 @@ static int factor_dev(BandPrec &bp, const int *dia, const int *dja, const double
     double *Lp = L.as<double>(), *Ep = E.as<double>();
     auto Lat = [&](int beta) { return Lp + (beta - ft) * bb; };   // diagonal block beta
     auto Eat = [&](int e) { return Ep + (e - e0) * bb; };         // sub-diagonal block e
-    RbHandle rb;
-    XT_RB(rocblas_create_handle(&rb.h));
+    if (!bp.rb) bp.rb = new (std::nothrow) RbHandle;
+    if (!bp.rb) return XT_E_NOMEM;
+    RbHandle &rb = *bp.rb;
+    if (!rb.h) XT_RB(rocblas_create_handle(&rb.h));
     XT_RB(rocblas_set_stream(rb.h, s));
     XT_RB(rocblas_set_pointer_mode(rb.h, rocblas_pointer_mode_host));
     if (ft > 0) {
@@ -1200,7 +1310,6 @@ static int factor_dev(BandPrec &bp, const int *dia, const int *dja, const double
     // of both chains at once; the last bottom block's update of the middle block goes to Km
     // (both chains may end in the same launch)
     int *ip = info.as<int>();
-    DevBuf Wb;
     const long long wsize = 2LL * (b / kCT) * kCT * kCT;
     XT_TRY(Wb.reserve(sizeof(double) * 4 * wsize));
     CholRun run[2];
@@ -1254,23 +1363,18 @@ static int factor_dev(BandPrec &bp, const int *dia, const int *dja, const double
             set_error("K is not positive definite (block %d, minor %d)", i, hinfo[i]);
             return XT_E_SINGULAR;
         }
-    hipLaunchKernelGGL(zero_upper_kernel, dim3(ceil_div(bb, 256 * 8), nr), dim3(256), 0, s, b, Lp);
-    XT_HIP(hipGetLastError());
-    // D_i = L_ii^-1 in place (column-major lower = D_i^T row-major: the backward set)
-    XT_RB(rocsolver_dtrtri_strided_batched(rb.h, rocblas_fill_lower, rocblas_diagonal_non_unit,
-                                           b, Lp, b, bb, ip + ft, nr));
-    XT_HIP(hipMemcpyAsync(hinfo.data(), ip, sizeof(int) * nb, hipMemcpyDeviceToHost, s));
-    XT_HIP(hipStreamSynchronize(s));
-    for (int i = ft; i < nb; ++i)
-        if (hinfo[i] != 0) {
-            set_error("singular diagonal factor block %d", i);
-            return XT_E_SINGULAR;
-        }
-    // nothing can fail numerically from here on: a partial factorization writes the new
-    // blocks into the kept sets, a full one into new ones
+    // nothing can fail numerically from here on: the new blocks go into the factor's own
+    // arrays (a full factorization's into new ones where those are missing or too small,
+    // allocated before anything is overwritten); an apply still running on another stream
+    // is waited for
     const bool full = ft == 0;
     int nlev = bp.nlev;
-    DevBuf lv[2][kLevels];
+    DevBuf fresh[4 + 2 * kLevels];
+    DevBuf *sets[4 + 2 * kLevels];
+    size_t bytes[4 + 2 * kLevels] = {};
+    for (int k = 0; k < 4 + 2 * kLevels; ++k)
+        sets[k] = k == 0 ? bp.Dl : k == 1 ? bp.Du : k == 2 ? bp.G : k == 3 ? bp.H
+                : bp.Lv[(k - 4) / kLevels][(k - 4) % kLevels];
     if (full) {
         // the levels that pay for the fewest columns (more columns use fewer of them);
         // XT_TUNE_BAND_LEVELS v: v - 1 levels (set before the factor is built)
@@ -1278,34 +1382,35 @@ static int factor_dev(BandPrec &bp, const int *dia, const int *dja, const double
         nlev = 0;
         while (nlev < maxlev && (nt >> (nlev + 1)) >= kMinChain) ++nlev;
         if (!kn) nlev = std::max(chain_levels(bp, nlev, 16, 8), chain_levels(bp, nlev, 16, 4));
-        XT_TRY(Dl.reserve(sizeof(double) * bb * nb));
-        if (nb > 1) {
-            XT_TRY(G.reserve(sizeof(double) * bk * (nb - 1)));
-            XT_TRY(H.reserve(sizeof(double) * bk * (nb - 1)));
-        }
+        bytes[0] = bytes[1] = sizeof(double) * bb * nb;
+        bytes[2] = bytes[3] = sizeof(double) * bk * (nb - 1);
         for (int dir = 0; dir < 2; ++dir)
             for (int l = 1; l <= nlev; ++l)
-                XT_TRY(lv[dir][l - 1].reserve(sizeof(double) * rc * (size_t)kw *
-                                              ((bp.steps(0, dir) >> l) + (bp.steps(1, dir) >> l))));
-    } else {
-        XT_HIP(hipMemcpyAsync(bp.Du[0].as<double>() + ft * bb, Lp, sizeof(double) * bb * nr,
-                              hipMemcpyDeviceToDevice, s));
+                bytes[4 + dir * kLevels + l - 1] = sizeof(double) * rc * (size_t)kw *
+                    ((bp.steps(0, dir) >> l) + (bp.steps(1, dir) >> l));
+        for (int k = 0; k < 4 + 2 * kLevels; ++k)
+            if (bytes[k] > sets[k][0].bytes) XT_TRY(fresh[k].reserve(bytes[k]));
     }
-    double *Dlp = full ? Dl.as<double>() : bp.Dl[0].as<double>();
-    double *Gp = full ? G.as<double>() : bp.G[0].as<double>();
-    double *Hp = full ? H.as<double>() : bp.H[0].as<double>();
-    hipLaunchKernelGGL(transpose_kernel, dim3(b / 32, b / 32, nr), dim3(256), 0, s, b,
-                       (const double *)Lp, Dlp + ft * bb);
+    XT_HIP(hipDeviceSynchronize());
+    auto dst = [&](int k) { return fresh[k].ptr ? fresh[k].as<double>() : sets[k][0].as<double>(); };
+    double *Dlp = dst(0), *Dup = dst(1), *Gp = dst(2), *Hp = dst(3);
+    // D_i = L_ii^-1: column-major lower = D_i^T row-major, the backward set, and row-major
+    const int ntl = b / kCT;
+    for (int d = 0; d < ntl; ++d)
+        hipLaunchKernelGGL(tri_inverse_kernel, dim3(d == 0 ? ntl * (ntl + 1) / 2 : ntl - d, nr),
+                           dim3(256), 0, s, b, ntl, d, (const double *)Lp, Dup + ft * bb,
+                           Dlp + ft * bb);
     XT_HIP(hipGetLastError());
+    auto Dat = [&](int beta) { return Dup + beta * bb; };
     // top chain: G_i from E_{ft-1} (with the new D_ft) on, H_i from block ft on; bottom chain:
     // all, its last block coupled to the middle block by the middle's last rows
-    XT_TRY(g_products(rb.h, bp, Eat(e0), 0, Lat(e0 + 1), Gp + e0 * bk, nt - e0));
-    XT_TRY(h_products(rb.h, bp, Eat(ft), 0, Lat(ft), Hp + ft * bk, nt - ft));
-    XT_TRY(g_products(rb.h, bp, Eat(nt), 0, Lat(nt + 2), Gp + nt * bk, nbt - 1));
-    XT_TRY(h_products(rb.h, bp, Eat(nt), 0, Lat(nt + 1), Hp + nt * bk, nbt - 1));
+    XT_TRY(g_products(rb.h, bp, Eat(e0), 0, Dat(e0 + 1), Gp + e0 * bk, nt - e0));
+    XT_TRY(h_products(rb.h, bp, Eat(ft), 0, Dat(ft), Hp + ft * bk, nt - ft));
+    XT_TRY(g_products(rb.h, bp, Eat(nt), 0, Dat(nt + 2), Gp + nt * bk, nbt - 1));
+    XT_TRY(h_products(rb.h, bp, Eat(nt), 0, Dat(nt + 1), Hp + nt * bk, nbt - 1));
     if (nbt > 0) {
-        XT_TRY(g_products(rb.h, bp, Eat(nb - 2), b - kw, Lat(nt), Gp + (nb - 2) * bk, 1));
-        XT_TRY(h_products(rb.h, bp, Eat(nb - 2), b - kw, Lat(nb - 1), Hp + (nb - 2) * bk, 1));
+        XT_TRY(g_products(rb.h, bp, Eat(nb - 2), b - kw, Dat(nt), Gp + (nb - 2) * bk, 1));
+        XT_TRY(h_products(rb.h, bp, Eat(nb - 2), b - kw, Dat(nb - 1), Hp + (nb - 2) * bk, 1));
     }
     // first changed stored entry of the top chain's levels: forward entries whose G range
     // reaches index ft - 1, backward entries whose H range reaches block ft
@@ -1317,9 +1422,8 @@ static int factor_dev(BandPrec &bp, const int *dia, const int *dja, const double
                 first[dir][l] = dir == 0 ? std::min(cnt, (ft - 1) >> l)
                                          : std::max(0, cnt - 1 - ((nt - 1 - ft) >> l));
             if (ft > 0 && dir == 1 && ft >= nt) first[dir][l] = cnt;   // no changed H
-            const double *below = l == 1 ? (dir == 0 ? Gp : Hp)
-                                  : full ? lv[dir][l - 2].as<double>() : bp.Lv[dir][l - 2][0].as<double>();
-            double *out = full ? lv[dir][l - 1].as<double>() : bp.Lv[dir][l - 1][0].as<double>();
+            const double *below = l == 1 ? (dir == 0 ? Gp : Hp) : dst(4 + dir * kLevels + l - 2);
+            double *out = dst(4 + dir * kLevels + l - 1);
             XT_TRY(level_products(rb.h, bp, 0, dir, l, first[dir][l], cnt, below, out));
             XT_TRY(level_products(rb.h, bp, 1, dir, l, 0, bp.steps(1, dir) >> l, below, out));
         }
@@ -1335,30 +1439,21 @@ static int factor_dev(BandPrec &bp, const int *dia, const int *dja, const double
                 XT_TRY(to_f32_range(bp.Lv[dir][l - 1], off, n - off, s));
             }
         XT_HIP(hipStreamSynchronize(s));
+        band.ok = true;
         return XT_OK;
     }
-    bp.Du[0] = std::move(L);
-    bp.Dl[0] = std::move(Dl);
-    bp.G[0] = std::move(G);
-    bp.H[0] = std::move(H);
-    for (int dir = 0; dir < 2; ++dir)
-        for (int l = 0; l < kLevels; ++l) bp.Lv[dir][l][0] = std::move(lv[dir][l]);
+    band.ok = true;
     bp.nlev = nlev;
     for (int k = 0; k < 4 + 2 * kLevels; ++k) {
-        DevBuf *src = k == 0 ? bp.Dl : k == 1 ? bp.Du : k == 2 ? bp.G : k == 3 ? bp.H
-                    : bp.Lv[(k - 4) / kLevels][(k - 4) % kLevels];
-        if (!src[0].ptr) continue;
-        const long long n = (long long)(src[0].bytes / sizeof(double));
-        XT_TRY(src[1].reserve(sizeof(float) * n));
-        XT_TRY(to_f32_range(src, 0, n, s));
+        if (fresh[k].ptr) sets[k][0] = std::move(fresh[k]);
+        if (bytes[k] == 0) continue;
+        XT_TRY(sets[k][1].reserve(bytes[k] / 2));
+        XT_TRY(to_f32_range(sets[k], 0, (long long)(bytes[k] / sizeof(double)), s));
     }
     XT_HIP(hipStreamSynchronize(s));
     if (!bp.keep64)
-        for (int k = 0; k < 4 + 2 * kLevels; ++k) {
-            DevBuf *src = k == 0 ? bp.Dl : k == 1 ? bp.Du : k == 2 ? bp.G : k == 3 ? bp.H
-                        : bp.Lv[(k - 4) / kLevels][(k - 4) % kLevels];
-            src[0].release();
-        }
+        for (DevBuf *set : sets) set[0].release();
+    bp.built = true;
     return XT_OK;
 }
 
