@@ -538,6 +538,11 @@ int xt_graphs_enable(int on);
  *   XT_TUNE_BAND_PAIR     banded-factor sweeps: the factor's pairing levels never 1,
  *                         always 2 (built-in: the levels with the least estimated time for
  *                         the columns)                                      1, 2
+ *   XT_TUNE_SPMM_GROUP    node-block SpMM, several load cases: the kernel that reads each
+ *                         neighbour's rows of X once for a group of four nodes never 1,
+ *                         always 2 (built-in: from 100000 to 300000 nodes times cases
+ *                         on, by precision and cases); where it runs, UNR, WPB and LDS
+ *                         have no effect                                    1, 2
  * XT_E_ARG for a value a knob does not take. */
 #define XT_TUNE_SPMM_UNR 0
 #define XT_TUNE_SPMM_WPB 1
@@ -555,7 +560,8 @@ int xt_graphs_enable(int on);
 #define XT_TUNE_GMRES_COMPACT 13
 #define XT_TUNE_BAND_CHAIN_FEW 14
 #define XT_TUNE_BAND_PAIR 15
-#define XT_TUNE_NKNOBS 16
+#define XT_TUNE_SPMM_GROUP 16
+#define XT_TUNE_NKNOBS 17
 int xt_tune_set(int knob, int value);
 /* Current value of a knob (0 = built-in choice), -1 for an unknown knob. */
 int xt_tune_get(int knob);

@@ -18,13 +18,20 @@
 // values (row-major) and the 3 diagonal M values (12 numbers), plus one int32
 // column-node index.
 //
-// Work mapping: one lane per (node row, load case r).  The lane accumulates the
-// 3 rows x 6 temporal columns of K X and M X for its node in registers (72 FMA
-// per block), then applies the 6x6 temporal matrices of its load case in
-// registers and stores its 18 outputs once.  A wave covers 64/LPN nodes of one
-// slice (LPN = load cases rounded up to a power of two), so loop bounds are
-// wave-uniform.  The path is for q = 6 temporal functions (three quadratic
-// temporal nodes, each with a sine enrichment: 2*nnte, main3d.f90:172).
+// Work mapping of the slices: one lane per (node row, load case r), or SPL lanes with the
+// entries split between them.  The lane accumulates the 3 rows x 6 temporal columns of
+// K X and M X for its node in registers (72 FMA per block), then applies the 6x6
+// temporal matrices of its load case in registers and stores its outputs once.  A wave
+// covers 64 / (LPN SPL) nodes of one slice (LPN = load cases rounded up to a power of
+// two), so loop bounds are wave-uniform.
+//
+// Storage ("node groups", kron_group_kernel, several load cases on enough nodes): kG
+// consecutive nodes share the sorted union of their neighbours; the blocks stand
+// neighbour by neighbour (only the couplings that exist), so a wave whose lanes are
+// columns reads each neighbour's rows of X once for all nodes of the group.
+//
+// The path is for q = 6 temporal functions (three quadratic temporal nodes, each with a
+// sine enrichment: 2*nnte, main3d.f90:172).
 #include <algorithm>
 #include <vector>
 
@@ -44,6 +51,11 @@ struct BsrPlan {
     DevBuf bval32, bval64;  // [nblocks][12]
     DevBuf kmap, mmap;      // value position in bval of every CSR entry of K and of M
     long long nk = 0, nm = 0;
+    // Group form: neighbours gptr[s] .. gptr[s + 1] - 1 of group s as (node, 16 b + mask of the
+    // group's nodes it couples to), its blocks from gblk[s] + b on (nodes ascending); gkmap,
+    // gmmap as kmap, mmap.
+    int ngroups = 0;
+    DevBuf gptr, gblk, gnbr, gval32, gval64, gkmap, gmmap;
     // Staged form: the distinct column nodes of each slice (its neighbour set, sorted),
     // unode[ubase[s] .. ubase[s] + ulen[s]), and for every stored block the position of
     // its column node in that list (uint16), so a workgroup can stage the slice's rows
@@ -53,9 +65,24 @@ struct BsrPlan {
 };
 
 static constexpr int kSlice = 64;
+static constexpr int kG = 4;   // nodes of a group
+static constexpr int kTS = 73;   // LDS stride of a case's temporal matrices (odd)
 
-// Build the node-slice form; returns XT_E_UNSUPPORTED if K/M are not 3x3-blocked
-// with diagonal M blocks.
+__global__ void __launch_bounds__(256)
+bsr_scatter_kernel(long long n, const int *__restrict__ map, const int *__restrict__ gmap,
+                   const double *__restrict__ v, double *__restrict__ b64,
+                   float *__restrict__ b32, double *__restrict__ g64, float *__restrict__ g32);
+__global__ void __launch_bounds__(256) bsr_zero_kernel(long long n, double *d, float *f) {
+    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) {
+        d[i] = 0.0;
+        f[i] = 0.0f;
+    }
+}
+int bsr_set_values(BsrPlan &P, const double *kv, const double *mv, hipStream_t s);
+
+// Build the node-slice and node-group forms (kv, mv: the CSR values on the device); returns
+// XT_E_UNSUPPORTED if K/M are not 3x3-blocked with diagonal M blocks.
 int bsr_build(int p, const int *krp, const int *kci, const double *kv, const int *mrp,
               const int *mci, const double *mv, BsrPlan &P) {
     if (p % 3) return XT_E_UNSUPPORTED;
@@ -106,10 +133,41 @@ int bsr_build(int p, const int *krp, const int *kci, const double *kv, const int
     }
     if (nb * 12 > 0x7fffffffLL) return XT_E_UNSUPPORTED;
     std::vector<int> bcol(nb);
-    std::vector<double> bval((size_t)nb * 12, 0.0);
-    std::vector<int> pos(nn, -1);  // position of column node b in the current row
-    std::vector<int> kmap(krp[p]), mmap(mrp[p]);
+    std::vector<int> pos(nn, -1), gat(nn, 0);  // entry and group block of column node b in the row
+    std::vector<int> kmap(krp[p]), mmap(mrp[p]), gkmap(krp[p]), gmmap(mrp[p]);
+    // groups: merge the kG sorted neighbour lists; gpos: block of each of row a's neighbours,
+    // from cfirst[a] on
+    const int ngroups = ceil_div(nn, kG);
+    std::vector<int> gptr(ngroups + 1, 0), gblk(ngroups + 1, 0), gnbr;
+    std::vector<int> cfirst(nn + 1, 0);
+    for (int a = 0; a < nn; ++a) cfirst[a + 1] = cfirst[a] + (int)cols[a].size();
+    std::vector<int> gpos(cfirst[nn]);
+    {
+        int blk = 0;
+        for (int s = 0; s < ngroups; ++s) {
+            const int a0 = s * kG, na = std::min(kG, nn - a0);
+            int at[kG] = {};
+            gblk[s] = blk;
+            for (;;) {
+                int m = nn;
+                for (int i = 0; i < na; ++i)
+                    if (at[i] < (int)cols[a0 + i].size()) m = std::min(m, cols[a0 + i][at[i]]);
+                if (m == nn) break;
+                int e = (blk - gblk[s]) << 4;
+                for (int i = 0; i < na; ++i)
+                    if (at[i] < (int)cols[a0 + i].size() && cols[a0 + i][at[i]] == m) {
+                        gpos[cfirst[a0 + i] + at[i]++] = blk++;
+                        e |= 1 << i;
+                    }
+                gnbr.push_back(m);
+                gnbr.push_back(e);
+            }
+            gptr[s + 1] = (int)(gnbr.size() / 2);
+        }
+        gblk[ngroups] = blk;
+    }
     long long nreal = 0;
+    std::vector<int> klast(p, -1), mlast(p, -1);   // last entry of a column (of this row: >= its first)
     for (int s = 0; s < nslices; ++s)
         for (int k = 0; k < kSlice; ++k) {
             const int a = s * kSlice + k;
@@ -140,19 +198,24 @@ int bsr_build(int p, const int *krp, const int *kci, const double *kv, const int
             } else {
                 for (int e = 0; e < (int)c.size(); ++e) pos[c[e]] = e;
             }
+            for (int e = 0; e < (int)c.size(); ++e) gat[c[e]] = gpos[cfirst[a] + e];
             for (int d = 0; d < 3; ++d) {
                 const int i = 3 * a + d;
                 for (int e = krp[i]; e < krp[i + 1]; ++e) {
                     const int b = kci[e] / 3, cd = kci[e] % 3;
                     const long long idx = (long long)base[s] + (long long)pos[b] * kSlice + k;
-                    bval[idx * 12 + d * 3 + cd] = kv[e];
                     kmap[e] = (int)(idx * 12 + d * 3 + cd);
+                    gkmap[e] = gat[b] * 12 + d * 3 + cd;
+                    if (klast[kci[e]] >= krp[i]) kmap[klast[kci[e]]] = -1;   // the last one stands
+                    klast[kci[e]] = e;
                 }
                 for (int e = mrp[i]; e < mrp[i + 1]; ++e) {
                     const int b = mci[e] / 3;
                     const long long idx = (long long)base[s] + (long long)pos[b] * kSlice + k;
-                    bval[idx * 12 + 9 + d] = mv[e];
                     mmap[e] = (int)(idx * 12 + 9 + d);
+                    gmmap[e] = gat[b] * 12 + 9 + d;
+                    if (mlast[mci[e]] >= mrp[i]) mmap[mlast[mci[e]]] = -1;
+                    mlast[mci[e]] = e;
                 }
             }
             for (int b : c) pos[b] = -1;
@@ -198,9 +261,24 @@ int bsr_build(int p, const int *krp, const int *kci, const double *kv, const int
     P.nm = mrp[p];
     if (P.nk) XT_TRY(P.kmap.upload(kmap.data(), sizeof(int) * P.nk));
     if (P.nm) XT_TRY(P.mmap.upload(mmap.data(), sizeof(int) * P.nm));
-    XT_TRY(P.bval64.upload(bval.data(), sizeof(double) * bval.size()));
-    std::vector<float> b32(bval.begin(), bval.end());
-    XT_TRY(P.bval32.upload(b32.data(), sizeof(float) * b32.size()));
+    if (P.nk) XT_TRY(P.gkmap.upload(gkmap.data(), sizeof(int) * P.nk));
+    if (P.nm) XT_TRY(P.gmmap.upload(gmmap.data(), sizeof(int) * P.nm));
+    P.ngroups = ngroups;
+    XT_TRY(P.gptr.upload(gptr.data(), sizeof(int) * gptr.size()));
+    XT_TRY(P.gblk.upload(gblk.data(), sizeof(int) * gblk.size()));
+    XT_TRY(P.gnbr.upload(gnbr.data(), sizeof(int) * gnbr.size()));
+    // the values, from the CSR values already on the device
+    const long long nv = nb * 12, ng = ((long long)gblk[ngroups] + 1) * 12;
+    XT_TRY(P.bval64.reserve(sizeof(double) * nv));
+    XT_TRY(P.bval32.reserve(sizeof(float) * nv));
+    XT_TRY(P.gval64.reserve(sizeof(double) * ng));
+    XT_TRY(P.gval32.reserve(sizeof(float) * ng));
+    hipLaunchKernelGGL(bsr_zero_kernel, dim3(ceil_div(nv, 256)), dim3(256), 0, 0, nv,
+                       P.bval64.as<double>(), P.bval32.as<float>());
+    hipLaunchKernelGGL(bsr_zero_kernel, dim3(ceil_div(ng, 256)), dim3(256), 0, 0, ng,
+                       P.gval64.as<double>(), P.gval32.as<float>());
+    XT_HIP(hipGetLastError());
+    XT_TRY(bsr_set_values(P, kv, mv, 0));
     XT_HIP(hipDeviceSynchronize());
     return XT_OK;
 }
@@ -462,6 +540,304 @@ kron_bsr3_lds_kernel(int nslices, int nch, const int *__restrict__ slot_node,
     }
 }
 
+using F4 = float __attribute__((ext_vector_type(4)));
+
+// Value of the neighbouring lane of a pair (2 k, 2 k + 1), by DPP.
+static __device__ inline float pair_swap(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, true));
+}
+static __device__ inline double pair_swap(double v) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0xB1, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0xB1, 0xF, 0xF, true);
+    return __hiloint2double(hi, lo);
+}
+
+// Row I of a node's block times the neighbour's X, three columns: K += the row's three
+// values times X, M += its mass value times X's row I.  Lane t of each row of 16 lanes
+// holds value t of the block; the row broadcast is part of each multiply-add.  (Two wait
+// states stand between a write of kv and its first use by a lane-crossing operand.)
+template <int I>
+static __device__ inline void block_row(double kv, const double (&x)[3][3], double (&k)[3],
+                                        double (&m)[3]) {
+#define XT_FMA(acc, val, xv)                                                                   \
+    "v_fmac_f64_dpp " acc ", %6, " xv " row_newbcast:" val                                     \
+    " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+#define XT_BLOCK_ROW                                                                     \
+    asm("s_nop 1\n\t"                                                                          \
+        XT_FMA("%0", "%16", "%7") XT_FMA("%1", "%16", "%8") XT_FMA("%2", "%16", "%9")          \
+        XT_FMA("%3", "%19", "%20") XT_FMA("%4", "%19", "%21") XT_FMA("%5", "%19", "%22")       \
+        XT_FMA("%0", "%17", "%10") XT_FMA("%1", "%17", "%11") XT_FMA("%2", "%17", "%12")       \
+        XT_FMA("%0", "%18", "%13") XT_FMA("%1", "%18", "%14") XT_FMA("%2", "%18", "%15")       \
+        : "+&v"(k[0]), "+&v"(k[1]), "+&v"(k[2]), "+&v"(m[0]), "+&v"(m[1]), "+&v"(m[2])               \
+        : "v"(kv), "v"(x[0][0]), "v"(x[0][1]), "v"(x[0][2]), "v"(x[1][0]), "v"(x[1][1]),       \
+          "v"(x[1][2]), "v"(x[2][0]), "v"(x[2][1]), "v"(x[2][2]), "n"(3 * I), "n"(3 * I + 1),  \
+          "n"(3 * I + 2), "n"(9 + I), "v"(x[I][0]), "v"(x[I][1]), "v"(x[I][2]))
+    XT_BLOCK_ROW;
+#undef XT_FMA
+}
+template <int I>
+static __device__ inline void block_row(float kv, const float (&x)[3][3], float (&k)[3],
+                                        float (&m)[3]) {
+#define XT_FMA(acc, val, xv)                                                                   \
+    "v_fmac_f32_dpp " acc ", %6, " xv " row_newbcast:" val                                     \
+    " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+    XT_BLOCK_ROW;
+#undef XT_FMA
+#undef XT_BLOCK_ROW
+}
+
+// Several load cases: 2 lanes per load case (three temporal columns each), so a group of kG
+// nodes takes LPG lanes (2 per case, whole rows of 16) and a wave holds 64 / LPG groups
+// ("slots").  Each neighbour's rows of X are read once for the group, two neighbours ahead,
+// 16 bytes and 8 a lane so that a row costs the address unit 2 instructions of 16 cycles
+// (24-byte pieces a lane cost 64 each, 8-byte ones three of 16).  The blocks are staged in
+// LDS, CH neighbours (up to CH kG blocks) at a time; a row of 16 lanes reads a block's 12
+// values, one a lane, and they enter the multiply-adds by row broadcast.  A wave goes on to
+// its next groups, the first chunk of which is loaded during the last of the one before.
+//
+// 145323 nodes (241 x 201 x 3), 32 cases, FP64: 1704 us by the slice kernel (every lane loads
+// its node's block and its neighbours' rows: 15 loads an entry through the CU's vector
+// cache), 687 here.  Block values through scalar loads, a column or three a lane: 1460,
+// 1160 (a dependent scalar load a block); by LDS reads of 16 bytes at one address: 880;
+// one neighbour ahead, one group a wave: 760.  What is left: the rows of X reach a CU at 9 TB/s over
+// all CUs with half of them missing the L2 (the vector cache waits on about 80 lines of 128
+// bytes at 600 cycles each), and the clock sinks to 1.7 - 1.9 GHz.  Groups taken in strips of
+// the section rather than in order halve the misses for 10 % of the time, but need the
+// section's width, which the pattern does not give.
+template <typename T, int LPG>
+struct GroupGeom {
+    static constexpr int CH = LPG >= 48 ? 6 : 3;              // neighbours of a chunk
+    static constexpr int PPB = 12 * sizeof(T) / 16;           // 16-byte pieces of a block
+    static constexpr int VP = CH * kG * PPB;                  // pieces of a chunk, at most
+    static constexpr int NQ = (VP + LPG - 1) / LPG;
+    static constexpr int MIX = 18 * LPG * sizeof(T) / 16;     // a node's rows of K X and M X
+    static constexpr int SLOT = (VP > MIX ? VP : MIX) + (CH + 3) / 2;
+    static constexpr int NS = 64 / LPG;
+    static constexpr int BPC = sizeof(T) == 4 ? 3 : 2;        // workgroups a CU
+};
+
+template <typename T, int LPG>
+__global__ void __launch_bounds__(256, (GroupGeom<T, LPG>::BPC))
+kron_group_kernel(int ngroups, int nn, const int *__restrict__ gptr,
+                  const int *__restrict__ gblk, const int2 *__restrict__ gnbr,
+                  const T *__restrict__ gval, int R, int per, int c,
+                  const T *__restrict__ tmat, T alpha, T beta, const T *__restrict__ x,
+                  T *__restrict__ y) {
+    using G = GroupGeom<T, LPG>;
+    constexpr int CH = G::CH, PPB = G::PPB;
+    using T2 = T __attribute__((ext_vector_type(2), aligned(sizeof(T))));
+    extern __shared__ F4 smem[];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const bool spare = lane >= G::NS * LPG;      // spare lanes repeat slot 0 and store nothing
+    const int slot = spare ? 0 : lane / LPG;
+    const int li = spare ? lane - G::NS * LPG : lane - slot * LPG;
+    const int r0 = blockIdx.y * per, cc = min(R - r0, per) * 6;   // the chunk's columns
+    F4 *sv = smem + (size_t)(wave * G::NS + slot) * G::SLOT;
+    int2 *se = (int2 *)(sv + G::SLOT - (CH + 3) / 2);   // CH + 2 entries
+    T *st = (T *)(smem + (size_t)4 * G::NS * G::SLOT);            // the chunk's temporal matrices
+    // this wave's items of NS groups: each XCD has an eighth of them, its waves side by side
+    const int items = (ngroups + G::NS - 1) / G::NS, perx = (items + 7) / 8;
+    const int xcd = blockIdx.x & 7, step = (int)(gridDim.x >> 3) * 4;
+    const int end = min(items, (xcd + 1) * perx);
+    int item = xcd * perx + (int)(blockIdx.x >> 3) * 4 + wave;
+    // a slot that fills the wave has uniform entries
+    auto uni = [](int v) { return LPG == 64 ? __builtin_amdgcn_readfirstlane(v) : v; };
+    // this lane's columns, wide and contiguous across the slot's lanes: two, then one
+    const int p0 = 2 * li, p2 = 2 * LPG + li;
+    const int c0 = p0 < cc ? p0 : 0, c2 = p2 < cc ? p2 : 0;
+    const T *xc = x + (size_t)r0 * 6;
+    auto gather = [&](int m, T (&xv)[3][3]) {
+        const T *q = xc + (size_t)m * 3 * c;
+#pragma unroll
+        for (int d = 0; d < 3; ++d, q += c) {
+            const T2 w = *(const T2 *)(q + c0);
+            xv[d][0] = w[0];
+            xv[d][1] = w[1];
+            xv[d][2] = q[c2];
+        }
+    };
+    struct Group {
+        int grp, u0, u1, b0, b1;   // neighbours u0 .. u1 - 1, blocks b0 .. b1 - 1
+    };
+    auto group_of = [&](int it) {   // (the last group where there is none)
+        Group g;
+        const int q = it * G::NS + slot;
+        g.grp = uni(q < ngroups ? q : ngroups - 1);
+        g.u0 = gptr[g.grp];
+        g.u1 = gptr[g.grp + 1];
+        g.b0 = gblk[g.grp];
+        g.b1 = gblk[g.grp + 1];
+        return g;
+    };
+    F4 rq[G::NQ] = {};
+    int2 re = {};
+    // chunk of a group: neighbours from us on, blocks from the group's block off on
+    auto fetch = [&](int us, int u1, int b0, int b1, int off) {
+        re = gnbr[us + li < u1 ? us + li : u1 - 1];
+        const F4 *vsrc = (const F4 *)(gval + (size_t)b0 * 12);
+        const int last = max((b1 - b0) * PPB - 1, 0);
+#pragma unroll
+        for (int i = 0; i < G::NQ; ++i) {
+            const int q = off * PPB + i * LPG + li;
+            rq[i] = vsrc[q < last ? q : last];
+        }
+    };
+    Group cur = group_of(item);
+    fetch(cur.u0, cur.u1, cur.b0, cur.b1, 0);
+    {   // (unrolled: the loads are in flight together, and with those above)
+        T v[9];
+#pragma unroll
+        for (int q = 0; q < 9; ++q) {
+            const int e = threadIdx.x + 256 * q, k = e / 72, j = e - k * 72;
+            if (k < per) v[q] = tmat[(size_t)(r0 + min(k, R - r0 - 1)) * 72 + j];
+        }
+#pragma unroll
+        for (int q = 0; q < 9; ++q) {
+            const int e = threadIdx.x + 256 * q, k = e / 72, j = e - k * 72;
+            if (k < per) st[k * kTS + j] = v[q];
+        }
+    }
+    __syncthreads();
+    const int kc = min(li >> 1, per - 1), j0 = (li & 1) * 3;
+    const T *own = st + kc * kTS + j0 * 7, *other = st + kc * kTS + j0 * 5 + 3;
+    T *sm = (T *)sv;
+    for (; item < end; item += step) {
+        const Group next = group_of(item + step < end ? item + step : item);
+        int us = cur.u0, trips = (cur.u1 - us + CH - 1) / CH;   // the longest slot's
+#pragma unroll
+        for (int o = 32; o >= LPG; o >>= 1) trips = max(trips, __shfl_xor(trips, o));
+        trips = __builtin_amdgcn_readfirstlane(trips);
+        T aK[kG][3][3], aM[kG][3][3];
+#pragma unroll
+        for (int g = 0; g < kG; ++g)
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+#pragma unroll
+                for (int n = 0; n < 3; ++n) { aK[g][i][n] = T(0); aM[g][i][n] = T(0); }
+        auto stage = [&]() {
+            __builtin_amdgcn_wave_barrier();   // (a wave's LDS accesses complete in order)
+            if (li < CH + 2) se[li] = make_int2(re.x, us + li < cur.u1 ? re.y : 0);   // 0: past the end
+#pragma unroll
+            for (int i = 0; i < G::NQ; ++i)
+                if (i * LPG + li < G::VP) sv[i * LPG + li] = rq[i];
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        };
+        stage();
+        T xv[3][3][3];   // two neighbours ahead
+        gather(uni(se[0].x), xv[0]);
+        gather(uni(se[1].x), xv[1]);
+        for (;;) {
+            {   // the next chunk, of this group or of the next
+                const bool more = trips > 1;
+                const int off = se[CH].y >> 4;
+                fetch(more ? (us + CH < cur.u1 ? us + CH : cur.u1) : next.u0,
+                      more ? cur.u1 : next.u1, more ? cur.b0 : next.b0, more ? cur.b1 : next.b1,
+                      more ? off : 0);
+            }
+            const T *bv = (const T *)sv + min(lane & 15, 11);
+            T kv = *bv;
+            auto neighbour = [&](int mask, const T (&xv)[3][3]) {
+#pragma unroll
+                for (int g = 0; g < kG; ++g) {
+                    if (!((mask >> g) & 1)) continue;
+                    bv += 12;
+                    const T nx = *bv;   // (past the last block: what stands behind it)
+                    block_row<0>(kv, xv, aK[g][0], aM[g][0]);
+                    block_row<1>(kv, xv, aK[g][1], aM[g][1]);
+                    block_row<2>(kv, xv, aK[g][2], aM[g][2]);
+                    kv = nx;
+                }
+            };
+            int2 e0 = se[0], e1 = se[1];
+#pragma unroll
+            for (int t = 0; t < CH; ++t) {
+                const int2 e2 = se[t + 2];
+                gather(uni(e2.x), xv[(t + 2) % 3]);
+                __builtin_amdgcn_sched_barrier(0);
+                neighbour(uni(e0.y) & 15, xv[t % 3]);
+                __builtin_amdgcn_sched_barrier(0);
+                e0 = e1;
+                e1 = e2;
+            }
+            if (--trips == 0) break;
+            us += CH;
+            stage();
+        }
+        // Y = K X A^T + M X B^T, a node at a time: through LDS to three consecutive columns a
+        // lane (the case's other three are its pair lane's) and back.
+        const bool out_slot = !spare && item * G::NS + slot < ngroups;
+        T ta[3][6], tb[3][6];   // own columns first, then the pair lane's
+#pragma unroll
+        for (int g = 0; g < kG; ++g) {
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                T *sk = sm + i * 6 * LPG;
+                sk[p0] = aK[g][i][0];
+                sk[p0 + 1] = aK[g][i][1];
+                sk[p2] = aK[g][i][2];
+                sk[3 * LPG + p0] = aM[g][i][0];
+                sk[3 * LPG + p0 + 1] = aM[g][i][1];
+                sk[3 * LPG + p2] = aM[g][i][2];
+            }
+            if (g == 0) {
+#pragma unroll
+                for (int n = 0; n < 3; ++n)
+#pragma unroll
+                    for (int j = 0; j < 6; ++j) {
+                        const T *t = (j < 3 ? own : other) + n * 6 + (j < 3 ? j : j - 3);
+                        ta[n][j] = t[0];
+                        tb[n][j] = t[36];
+                    }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                T *sk = sm + i * 6 * LPG + 3 * li;
+                T out[3] = {T(0), T(0), T(0)};
+#pragma unroll
+                for (int j = 0; j < 3; ++j) {
+                    const T zk = sk[j], zm = sk[3 * LPG + j];
+                    const T pk = pair_swap(zk), pm = pair_swap(zm);
+#pragma unroll
+                    for (int n = 0; n < 3; ++n) {
+                        out[n] += ta[n][j] * zk + tb[n][j] * zm;
+                        out[n] += ta[n][3 + j] * pk + tb[n][3 + j] * pm;
+                    }
+                }
+                // (a row's values are read by the lanes that hold them before they are replaced)
+#pragma unroll
+                for (int n = 0; n < 3; ++n) sk[n] = alpha * out[n];
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            const int node = cur.grp * kG + g;
+            if (out_slot && node < nn) {
+                T *yr = y + (size_t)node * 3 * c + (size_t)r0 * 6;
+#pragma unroll
+                for (int i = 0; i < 3; ++i, yr += c) {
+                    const T *sk = sm + i * 6 * LPG;
+                    if (p0 < cc) {
+                        T2 o = {sk[p0], sk[p0 + 1]};
+                        T2 *q = (T2 *)(yr + p0);
+                        if (beta != T(0)) {
+                            const T2 old = *q;
+                            o[0] += beta * old[0];
+                            o[1] += beta * old[1];
+                        }
+                        *q = o;
+                    }
+                    if (p2 < cc) yr[p2] = beta == T(0) ? sk[p2] : sk[p2] + beta * yr[p2];
+                }
+            }
+        }
+        cur = next;
+    }
+}
+
 // Sum over aligned groups of 4 or 8 lanes with DPP moves (swap neighbours, swap pairs
 // in a quad, mirror in the half-row): every lane of the group ends with the group's sum.
 template <int CTRL>
@@ -593,25 +969,32 @@ kron_bsr3_r1_kernel(int nslices, const int *__restrict__ slot_node,
     }
 }
 
-// New K and M values (CSR entries in the order the plan was built from) into the node
-// blocks, FP64 and FP32.
+// K and M values (CSR entries in the order the plan was built from) into the node blocks of
+// both forms, FP64 and FP32.
 __global__ void __launch_bounds__(256)
-bsr_scatter_kernel(long long n, const int *__restrict__ map, const double *__restrict__ v,
-                   double *__restrict__ b64, float *__restrict__ b32) {
+bsr_scatter_kernel(long long n, const int *__restrict__ map, const int *__restrict__ gmap,
+                   const double *__restrict__ v, double *__restrict__ b64,
+                   float *__restrict__ b32, double *__restrict__ g64, float *__restrict__ g32) {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const int t = map[i];
-    b64[t] = v[i];
-    b32[t] = (float)v[i];
+    const int t = map[i], u = gmap[i];
+    if (t < 0) return;   // an entry that a later one of the row replaces
+    const double w = v[i];
+    b64[t] = w;
+    b32[t] = (float)w;
+    g64[u] = w;
+    g32[u] = (float)w;
 }
 
 int bsr_set_values(BsrPlan &P, const double *kv, const double *mv, hipStream_t s) {
     if (P.nk)
         hipLaunchKernelGGL(bsr_scatter_kernel, dim3(ceil_div(P.nk, 256)), dim3(256), 0, s, P.nk,
-                           P.kmap.as<int>(), kv, P.bval64.as<double>(), P.bval32.as<float>());
+                           P.kmap.as<int>(), P.gkmap.as<int>(), kv, P.bval64.as<double>(),
+                           P.bval32.as<float>(), P.gval64.as<double>(), P.gval32.as<float>());
     if (P.nm)
         hipLaunchKernelGGL(bsr_scatter_kernel, dim3(ceil_div(P.nm, 256)), dim3(256), 0, s, P.nm,
-                           P.mmap.as<int>(), mv, P.bval64.as<double>(), P.bval32.as<float>());
+                           P.mmap.as<int>(), P.gmmap.as<int>(), mv, P.bval64.as<double>(),
+                           P.bval32.as<float>(), P.gval64.as<double>(), P.gval32.as<float>());
     XT_HIP(hipGetLastError());
     return XT_OK;
 }
@@ -640,6 +1023,23 @@ static int stage_cols(const BsrPlan &P, int c) {
     for (int cc : {48, 24, 12})
         if (c % cc == 0 && (size_t)P.umax * 3 * cc * sizeof(T) <= kStageLds) return cc;
     return 0;
+}
+
+// The group kernel from enough work on: a wave takes 25 (64 lanes a group) to 36 us (16) for
+// its first group, a chain of loads, whatever the number of groups.  Slices against groups,
+// us (lanes of the slice kernel: nodes times cases rounded up to a power of two):
+//   FP64  4879 nodes 16 cases 32 / 37, 17 cases 57 / 39; 23735 nodes 4 cases 36 / 57,
+//         5 cases 58 / 58, 8 cases 67 / 62, 9 cases 115 / 72; 32513 nodes 5 cases 78 / 65;
+//         61004 nodes 2 cases 55 / 83, 3 cases 85 / 86, 5 cases 144 / 89
+//   FP32  4879 nodes 32 cases 32 / 34, 33 cases 55 / 45; 23735 nodes 8 cases 38 / 48, 9 cases
+//         65 / 57; 32513 nodes 8 cases 49 / 51; 61004 nodes 4 cases 49 / 56, 5 cases 86 / 57
+static bool group_form(const BsrPlan &P, int R, bool f32) {
+    const int k = tune_knob(XT_TUNE_SPMM_GROUP);
+    if (R < 2 || k == 1) return false;
+    if (k == 2) return true;
+    int lpn = 1;
+    while (lpn < R) lpn <<= 1;
+    return (long long)P.nn * lpn >= (f32 ? 300000 : R > 16 ? 100000 : 200000);
 }
 
 template <typename T>
@@ -677,6 +1077,38 @@ int bsr_apply(const BsrPlan &P, int R, const T *tmat, double alpha, double beta,
                                  (double)(P.unode.bytes) + vec * (beta != 0 ? 3 : 2);
             const double flops = 2.0 * 12 * P.nreal * c + 2.0 * 2 * 6 * (3.0 * P.nn) * c;
             prof_end(XT_PROF_SPMM, s, bytes, flops);
+        }
+        XT_HIP(hipGetLastError());
+        return XT_OK;
+    }
+    if (group_form(P, R, f32)) {
+        // cases split evenly over launches' second dimension, at most 32 a wave
+        const int nchunk = ceil_div(R, 32), per = ceil_div(R, nchunk);
+        const T *gv = f32 ? (const T *)P.gval32.ptr : (const T *)P.gval64.ptr;
+        if (prof_on(XT_PROF_SPMM)) prof_begin(XT_PROF_SPMM, s);
+#define XT_GROUP(LPG)                                                                          \
+    {                                                                                          \
+        using G = GroupGeom<T, LPG>;                                                           \
+        const int need = ceil_div(P.ngroups, 4 * G::NS), most = std::max(1, 256 * G::BPC / nchunk); \
+        hipLaunchKernelGGL((kron_group_kernel<T, LPG>),                                        \
+                           dim3(ceil_div(std::min(need, most), 8) * 8, nchunk),                \
+                           dim3(256), 64 * G::NS * G::SLOT + sizeof(T) * kTS * per, s,         \
+                           P.ngroups, P.nn, P.gptr.as<int>(), P.gblk.as<int>(),                \
+                           P.gnbr.as<const int2>(), gv, R, per, c, tmat, (T)alpha, (T)beta, x, \
+                           y);                                                                 \
+    }
+        if (per <= 8) XT_GROUP(16)
+        else if (per <= 16) XT_GROUP(32)
+        else if (per <= 24) XT_GROUP(48)
+        else XT_GROUP(64)
+#undef XT_GROUP
+        if (prof_on(XT_PROF_SPMM)) {
+            // 12 values per block, the neighbour lists, X read, Y written (and read)
+            const double sv = sizeof(T), vec = (double)P.nn * 3 * c * sv;
+            const double bytes = (double)P.nreal * 12 * sv + (double)P.gnbr.bytes +
+                                 8.0 * P.ngroups + vec * (beta != 0 ? 3 : 2);
+            prof_end(XT_PROF_SPMM, s, bytes,
+                     2.0 * 12 * P.nreal * c + 2.0 * 2 * 6 * (3.0 * P.nn) * c);
         }
         XT_HIP(hipGetLastError());
         return XT_OK;

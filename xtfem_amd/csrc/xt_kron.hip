@@ -349,8 +349,8 @@ int xt_op_create(int p, int q, int nterms, const int *const *rowptr, const int *
         for (long long e = 0; e < nk; ++e) kci[e] = colidx[0][e] - 1;
         for (long long e = 0; e < nm; ++e) mci[e] = colidx[1][e] - 1;
         op->bsr = bsr_new();
-        int rc = bsr_build(p, krp.data(), kci.data(), vals[0], mrp.data(), mci.data(), vals[1],
-                           *op->bsr);
+        int rc = bsr_build(p, krp.data(), kci.data(), op->S[0].val64.as<double>(), mrp.data(),
+                           mci.data(), op->S[1].val64.as<double>(), *op->bsr);
         if (rc == XT_E_UNSUPPORTED) {
             bsr_delete(op->bsr);
             op->bsr = nullptr;

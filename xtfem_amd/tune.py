@@ -6,7 +6,8 @@ the launching stream (the library's per-launch profiler), the candidates of
 
 * the node-block Kron-SpMM: entries in flight per pass (2, 4, 8), waves per workgroup
   (1, 2, 4), for one load case lanes per node row (4, 8), for several the kernel that
-  stages each slice's neighbour rows of X in LDS (off, on);
+  stages each slice's neighbour rows of X in LDS (off, on) and the one that reads them
+  once for a group of four nodes (off, on);
 * the banded-factor sweeps: the tile rows of the batched passes (64, 128 in FP32), and
   for a few columns the rows of a workgroup (16, 32, or by the number of workgroups);
 * the slab solve, timed on whole solves when a solve is given: the least residual
@@ -34,7 +35,7 @@ KNOBS = {"spmm_unr": 0, "spmm_wpb": 1, "spmm_r1split": 2, "band_tile": 3, "gmres
          "spmm_lds": 5, "band_smallc": 6, "ir_fp32_cycle": 7, "ir_min_gain": 8,
          "ir_skip32": 9, "band_chain": 10, "band_levels": 11,
          "gmres_reorth": 12, "gmres_compact": 13, "band_chain_few": 14,
-         "band_pair": 15}
+         "band_pair": 15, "spmm_group": 16}
 XT_PROF_SPMM, XT_PROF_BAND, XT_PROF_BAND64 = 0, 1, 4
 _CACHE: dict = {}
 
@@ -131,8 +132,11 @@ def autotune(op, pr, R, fp32=True, reps=7, solve=None):
     spmm = lambda: op.apply(T, x, y, R, fp32=fp32)
     out = {"signature": key, "picks": {}, "timings_ms": {}}
     if op.format == "blocks":
+        if R > 1:
+            set_knob("spmm_group", 1)         # the slice kernel's variants first
         for name, cands in (("spmm_unr", (2, 4, 8)), ("spmm_wpb", (1, 2, 4))) + \
-                ((("spmm_r1split", (4, 8)),) if R == 1 else (("spmm_lds", (1, 2)),)):
+                ((("spmm_r1split", (4, 8)),) if R == 1 else
+                 (("spmm_lds", (1, 2)), ("spmm_group", (1, 2)))):
             best, res = _pick(name, cands, XT_PROF_SPMM, spmm, reps)
             out["picks"][name] = best
             out["timings_ms"][name] = res
