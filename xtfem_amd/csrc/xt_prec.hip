@@ -79,30 +79,52 @@ trsv_onewg_kernel(int n_, int nlevL, const int *__restrict__ lpL, const int *__r
         for (int i = threadIdx.x; i < n_ * c; i += blockDim.x) xg[i] = x[i];
 }
 
-// Both sweeps in one workgroup without a barrier per level: each wave takes rows in
-// level order (tasks w, w + nwaves, ... of the level-ordered rows of L, then of U) and
-// starts a row as soon as the rows it reads are finished, told by per-row flags in LDS
-// (1: forward result, 2: backward result).  Every row depends only on rows earlier in
-// that order and each wave walks its rows in that order, so the earliest unfinished
-// row can always proceed.  Each row's leading entries sit in a fixed-size slot in
-// level order, so a wave loads its next two rows' entries with no dependent address
-// while it waits for and computes the current one; the solution, the inverse diagonal
-// and the flags live in LDS.  Lanes: S slices of the row's entries times 64/S column
-// groups; the slices' partial sums are reduced by DPP lane moves in a fixed order.  Waits are bounded: a wave that waits past kSpinMax polls raises an abort
-// flag that releases every wave, and the output is then NaN.
+// Both sweeps of kSfCols columns in one workgroup without a barrier per level (the columns
+// are independent, a workgroup for each kSfCols of them): each wave takes rows in level order
+// (tasks w, w + nwaves, ... of the level-ordered rows of L, then of U) and starts a row as
+// soon as the rows it reads are finished.  The forward and the backward results live in LDS
+// and are their own flags: an entry holds a NaN of a reserved bit pattern until its value is
+// stored, so one LDS read tells a lane both that its row is finished and its value.  Every
+// row depends only on rows earlier in that order and each wave walks its rows in that order,
+// so the earliest unfinished row can always proceed.  Half a wave works on a column: the
+// entry whose row comes last in the order is left for the end, the next kSlot sit in a
+// fixed-size slot in level order, one a lane, so a wave loads its next two rows' entries with
+// no dependent address while it waits for and computes the current one, and their products
+// are summed by DPP lane moves in a fixed order before the last entry is waited for.  Waits
+// are bounded: a wave that waits past kSpinMax polls raises an abort flag that releases every
+// wave, and the output is then NaN.
+//
+// What bounds it: the chain of levels, each a store to LDS, a poll that sees it and the last
+// product, 220 to 280 ns.  6 columns: 975 rows, 286 + 243 levels 287 us (one workgroup for
+// all columns, separate flags, 8 lanes a column) -> 148; 2727 rows, 1936 + 1808 levels,
+// which did not fit one workgroup's LDS, 5 ms (a barrier a level) -> 0.84.  Without the last entry kept
+// apart 149 and 1010; polls with pauses, 8 or 16 waves: no better.
 constexpr int kSlot = 32;           // leading entries of a row kept in its fixed-size slot
+constexpr int kSfCols = 64 / kSlot; // columns of a workgroup
 constexpr int kSfMaxRows = 4096;    // slots are built for factors up to this order
 constexpr int kSpinMax = 1 << 22;
 
-// LDS: x [(n + 1) c] (row n stays zero), inverse diagonal [n], flags [n + 1] (flag[n] = 3,
-// always satisfied), row pointers of L and U [n + 1] each, abort flag.
+// LDS: forward and backward results [(n + 1) kSfCols] each (row n: always finished, zero),
+// abort flag.  (At most 131 KB.)
 template <typename T>
-static size_t sf_lds_bytes(int n, int c) {
-    return sizeof(T) * ((size_t)(n + 1) * c + n) + sizeof(int) * (3 * (size_t)n + 4);
+static size_t sf_lds_bytes(int n) {
+    return sizeof(T) * 2 * ((size_t)n + 1) * kSfCols + 16;
 }
 
-// Sum over aligned groups of S lanes (S = 4 or 8) with DPP lane moves: swap
-// neighbours, swap pairs within a quad, then mirror within the half-row of 8.
+// An entry that is not finished yet; results never hold the pattern (they are NaN then, and
+// a NaN of another pattern is stored).
+template <typename T> struct Unfinished;
+template <> struct Unfinished<double> {
+    static constexpr int kHigh = 0x7FFADEAD;
+    static __device__ __forceinline__ double pattern() { return __hiloint2double(kHigh, 0); }
+    static __device__ __forceinline__ bool is(double v) { return __double2hiint(v) == kHigh; }
+};
+template <> struct Unfinished<float> {
+    static constexpr int kBits = 0x7FDADEAD;
+    static __device__ __forceinline__ float pattern() { return __int_as_float(kBits); }
+    static __device__ __forceinline__ bool is(float v) { return __float_as_int(v) == kBits; }
+};
+
 template <int CTRL>
 __device__ __forceinline__ float dpp_move(float v) {
     return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, true));
@@ -114,141 +136,151 @@ __device__ __forceinline__ double dpp_move(double v) {
     const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xF, 0xF, true);
     return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
-template <int S, typename T>
-__device__ __forceinline__ T group_sum(T s) {
-    if (S >= 2) s += dpp_move<0xB1>(s);    // quad_perm [1,0,3,2]
-    if (S >= 4) s += dpp_move<0x4E>(s);    // quad_perm [2,3,0,1]
-    if (S >= 8) s += dpp_move<0x141>(s);   // row_half_mirror
-    return s;
+// Sum over each half of the wave, in its last 16 lanes: within each row of 16 lanes by
+// swapping neighbours, pairs, quads and eights, then the lower row's sum to the upper.
+template <typename T>
+__device__ __forceinline__ T half_sum(T s) {
+    s += dpp_move<0xB1>(s);     // quad_perm [1,0,3,2]
+    s += dpp_move<0x4E>(s);     // quad_perm [2,3,0,1]
+    s += dpp_move<0x141>(s);    // row_half_mirror
+    s += dpp_move<0x140>(s);    // row_mirror
+    return s + dpp_move<0x142>(s);   // row_bcast:15
 }
 
-__device__ __forceinline__ int lds_flag(const int *f) {
+template <typename V>
+__device__ __forceinline__ V lds_load(const V *f) {
     return __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// One triangle as the single-workgroup sweep reads it (device pointers): rows in level
-// order (bit 30 set when the row has more than kSlot entries), the first kSlot entries
-// of each of those rows in its slot (columns past the row are n, values 0), and the
-// CSR for the entries past the slot.
+// One triangle as the single-workgroup sweep reads it (device pointers): the first kSlot
+// entries of each row in its slot, rows in level order (the column, n past the row; the row in
+// bits 13 to 25, bit 30 set when it has more than kSlot entries; values, 0 past the row), and
+// the CSR for the entries past the slot.
+constexpr int kSfBits = 13;
+static_assert(kSfMaxRows < (1 << kSfBits), "column and row share a word");
 struct SfTri {
-    const int *trow, *sci, *rp, *ci;
-    const void *sv, *v;
+    const int *sci, *lci, *rp, *ci;
+    const void *sv, *lv, *v;
 };
 
-template <typename T, int S>
-__global__ void __launch_bounds__(1024)
-trsv_sf_kernel(int n, int c, SfTri L, SfTri U, const T *__restrict__ dinv,
-               const T *__restrict__ b, T *__restrict__ xg) {
-    constexpr int E = kSlot / S;    // slot entries per lane
+template <typename T>
+__global__ void __launch_bounds__(768)
+trsv_sf_kernel(int n, int c, SfTri L, SfTri U, const T *__restrict__ dinv, const T *b, T *xg) {
+    using Un = Unfinished<T>;
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    T *x = reinterpret_cast<T *>(smem_raw);
-    T *sdinv = x + (size_t)(n + 1) * c;
-    int *flag = reinterpret_cast<int *>(sdinv + n);
-    int *spL = flag + n + 1, *spU = spL + n + 1;
-    int *abort_flag = spU + n + 1;
+    T *xf = reinterpret_cast<T *>(smem_raw);
+    T *xb = xf + (size_t)(n + 1) * kSfCols;
+    int *abort_flag = reinterpret_cast<int *>(xb + (size_t)(n + 1) * kSfCols);
     const int tid = threadIdx.x, nt = blockDim.x;
-    for (int i = tid; i < n * c; i += nt) x[i] = b[i];
-    for (int i = tid; i < c; i += nt) x[(size_t)n * c + i] = T(0);
-    for (int i = tid; i < n; i += nt) {
-        sdinv[i] = dinv[i];
-        flag[i] = 0;
+    const int c0 = blockIdx.x * kSfCols, nc = min(kSfCols, c - c0);
+    for (int i = tid; i < (n + 1) * kSfCols; i += nt) {
+        xf[i] = i < n * kSfCols ? Un::pattern() : T(0);
+        xb[i] = i < n * kSfCols ? Un::pattern() : T(0);
     }
-    for (int i = tid; i <= n; i += nt) {
-        spL[i] = L.rp[i];
-        spU[i] = U.rp[i];
-    }
-    if (tid == 0) {
-        flag[n] = 3;
-        *abort_flag = 0;
-    }
+    if (tid == 0) *abort_flag = 0;
     __syncthreads();
-    const int lane = tid & 63, wave = tid >> 6, nw = nt >> 6, ntask = 2 * n;
-    const int slice = lane % S, cg = lane / S, ncg = 64 / S;
+    const int lane = tid & 63, nw = nt >> 6, ntask = 2 * n;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int q = lane & (kSlot - 1), col = lane / kSlot;
+    const int colb = col < nc ? col : 0;     // (a missing column repeats the first)
+    auto sf_row = [](int w) { return (w >> kSfBits) & ((1 << kSfBits) - 1); };
+    struct Task {
+        int pc, lc;          // row and column of this lane's entry, column of the last one
+        T pv, lv, own, di;   // their values; b of the row, inverse diagonal
+    };
     // task t < n: forward row of level-ordered position t; t >= n: backward row at t - n.
     // Branch-free loads (t clamped to the last task) with no use here, so they stay in
     // flight while the wave works on earlier tasks.
-    auto task_load = [&](int t, int &row, T *pv, int *pc) {
+    auto load_row = [&](int t, Task &k) {
         t = t < ntask ? t : ntask - 1;
         const bool up = t >= n;
-        const int k = up ? t - n : t;
-        const int *trow = up ? U.trow : L.trow, *sci = up ? U.sci : L.sci;
-        const T *sv = static_cast<const T *>(up ? U.sv : L.sv);
-        row = trow[k];
-        const size_t base = (size_t)k * kSlot + slice;
-#pragma unroll
-        for (int j = 0; j < E; ++j) {
-            pv[j] = sv[base + j * S];
-            pc[j] = sci[base + j * S];
-        }
+        const int pos = up ? t - n : t;
+        const size_t e = (size_t)pos * kSlot + q;
+        k.pc = (up ? U.sci : L.sci)[e];
+        k.pv = static_cast<const T *>(up ? U.sv : L.sv)[e];
+        const int z = pos + (lane >> 6);     // (a vector load)
+        k.lc = (up ? U.lci : L.lci)[z];
+        k.lv = static_cast<const T *>(up ? U.lv : L.lv)[z];
     };
-    auto process = [&](int t, int rowf, const T *pv, const int *pc) {
+    auto load_own = [&](Task &k) {           // once its row is known
+        const int row = sf_row(k.pc);
+        k.own = b[(size_t)row * c + c0 + colb];
+        k.di = dinv[row];
+    };
+    auto process = [&](int t, const Task &k) {
         const bool up = t >= n;
-        const int row = rowf & 0x3fffffff;
-        const bool longrow = (rowf >> 30) != 0;
-        const int need = up ? 2 : 1;
-        const int *rp = up ? spU : spL;
-        const int *ci = up ? U.ci : L.ci;
-        const T *v = static_cast<const T *>(up ? U.v : L.v);
-        // wait for the rows this one reads (all flag reads issued together)
-        for (int spins = 0;; ++spins) {
-            int f[E];
-#pragma unroll
-            for (int j = 0; j < E; ++j) f[j] = lds_flag(flag + pc[j]);
-            const int fo = up ? lds_flag(flag + row) : 1;
-            const int ab = lds_flag(abort_flag);
-            bool ok = fo >= 1;
-#pragma unroll
-            for (int j = 0; j < E; ++j) ok = ok && f[j] >= need;
-            if (longrow)
-                for (int e = rp[row] + kSlot + slice; e < rp[row + 1]; e += S)
-                    ok = ok && lds_flag(flag + ci[e]) >= need;
-            if (__all(ok) || ab) break;
-            if (spins >= kSpinMax) {
-                __hip_atomic_store(abort_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                break;
+        const int row = sf_row(k.pc);
+        T *xs = up ? xb : xf;
+        const T *pe = xs + (k.pc & ((1 << kSfBits) - 1)) * kSfCols + col;
+        // backward: the row's forward result as well (forward: the finished zero)
+        const T *po = xf + (up ? row : n) * kSfCols + col;
+        T v, own;
+        int spins = 0;
+        auto give_up = [&]() {   // after too many polls, or when another wave did
+            if ((++spins & 63) == 0) {
+                if (lds_load(abort_flag)) return true;
+                if (spins >= kSpinMax) {
+                    __hip_atomic_store(abort_flag, 1, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_WORKGROUP);
+                    return true;
+                }
+            }
+            return false;
+        };
+        for (;;) {
+            v = lds_load(pe);
+            own = lds_load(po);
+            if (__all(!Un::is(v) && !Un::is(own)) || give_up()) break;
+        }
+        T s = k.pv * v;
+        if (k.pc >> 30) {
+            const int *rp = up ? U.rp : L.rp, *ci = up ? U.ci : L.ci;
+            const T *va = static_cast<const T *>(up ? U.v : L.v);
+            for (int e = rp[row] + kSlot + 1 + q; e < rp[row + 1]; e += kSlot) {
+                const T *px = xs + ci[e] * kSfCols + col;
+                while (v = lds_load(px), Un::is(v) && !give_up()) {}
+                s += va[e] * v;
             }
         }
-        // a wave's LDS operations complete in order: a compiler fence keeps the x reads
-        // after the flag reads (a workgroup fence would also wait for the prefetches)
-        __atomic_signal_fence(__ATOMIC_SEQ_CST);
-        for (int col = cg; col < c; col += ncg) {
-            const size_t o = (size_t)row * c + col;
-            const T xo = x[o];
-            T s = 0;
-#pragma unroll
-            for (int j = 0; j < E; ++j) s += pv[j] * x[(size_t)pc[j] * c + col];
-            if (longrow)
-                for (int e = rp[row] + kSlot + slice; e < rp[row + 1]; e += S)
-                    s += v[e] * x[(size_t)ci[e] * c + col];
-            s = group_sum<S>(s);
-            if (slice == 0) x[o] = up ? sdinv[row] * (xo - s) : xo - s;
+        const T part = (up ? own : k.own) - half_sum(s);
+        const T *pl = xs + k.lc * kSfCols + col;
+        for (;;) {
+            v = lds_load(pl);
+            if (__all(!Un::is(v)) || give_up()) break;
         }
-        __atomic_signal_fence(__ATOMIC_SEQ_CST);   // x stores before the flag store
-        if (lane == 0)
-            __hip_atomic_store(flag + row, need, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        T r = part - k.lv * v;
+        if (up) r *= k.di;
+        if (Un::is(r)) r = T(__builtin_nan(""));
+        if (q == kSlot - 1)
+            __hip_atomic_store(xs + row * kSfCols + col, r, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_WORKGROUP);
     };
-    // three register sets in turn: the loads of tasks t + nw and t + 2 nw fly while task
-    // t is processed (compiler fences keep them issued before the current task's work)
-    T av[E], bv[E], cv[E];
-    int ac[E], bc[E], cc[E], ar, br, cr;
-    task_load(wave, ar, av, ac);
-    task_load(wave + nw, br, bv, bc);
+    // three register sets in turn: the entries of tasks t + nw and t + 2 nw and the own
+    // values of t + nw fly while task t is processed (compiler fences keep them issued
+    // before the current task's work)
+    Task A, B, C;
+    load_row(wave, A);
+    load_row(wave + nw, B);
+    load_own(A);
+#define XT_SF_STEP(T0, K, K1, K2)                                                              \
+    load_row((T0) + 2 * nw, K2);                                                               \
+    load_own(K1);                                                                              \
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);                                                   \
+    process(T0, K);
     for (int t = wave; t < ntask; t += 3 * nw) {
-        task_load(t + 2 * nw, cr, cv, cc);
-        __atomic_signal_fence(__ATOMIC_SEQ_CST);
-        process(t, ar, av, ac);
+        XT_SF_STEP(t, A, B, C)
         if (t + nw >= ntask) break;
-        task_load(t + 3 * nw, ar, av, ac);
-        __atomic_signal_fence(__ATOMIC_SEQ_CST);
-        process(t + nw, br, bv, bc);
+        XT_SF_STEP(t + nw, B, C, A)
         if (t + 2 * nw >= ntask) break;
-        task_load(t + 4 * nw, br, bv, bc);
-        __atomic_signal_fence(__ATOMIC_SEQ_CST);
-        process(t + 2 * nw, cr, cv, cc);
+        XT_SF_STEP(t + 2 * nw, C, A, B)
     }
+#undef XT_SF_STEP
     __syncthreads();
-    const bool bad = lds_flag(abort_flag) != 0;
-    for (int i = tid; i < n * c; i += nt) xg[i] = bad ? T(__builtin_nan("")) : x[i];
+    const bool bad = lds_load(abort_flag) != 0;
+    for (int i = tid; i < n * nc; i += nt) {
+        const int row = i / nc, j = i - row * nc;
+        xg[(size_t)row * c + c0 + j] = bad ? T(__builtin_nan("")) : xb[row * kSfCols + j];
+    }
 }
 
 // Level schedule of a triangular CSR: forward (lower) or backward (upper).
@@ -282,7 +314,7 @@ struct Tri {
     std::vector<long long> lev_nnz;  // entries per level (algorithmic bytes)
     // single-workgroup sweeps (small factors only): level-ordered rows with the long-row
     // bit, fixed-size entry slots
-    DevBuf task_row, slot_ci, slot_v64, slot_v32;
+    DevBuf last_ci, last_v64, last_v32, slot_ci, slot_v64, slot_v32;
 };
 
 }  // namespace xt
@@ -341,18 +373,27 @@ static int upload_tri(int n, const std::vector<int> &rp, const std::vector<int> 
             T.lev_nnz[l] += rp[lrows[k] + 1] - rp[lrows[k]];
     XT_TRY(T.lev_rows.upload(lrows.data(), sizeof(int) * n));
     if (n <= kSfMaxRows) {
-        std::vector<int> trow(n), sci((size_t)n * kSlot, n);
-        std::vector<double> sv((size_t)n * kSlot, 0.0);
+        std::vector<int> sci((size_t)n * kSlot), lci(n), at(n);
+        std::vector<double> sv((size_t)n * kSlot, 0.0), lv(n, 0.0);
+        for (int k = 0; k < n; ++k) at[lrows[k]] = k;
         for (int k = 0; k < n; ++k) {
-            const int r = lrows[k], len = rp[r + 1] - rp[r];
-            trow[k] = r | (len > kSlot ? (1 << 30) : 0);
-            for (int q = 0; q < std::min(len, kSlot); ++q) {
-                sci[(size_t)k * kSlot + q] = ci[rp[r] + q];
-                sv[(size_t)k * kSlot + q] = v[rp[r] + q];
+            const int r = lrows[k], len = rp[r + 1] - rp[r], flag = len > kSlot + 1 ? 1 << 30 : 0;
+            int last = rp[r];                // among the first kSlot + 1 entries
+            for (int e = rp[r]; e < rp[r] + std::min(len, kSlot + 1); ++e)
+                if (at[ci[e]] > at[ci[last]]) last = e;
+            lci[k] = len ? ci[last] : n;
+            lv[k] = len ? v[last] : 0.0;
+            for (int q = 0, e = rp[r]; q < kSlot; ++q, ++e) {
+                if (e == last && len) ++e;
+                const bool in = e < rp[r + 1];
+                sci[(size_t)k * kSlot + q] = (in ? ci[e] : n) | r << kSfBits | flag;
+                if (in) sv[(size_t)k * kSlot + q] = v[e];
             }
         }
-        std::vector<float> sv32(sv.begin(), sv.end());
-        XT_TRY(T.task_row.upload(trow.data(), sizeof(int) * n));
+        std::vector<float> sv32(sv.begin(), sv.end()), lv32(lv.begin(), lv.end());
+        XT_TRY(T.last_ci.upload(lci.data(), sizeof(int) * n));
+        XT_TRY(T.last_v64.upload(lv.data(), sizeof(double) * n));
+        XT_TRY(T.last_v32.upload(lv32.data(), sizeof(float) * n));
         XT_TRY(T.slot_ci.upload(sci.data(), sizeof(int) * sci.size()));
         XT_TRY(T.slot_v64.upload(sv.data(), sizeof(double) * sv.size()));
         XT_TRY(T.slot_v32.upload(sv32.data(), sizeof(float) * sv32.size()));
@@ -391,10 +432,6 @@ static int run_tri(const Tri &tri, const T *vals, const T *dinv, int c, const T 
 constexpr long long kOneWgWork = 4LL << 20;
 // ... and keep the solution vector in LDS when it fits this many bytes.
 constexpr size_t kOneWgLds = 128 * 1024;
-// LDS of one workgroup (gfx950: 160 KB); the staged single-workgroup sweeps are used
-// when the solution and the level schedule fit.
-constexpr size_t kWgLdsMax = 160 * 1024;
-
 // ILUT sweeps Y = (LU)^-1 X Minv_r^T.  stage: p*q*R elements of device memory for the
 // temporal mix (used only when minv is given); timed: per-launch HIP-event timing when
 // enabled (it creates events, so the allocation-free entry point passes false).
@@ -410,33 +447,34 @@ static int ilut_apply(xt_prec pr, int R, int q, const T *minv, const T *x, T *y,
     const T *lv = f32 ? (const T *)pr->L.m.val32.ptr : (const T *)pr->L.m.val64.ptr;
     const T *uv = f32 ? (const T *)pr->U.m.val32.ptr : (const T *)pr->U.m.val64.ptr;
     const T *dv = f32 ? (const T *)pr->dinv32.ptr : (const T *)pr->dinv64.ptr;
-    // Small factors: both sweeps in one workgroup (row flags in LDS when the solution
-    // fits there, else a barrier per level) instead of a launch per level; large ones:
-    // one launch per level over the whole device.
+    // Factors with slots and levels of 100 rows at most (mean of both sweeps): both sweeps of
+    // two columns in one workgroup (0.3 us a level, 0.04 a row; 512 columns at a time).
+    // Others of little work: one workgroup with a barrier per level (2.5 us); else one launch
+    // per level over the whole device (4 us).
     const long long work = (pr->L.m.nnz + pr->U.m.nnz + 2LL * pr->p) * c;
-    if (work <= kOneWgWork) {
+    const long long levels = (long long)pr->L.lev_ptr.size() + pr->U.lev_ptr.size() - 2;
+    const bool slots = pr->L.slot_ci.ptr && pr->U.slot_ci.ptr && 50 * levels >= pr->p && c <= 4096;
+    if (slots || work <= kOneWgWork) {
         const bool prof = timed && prof_on(XT_PROF_TRSV);
         if (prof) prof_begin(XT_PROF_TRSV, s);
         const size_t xl = sizeof(T) * (size_t)pr->p * c;
-        const size_t sl = sf_lds_bytes<T>(pr->p, c);
-        const int S = c <= 8 ? 8 : c <= 16 ? 4 : 0;   // entry slices per column
-        if (S && sl <= kWgLdsMax && pr->L.slot_ci.ptr && pr->U.slot_ci.ptr) {
+        if (slots) {
             auto tri = [&](const Tri &t, const T *vals) {
                 SfTri w;
-                w.trow = t.task_row.as<int>();
                 w.sci = t.slot_ci.as<int>();
                 w.sv = f32 ? t.slot_v32.ptr : t.slot_v64.ptr;
+                w.lci = t.last_ci.as<int>();
+                w.lv = f32 ? t.last_v32.ptr : t.last_v64.ptr;
                 w.rp = t.m.rowptr.as<int>();
                 w.ci = t.m.col.as<int>();
                 w.v = vals;
                 return w;
             };
-#define XT_SF(SS)                                                                           \
-    hipLaunchKernelGGL((trsv_sf_kernel<T, SS>), dim3(1), dim3(1024), sl, s, pr->p, c,       \
-                       tri(pr->L, lv), tri(pr->U, uv), dv, b, y)
-            if (S == 8) XT_SF(8);
-            else XT_SF(4);
-#undef XT_SF
+            // (12 waves: levels up to 6 rows wide keep that many busy; 16 poll more, 8 are few
+            // for the widest)
+            hipLaunchKernelGGL(trsv_sf_kernel<T>, dim3(ceil_div(c, kSfCols)), dim3(768),
+                               sf_lds_bytes<T>(pr->p), s, pr->p, c, tri(pr->L, lv),
+                               tri(pr->U, uv), dv, b, y);
         } else {
 #define XT_ONEWG(XLDS)                                                                      \
     hipLaunchKernelGGL((trsv_onewg_kernel<T, XLDS>), dim3(1), dim3(1024), XLDS ? xl : 0, s,  \
@@ -611,12 +649,12 @@ int xt_prec_create(int p, const double *alu, const int *jlu, const int *ju, xt_p
                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)kOneWgLds));
     XT_HIP(hipFuncSetAttribute((const void *)trsv_onewg_kernel<float, true>,
                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)kOneWgLds));
-#define XT_SF_ATTR(T, SS)                                                                   \
-    XT_HIP(hipFuncSetAttribute((const void *)trsv_sf_kernel<T, SS>,                          \
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)kWgLdsMax))
-    XT_SF_ATTR(double, 8); XT_SF_ATTR(double, 4);
-    XT_SF_ATTR(float, 8); XT_SF_ATTR(float, 4);
-#undef XT_SF_ATTR
+    XT_HIP(hipFuncSetAttribute((const void *)trsv_sf_kernel<double>,
+                               hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)sf_lds_bytes<double>(kSfMaxRows)));
+    XT_HIP(hipFuncSetAttribute((const void *)trsv_sf_kernel<float>,
+                               hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)sf_lds_bytes<float>(kSfMaxRows)));
     XT_ARG(jlu[0] == p + 2, "MSR factors must come from ilut (jlu(1) = n+2)");
     std::vector<int> lrp(p + 1, 0), urp(p + 1, 0), lci, uci;
     std::vector<double> lv, uv, dinv(p);
