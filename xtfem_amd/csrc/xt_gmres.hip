@@ -33,6 +33,9 @@ static constexpr int JB = 8;  // basis vectors per multidot block row
 // partial[b][j][col] = sum over the rows of chunk b of V_j[row][col] * w[row][col]; chunk b
 // covers rows chunks[b].x .. chunks[b].y - 1 (chunks never straddle two segments).
 // 256 / c row lanes of c columns; the block has at least those threads, at most 256.
+// Bound by memory with many columns (192: 4.8 TB/s); with few by the chain of its loads and
+// sums: the row lanes of all JB vectors are summed together, 6 us at 3 columns against 11 us
+// when one vector after the other went through LDS with one thread a column.
 // skip (device flag, may be NULL): nonzero makes the launch a no-op.  frozen (device,
 // per instance, may be NULL): the columns of frozen instances are taken as zero.
 __global__ void __launch_bounds__(256)
@@ -41,7 +44,7 @@ multidot_partial(int c, int k, const int2 *__restrict__ chunks, const double *__
                  const int *skip, int q, int R, const int *__restrict__ seg_of,
                  const int *__restrict__ frozen) {
     if (skip && *skip) return;   // a second Gram-Schmidt pass found unnecessary
-    __shared__ double sh[256];
+    __shared__ double sh[JB][256], sp[256];
     const int rpl = 256 / c;
     const int lr = threadIdx.x / c;
     const int col = threadIdx.x - lr * c;
@@ -82,17 +85,34 @@ multidot_partial(int c, int k, const int2 *__restrict__ chunks, const double *__
                 if (j0 + jj < k) acc[jj] += V[(size_t)(j0 + jj) * ldv + o] * wv;
         }
     }
+    // the row lanes' sums of all JB vectors together: output o = jj c + col, its row lanes
+    // split over the parts of the block, then the parts' sums
+    const int nj = min(JB, k - j0), nout = nj * c;
 #pragma unroll
-    for (int jj = 0; jj < JB; ++jj) {
-        if (j0 + jj >= k) break;
-        sh[threadIdx.x] = (lr < rpl) ? acc[jj] : 0.0;
-        __syncthreads();
-        if (threadIdx.x < c) {
+    for (int jj = 0; jj < JB; ++jj) sh[jj][threadIdx.x] = acc[jj];
+    __syncthreads();
+    const int parts = max(1, (int)blockDim.x / nout), part = threadIdx.x / nout;
+    double *out = partial + ((size_t)blockIdx.x * k + j0) * c;
+    if (parts == 1) {
+        for (int o = threadIdx.x; o < nout; o += blockDim.x) {
+            const int jj = o / c, cl = o - jj * c;
             double s = 0.0;
-            for (int l = 0; l < rpl; ++l) s += sh[l * c + threadIdx.x];
-            partial[((size_t)blockIdx.x * k + j0 + jj) * c + threadIdx.x] = s;
+            for (int l = 0; l < rpl; ++l) s += sh[jj][l * c + cl];
+            out[o] = s;
         }
-        __syncthreads();
+        return;
+    }
+    if (part < parts) {
+        const int o = threadIdx.x - part * nout, jj = o / c, cl = o - jj * c;
+        double s = 0.0;
+        for (int l = part; l < rpl; l += parts) s += sh[jj][l * c + cl];
+        sp[threadIdx.x] = s;
+    }
+    __syncthreads();
+    if (threadIdx.x < nout) {
+        double s = 0.0;
+        for (int q_ = 0; q_ < parts; ++q_) s += sp[q_ * nout + threadIdx.x];
+        out[threadIdx.x] = s;
     }
 }
 
@@ -205,21 +225,36 @@ givens_kernel(int R, int i, int K, const double *__restrict__ hcol,
     double *H = hh + (size_t)r * (K + 1) * K;
     auto h = [&](int a, int b) -> double & { return H[a + (size_t)b * (K + 1)]; };
     double *c_ = cs + (size_t)r * K, *s_ = sn + (size_t)r * K, *rs_ = rs + (size_t)r * (K + 1);
-    for (int j = 0; j <= i; ++j) h(j, i) = hcol[j * R + r] + hcol2[j * R + r];
-    h(i + 1, i) = sqrt(nrm2[r]);
-    for (int kk = 1; kk <= i; ++kk) {
-        const double t = h(kk - 1, i);
-        h(kk - 1, i) = c_[kk - 1] * t + s_[kk - 1] * h(kk, i);
-        h(kk, i) = -s_[kk - 1] * t + c_[kk - 1] * h(kk, i);
+    // (the running entry stays in a register and the loads of eight rotations are in flight
+    // together: through memory each rotation waited for the one before)
+    const double hn = sqrt(nrm2[r]);
+    double t = hcol[r] + hcol2[r];
+    for (int k0 = 1; k0 <= i; k0 += 8) {
+        double a[8], ck[8], sk[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int kk = min(k0 + u, i);
+            a[u] = hcol[kk * R + r] + hcol2[kk * R + r];
+            ck[u] = c_[kk - 1];
+            sk[u] = s_[kk - 1];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            if (k0 + u > i) break;
+            h(k0 + u - 1, i) = ck[u] * t + sk[u] * a[u];
+            t = -sk[u] * t + ck[u] * a[u];
+        }
     }
-    double gam = sqrt(h(i, i) * h(i, i) + h(i + 1, i) * h(i + 1, i));
+    h(i + 1, i) = hn;
+    double gam = sqrt(t * t + hn * hn);
     if (gam == 0.0) gam = 1.0e-16;
-    c_[i] = h(i, i) / gam;
-    s_[i] = h(i + 1, i) / gam;
-    rs_[i + 1] = -s_[i] * rs_[i];
-    rs_[i] = c_[i] * rs_[i];
-    h(i, i) = c_[i] * h(i, i) + s_[i] * h(i + 1, i);
-    const double ro = fabs(rs_[i + 1]);
+    const double ci = t / gam, si = hn / gam, rsi = rs_[i];
+    c_[i] = ci;
+    s_[i] = si;
+    rs_[i + 1] = -si * rsi;
+    rs_[i] = ci * rsi;
+    h(i, i) = ci * t + si * hn;
+    const double ro = fabs(-si * rsi);
     ro_last[r] = ro;
     if (hist && it < hist_cap) hist[it] = ro / hist_ro0;
     icyc[r] = i + 1;

@@ -72,15 +72,22 @@ struct KronArgs {
     const T *v[NT];
 };
 
-template <typename T, int NT>
+// S lanes share the entries of a row and column, and the loads of U entries of every term
+// are in flight together: with one lane walking the entries of one term after the other, a
+// row was a chain of some 50 loads.  Two terms of 27 entries a row, us, before / S = 8 / S = 1:
+// 23735 rows, 3 columns FP64 16.8 / 11.6, 12 columns 24.2 / 39 / 22.6, 96 columns 159 / - / 121,
+// FP32 127 / - / 64; 9455 rows, 12 columns 12.5 / 16.8 / 10.8.  (S = 8 gathers a column of X
+// at 8 rows at once: it pays while rows times columns are too few lanes to hide the chain.)
+template <typename T, int NT, int S>
 __global__ void __launch_bounds__(256)
 kron_csr_kernel(KronArgs<T, NT> A, int p, int c, int q, int col0, int ct, int rpb,
                 const T *__restrict__ tmat, T alpha, T beta, const T *__restrict__ x,
                 T *__restrict__ y) {
     extern __shared__ unsigned char smem_raw[];
     T *z = reinterpret_cast<T *>(smem_raw);  // [NT][rpb][ct]
-    const int lr = threadIdx.x / ct;
-    const int col = threadIdx.x - lr * ct;
+    const int unit = threadIdx.x / S, slice = threadIdx.x % S;
+    const int lr = unit / ct;
+    const int col = unit - lr * ct;
     const int row = blockIdx.x * rpb + lr;
     const bool inblk = lr < rpb;
     const bool active = inblk && row < p;
@@ -89,20 +96,53 @@ kron_csr_kernel(KronArgs<T, NT> A, int p, int c, int q, int col0, int ct, int rp
     for (int t = 0; t < NT; ++t) acc[t] = T(0);
     if (active) {
         const T *xc = x + col0 + col;
+        constexpr int U = S == 1 ? 3 : 4;   // entries in flight
+        int e0[NT], e1[NT], most = 0;
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-            const int e0 = A.rp[t][row], e1 = A.rp[t][row + 1];
-            T s = T(0);
-            for (int e = e0; e < e1; ++e) s += A.v[t][e] * xc[(size_t)A.ci[t][e] * c];
-            acc[t] = s;
+            e0[t] = A.rp[t][row] + slice;
+            e1[t] = A.rp[t][row + 1];
+            most = max(most, e1[t] - e0[t]);
+        }
+        for (int d = 0; d < most; d += U * S) {
+            T v[NT][U], w[NT][U];
+            int m[NT][U];
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+#pragma unroll
+                for (int u = 0; u < U; ++u) m[t][u] = 0;
+                if (e0[t] - slice < e1[t]) {   // (a term may have no entries at all)
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {   // (past the row's end: its last entry, unused)
+                        const int e = min(e0[t] + d + u * S, e1[t] - 1);
+                        m[t][u] = A.ci[t][e];
+                        v[t][u] = A.v[t][e];
+                    }
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int u = 0; u < U; ++u) w[t][u] = xc[(size_t)m[t][u] * c];
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    if (e0[t] + d + u * S < e1[t]) acc[t] += v[t][u] * w[t][u];
         }
     }
-    if (inblk) {
+    if (S > 1) {   // (a row and column's lanes are S neighbours of one wave)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int o = 1; o < S; o <<= 1) acc[t] += __shfl_xor(acc[t], o);
+    }
+    if (inblk && slice == 0) {
 #pragma unroll
         for (int t = 0; t < NT; ++t) z[(t * rpb + lr) * ct + col] = acc[t];
     }
     __syncthreads();
-    if (active) {
+    if (active && slice == 0) {
         const int gcol = col0 + col;
         const int r = gcol / q;
         const int i = gcol - r * q;
@@ -129,17 +169,23 @@ static int launch_kron(const DevCSR *S, int p, int q, int R, const T *tmat, doub
         A.v[t] = fp32 ? (const T *)S[t].val32.ptr : (const T *)S[t].val64.ptr;
     }
     const int c = q * R;
-    const int tile = (256 / q) * q;  // whole right-hand sides per tile
+    // (80000: 9455 rows with 9 columns equal, with 12 slower, by the figures at the kernel)
+    const int split = (long long)p * c <= 80000 && c <= 32 ? 8 : 1;
+    const int tile = (256 / split / q) * q;  // whole right-hand sides per tile
     for (int col0 = 0; col0 < c; col0 += tile) {
         const int ct = (c - col0) < tile ? (c - col0) : tile;
-        const int rpb = 256 / ct;
+        const int rpb = 256 / split / ct;
         const size_t lds = sizeof(T) * NT * rpb * ct;
         const int grid = ceil_div(p, rpb);
         if (grid == 0) break;
         const bool prof = prof_on(XT_PROF_SPMM);
         if (prof) prof_begin(XT_PROF_SPMM, s);
-        hipLaunchKernelGGL((kron_csr_kernel<T, NT>), dim3(grid), dim3(256), lds, s, A, p, c, q,
-                           col0, ct, rpb, tmat, (T)alpha, (T)beta, x, y);
+#define XT_CSR(SV)                                                                             \
+    hipLaunchKernelGGL((kron_csr_kernel<T, NT, SV>), dim3(grid), dim3(256), lds, s, A, p, c, q, \
+                       col0, ct, rpb, tmat, (T)alpha, (T)beta, x, y)
+        if (split == 8) XT_CSR(8);
+        else XT_CSR(1);
+#undef XT_CSR
         if (prof) {   // CSR values + column indices + row pointers per term, X, Y
             double nnz = 0.0;
             for (int t = 0; t < NT; ++t) nnz += (double)S[t].nnz;
