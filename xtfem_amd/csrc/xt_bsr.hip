@@ -1025,21 +1025,23 @@ static int stage_cols(const BsrPlan &P, int c) {
     return 0;
 }
 
-// The group kernel from enough work on: a wave takes 25 (64 lanes a group) to 36 us (16) for
-// its first group, a chain of loads, whatever the number of groups.  Slices against groups,
-// us (lanes of the slice kernel: nodes times cases rounded up to a power of two):
-//   FP64  4879 nodes 16 cases 32 / 37, 17 cases 57 / 39; 23735 nodes 4 cases 36 / 57,
-//         5 cases 58 / 58, 8 cases 67 / 62, 9 cases 115 / 72; 32513 nodes 5 cases 78 / 65;
-//         61004 nodes 2 cases 55 / 83, 3 cases 85 / 86, 5 cases 144 / 89
-//   FP32  4879 nodes 32 cases 32 / 34, 33 cases 55 / 45; 23735 nodes 8 cases 38 / 48, 9 cases
-//         65 / 57; 32513 nodes 8 cases 49 / 51; 61004 nodes 4 cases 49 / 56, 5 cases 86 / 57
+// The group kernel from enough work on: a wave takes 24 (64 lanes a group) to 36 us (16) for
+// its first group, a chain of loads, whatever the number of groups (a group's neighbours
+// shared by the four waves of a workgroup: 13 to 18 us, but slower at every size from 4879
+// nodes on in FP64 and 13237 in FP32, and no better than slices below).  lanes: of the slice
+// kernel, nodes times cases rounded up to a power of two (3 for 3 cases).  Slices / groups, us:
+//   FP64  lanes 78000 (9 cases) 29 / 36, 87000 (42) 33 / 28, 122000 (2) 55 / 77, 130000 (4) 50 / 61,
+//         156000 (17) 58 / 38, 183000 (3) 85 / 77, 190000 (5) 60 / 57, 212000 (9) 74 / 50
+//   FP32  lanes 156000 (32) 33 / 33, 190000 (8) 39 / 47, 212000 (9) 40 / 44, 244000 (4) 50 / 52,
+//         260000 (8) 50 / 49, 312000 (42) 58 / 45, 380000 (9) 66 / 55
 static bool group_form(const BsrPlan &P, int R, bool f32) {
     const int k = tune_knob(XT_TUNE_SPMM_GROUP);
     if (R < 2 || k == 1) return false;
     if (k == 2) return true;
     int lpn = 1;
     while (lpn < R) lpn <<= 1;
-    return (long long)P.nn * lpn >= (f32 ? 300000 : R > 16 ? 100000 : 200000);
+    const long long lanes = (long long)P.nn * (R == 3 ? 3 : lpn);
+    return lanes >= (f32 ? (R > 16 ? 200000 : 250000) : R > 8 ? 100000 : 180000);
 }
 
 template <typename T>
