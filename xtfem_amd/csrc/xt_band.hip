@@ -508,10 +508,10 @@ static int launch_prod(const Items<T> &it, int rows, int lda, int kdim, int tri,
 // the sub-diagonal block K_{i+1,i}), both column-major b x b with leading dimension b.
 // One launch per panel k (columns 64k..64k+63) of one or two eliminations (grid y), its
 // workgroups independent of each other:
-//   panel tiles t: the diagonal tile (k, k) and row tile k + t take the rank-64 update of
-//     panel k - 1, the diagonal tile is factored (identical arithmetic in each workgroup,
-//     so identical results) and the row tile solved against it, P = A_t L_kk^-T, alongside.
-//     Workgroup 0 solves the identity instead, which gives D_kk = L_kk^-1 (nothing reads
+//   panel tiles (t, half): the diagonal tile (k, k) and half of row tile k + t take the
+//     rank-64 update of panel k - 1, the diagonal tile is factored (identical arithmetic in
+//     each workgroup, so identical results) and the rows solved against it, P = A_t L_kk^-T,
+//     alongside.  t = 0 solves the identity instead, which gives D_kk = L_kk^-1 (nothing reads
 //     L_kk again).  Results go to the scratch W; the matrix is only read.
 //   trailing tiles: the rank-64 update of panel k - 1 on every tile right of column k: the
 //     lower tiles of L_i, all tiles of E_i, and the lower tiles of the next diagonal
@@ -520,10 +520,11 @@ static int launch_prod(const Items<T> &it, int rows, int lda, int kdim, int tri,
 // Panel 0 of a block applies and copies the last panel of the block before it (pL, pE); a
 // launch with k = nt only applies and copies the block's own last panel.
 // What bounds it is the chain of panels, each the path through one workgroup: the launch,
-// the tile loads, the two rank-64 updates (6,700 cycles of FP64 matrix-core time on a CU)
-// and four 16-column steps (9,500 cycles each, 5,900 of them the 16 x 16 Cholesky's chain):
-// 28 us a panel on 768-row blocks, where a panel kernel (31.4 us) and an update kernel
-// (18.9 us) followed each other before.
+// the tile loads (4,600 cycles), the rank-64 updates (6,600, 5,100 of FP64 matrix-core time on
+// a CU) and four 16-column steps (5,200 cycles each, 3,900 of them the 16 x 16 block's
+// chain): 22 us a panel on 768-row blocks.  Whole row tiles a workgroup: 9,600 for the updates;
+// rows by forward substitution, four lanes a row, instead of by the block's inverse: 2,600
+// more a step; a panel kernel (31.4 us) and an update kernel (18.9 us) after each other before.
 // ---------------------------------------------------------------------------
 constexpr int kCT = 64;   // panel width and tile size
 constexpr int kCW = 8;    // waves of a workgroup
@@ -549,7 +550,7 @@ struct CholItems {
 __host__ __device__ inline CholItems chol_items(int nt, int k, bool E, bool Wp) {
     const int ntot = E ? 2 * nt : nt, T = nt - 1 - k;
     CholItems c;
-    c.np = k < nt ? ntot - k : 0;
+    c.np = k < nt ? 2 * (ntot - k) : 0;
     c.nl = k < nt && Wp ? T * (T + 1) / 2 : 0;
     c.ne = k >= 1 && k < nt && E ? nt * T : 0;
     c.nk = k >= 1 && E ? nt * (nt + 1) / 2 : 0;
@@ -589,85 +590,109 @@ __device__ inline xt_d4c block_product(const double *P, const double *Q, int I, 
     return acc;
 }
 
-// value of v in lane G of this lane's quad
-template <int G>
-__device__ inline double quad_bcast(double v) {
-    constexpr int ctrl = G * 0x55;
-    const long long bits = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_mov_dpp((int)bits, ctrl, 0xF, 0xF, true);
-    const int hi = __builtin_amdgcn_mov_dpp((int)(bits >> 32), ctrl, 0xF, 0xF, true);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+// a_r += a_rJ t for the rows r0 + i (i < N), a_rJ lane J's value of each row of 16 lanes.  (Two
+// wait states stand between a write of a register and its read by lane-crossing operands.)
+#define XT_ELIM(i) "v_fmac_f64_dpp %" #i ", %" #i ", %[t] row_newbcast:%[j] row_mask:0xf bank_mask:0xf\n\t"
+template <int J>
+__device__ inline void eliminate1(double &a0, double t) {
+    asm("s_nop 1\n\t" XT_ELIM(0) : "+&v"(a0) : [t] "v"(t), [j] "n"(J));
 }
-__device__ inline double quad_bcast(double v, int g) {   // g: known when unrolled
-    return g == 0 ? quad_bcast<0>(v) : g == 1 ? quad_bcast<1>(v)
-         : g == 2 ? quad_bcast<2>(v) : quad_bcast<3>(v);
+template <int J>
+__device__ inline void eliminate5(double &a0, double &a1, double &a2, double &a3, double &a4,
+                                  double t) {
+    asm("s_nop 1\n\t" XT_ELIM(0) XT_ELIM(1) XT_ELIM(2) XT_ELIM(3) XT_ELIM(4)
+        : "+&v"(a0), "+&v"(a1), "+&v"(a2), "+&v"(a3), "+&v"(a4) : [t] "v"(t), [j] "n"(J));
+}
+template <int J>
+__device__ inline void eliminate4(double &a0, double &a1, double &a2, double &a3, double t) {
+    asm("s_nop 1\n\t" XT_ELIM(0) XT_ELIM(1) XT_ELIM(2) XT_ELIM(3)
+        : "+&v"(a0), "+&v"(a1), "+&v"(a2), "+&v"(a3) : [t] "v"(t), [j] "n"(J));
+}
+#undef XT_ELIM
+
+// Elimination of column J of a symmetric 16 x 16 block, unscaled: lane q of every row of 16
+// lanes holds column q, all 16 rows (the four rows of lanes do the same).  a_rc -= a_rJ a_Jc / p
+// for the rows r > J; above them stand the rows of the identity eliminated along, x_rc in place
+// of a_rc: row J becomes x_Jc = -a_Jc / p, the rows before it x_rc -= x_rJ a_Jc / p.
+// Finished columns (q <= J) keep their values.  Row J + 1, which holds the next pivot, is
+// eliminated at once, the other rows of column J - 1 (its t: tp) while 1 / p is on its way.
+template <int J>
+__device__ inline void chol_column(double (&a)[16], int q, double &tp) {
+    const double p = lane_bcast(a[J], J);
+    const double row = q > J ? -a[J] : 0.0;
+    // 1 / p: the hardware estimate (relative error e ~ 2^-24) and a third-order step
+    const double r = __builtin_amdgcn_rcp(p);
+    constexpr int P = J - 1;   // rows P + 2 .. P + 15 (mod 16): all but P and P + 1
+    auto at = [&](int k) -> double & { return a[(P + 2 + k) & 15]; };
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (J > 0) eliminate5<P>(at(0), at(1), at(2), at(3), at(4), tp);
+    __builtin_amdgcn_sched_barrier(0);
+    const double e = fma(-p, r, 1.0);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (J > 0) eliminate5<P>(at(5), at(6), at(7), at(8), at(9), tp);
+    __builtin_amdgcn_sched_barrier(0);
+    const double f = fma(e, e, e);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (J > 0) eliminate4<P>(at(10), at(11), at(12), at(13), tp);
+    __builtin_amdgcn_sched_barrier(0);
+    const double t = row * fma(r, f, r);
+    if constexpr (J < 15) eliminate1<J>(a[(J + 1) & 15], t);
+    a[J] = q > J ? t : a[J];
+    __builtin_amdgcn_sched_barrier(0);
+    tp = t;
 }
 
-// 16 x 16 Cholesky in place at columns c0 of the tile, by one wave: lane 4 r + h holds
-// columns 4 h .. 4 h + 3 of row r.  rdiag: 1 / L_jj; Ls[j][m]: L_mj below the diagonal, else
-// zero.  Returns the first non-positive pivot (1-based, 0: none).
-// Bound by the dependent chain pivot -> 1 / sqrt -> column -> next pivot: the next two
-// columns are updated by the one just scaled with lane broadcasts of their coefficients,
-// so the next pivot's root starts at once; the other columns' updates go through LDS, a
-// column behind.
-__device__ inline int chol16(double (*sA)[kCT + 1], int c0, int lane, double *rdiag,
-                             double (*Ls)[16], double (*colb)[16]) {
-    const int r = lane >> 2, h = lane & 3;
-    double a[4], prev = 0.0;
+// The upper triangle of X = L^-T of the 16 x 16 block at columns c0 of the tile (lower
+// triangle), L its Cholesky factor (X's other entries are left undefined), by one wave: the identity's rows eliminated along with the block, scaled by
+// 1 / sqrt(pivot) at the end.  Returns the first non-positive pivot (1-based, 0: none).
+// Bound by the dependent chain pivot -> 1 / pivot -> next pivot and some 26 instructions a
+// column, without a root, an LDS access or a lane exchange on the chain but the pivot's:
+// 3,900 cycles with the inverse and the block's way through LDS.  The rows of a column over
+// the four rows of lanes, exchanged by lane swaps, 4,400; a column scaled by its root, its
+// coefficients through lane reads and LDS, 5,900 without the inverse.
+__device__ inline int chol16_inverse(const double (*sA)[kCT + 1], int c0, int lane,
+                                     double (*X)[17]) {
+    const int q = lane & 15;
+    double a[16], tp = 0.0;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) a[e] = sA[c0 + r][c0 + 4 * h + e];
-    int bad = 0;
-    double pj = lane_bcast(a[0], 0);
+    for (int r = 0; r < 16; ++r) a[r] = sA[c0 + max(r, q)][c0 + min(r, q)];
+    chol_column<0>(a, q, tp);
+    chol_column<1>(a, q, tp);
+    chol_column<2>(a, q, tp);
+    chol_column<3>(a, q, tp);
+    chol_column<4>(a, q, tp);
+    chol_column<5>(a, q, tp);
+    chol_column<6>(a, q, tp);
+    chol_column<7>(a, q, tp);
+    chol_column<8>(a, q, tp);
+    chol_column<9>(a, q, tp);
+    chol_column<10>(a, q, tp);
+    chol_column<11>(a, q, tp);
+    chol_column<12>(a, q, tp);
+    chol_column<13>(a, q, tp);
+    chol_column<14>(a, q, tp);
+    chol_column<15>(a, q, tp);
+    // (column 15 has no columns behind it)
+    double piv = a[0];
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-        const int hj = j >> 2, ej = j & 3;
-        bad = (!(pj > 0.0) && !bad) ? j + 1 : bad;
-        // y = 1 / sqrt(pj): the hardware estimate (relative error e ~ 2^-24) and one step of
-        // third order, y (1 + e/2 + 3 e^2/8) with e = 1 - pj y^2: error 0.3 e^3
-        double rd = __builtin_amdgcn_rsq(pj), cl[4];
-        if (j > 0) {   // column j - 1 for its update at the end of this step
+    for (int r = 1; r < 16; ++r) piv = q >= r ? a[r] : piv;
+    // 1 / sqrt(p): y (1 + e/2 + 3 e^2/8) with e = 1 - p y^2, error 0.3 e^3
+    const double y = __builtin_amdgcn_rsq(piv), er = fma(-piv * y, y, 1.0);
+    const double rd = fma(y * er, fma(0.375, er, 0.5), y);
+    if (lane < 16) {   // (a wave's LDS accesses complete in order)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) cl[e] = colb[(j - 1) & 1][4 * h + e];
-        }
-        const double er = fma(-pj * rd, rd, 1.0);
-        rd = fma(rd * er, fma(0.375, er, 0.5), rd);
-        const double col = r > j ? a[ej] * rd : (r == j ? pj * rd : 0.0);
-        a[ej] = h == hj ? col : a[ej];
-        const double cq = quad_bcast(col, hj);
-        if (j < 15) {
-            const int h1 = (j + 1) >> 2, e1 = (j + 1) & 3;
-            const double c1 = lane_bcast(cq, 4 * (j + 1));
-            a[e1] = fma(-cq, h == h1 ? c1 : 0.0, a[e1]);
-            pj = lane_bcast(a[e1], 4 * (j + 1) + h1);
-        }
-        if (j < 14) {
-            const int h2 = (j + 2) >> 2, e2 = (j + 2) & 3;
-            const double c2 = lane_bcast(cq, 4 * (j + 2));
-            a[e2] = fma(-cq, h == h2 ? c2 : 0.0, a[e2]);
-        }
-        if (j > 0 && j < 15) {   // columns past j + 1 (rows 0..j + 1 of cl are zero)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) a[e] = fma(-prev, cl[e], a[e]);
-        }
-        if (h == 0) colb[j & 1][r] = r > j + 2 ? cq : 0.0;
-        __builtin_amdgcn_wave_barrier();
-        prev = cq;
-        if (lane == 0) rdiag[j] = rd;
+        for (int r = 0; r < 15; ++r) X[r][q] = a[r] * rd;
+        X[q][q] = rd;
     }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        sA[c0 + r][c0 + 4 * h + e] = a[e];
-        Ls[4 * h + e][r] = r > 4 * h + e ? a[e] : 0.0;
-    }
-    return bad;
+    const unsigned long long bad = __ballot(!(piv > 0.0)) & 0xFFFF;
+    return bad ? __ffsll(bad) : 0;
 }
 
 __global__ void __launch_bounds__(64 * kCW)
 chol_step_kernel(int b, int nt, int k, CholSides cs) {
     // panel: the diagonal tile and this workgroup's row tile, [row][column]; trailing: P, Q
     __shared__ double lds[2][kCT][kCT + 1];
-    __shared__ double rdiag[16], colb[2][16];
-    __shared__ __align__(16) double Ls[16][16];
+    __shared__ double sL[16][17];      // L^-T of the step's 16 x 16 diagonal block
     __shared__ int sbad;
     const CholSide &S = cs.s[blockIdx.y];
     double *L = S.L, *E = S.E;
@@ -736,63 +761,81 @@ chol_step_kernel(int b, int nt, int k, CholSides cs) {
         }
         return;
     }
-    const int t = id;
+    constexpr int HR = kCT / 2;       // rows of a half row tile
+    const int t = id >> 1, hr = (id & 1) * HR;
     double (*sA)[kCT + 1] = lds[0], (*sX)[kCT + 1] = lds[1];
     const double *D = tall_tile(L, E, b, nt, k, k);
-    const double *At = tall_tile(L, E, b, nt, k + t, k);
-    // the two tiles into registers and the panel before's tiles k and k + t into LDS (every
-    // wave needs most of them: 16 loads of one wave's column instead of 64)
-    constexpr int NE = kCT / kCW;     // columns of a tile each wave loads
-    double dv[NE], xv[NE];
+    const double *At = tall_tile(L, E, b, nt, k + t, k) + hr;
+    // the tile and the half row tile into registers and the panel before's tiles k and k + t
+    // into LDS (every wave needs most of them: 16 loads of one wave's column instead of 64)
+    constexpr int NE = kCT / kCW, NX = HR * kCT / (64 * kCW);   // loads a lane
+    const int xr = tid & (HR - 1), xc = tid / HR;               // row and column of load 0
+    double dv[NE], xv[NX];
 #pragma unroll
-    for (int e = 0; e < NE; ++e) {
-        dv[e] = D[(size_t)(wave + kCW * e) * b + lane];
-        xv[e] = t > 0 ? At[(size_t)(wave + kCW * e) * b + lane]
-                      : lane == wave + kCW * e ? 1.0 : 0.0;
+    for (int e = 0; e < NE; ++e) dv[e] = D[(size_t)(wave + kCW * e) * b + lane];
+#pragma unroll
+    for (int e = 0; e < NX; ++e) {
+        const int c = xc + e * (64 * kCW / HR);
+        xv[e] = t > 0 ? At[(size_t)c * b + xr] : hr + xr == c ? 1.0 : 0.0;
     }
-    // rank-64 update of the panel before: the diagonal tile's lower blocks and the row
-    // tile's (panel 0 leaves the rows of E alone); wave (I, H): blocks (I, 2 H), (I, 2 H + 1)
+    // rank-64 update of the panel before: the half row tile's 8 blocks by waves 0 - 3 (panel 0
+    // leaves the rows of E alone), the diagonal tile's lower 10 by waves 4 - 7, two or three
+    // blocks a wave, of one block row (its operand is read from LDS once) but wave 7's third
     const bool upx = t > 0 && (k > 0 || t < nt);
-    const int I = wave & 3, J0 = 2 * (wave >> 2);
-    xt_d4c ax[2], ad[2];
+    const bool xw = wave < 4, w3 = wave >= 6;   // of the row tile; three blocks
+    auto block_row = [&](int h) { return xw ? wave >> 1 : wave < 6 ? 3 : wave == 6 ? 2 : h < 2; };
+    auto block_col = [&](int h) { return wave < 6 ? 2 * (wave & 1) + h : wave == 6 ? h : h & 1; };
+    constexpr int UW = 3;
+    xt_d4c au[UW];
     if (Wp) {
         double *sk = &lds[0][0][0], *st = &lds[1][0][0];
-        const double *Pk = wp(k), *Pt = wp(k + t);
-        double pk[NE], pt[NE];
+        const double *Pk = wp(k), *Pt = wp(k + t) + hr;
+        double pk[NE], pt[NX];
 #pragma unroll
-        for (int e = 0; e < NE; ++e) {
-            pk[e] = Pk[tid + 64 * kCW * e];
-            pt[e] = upx ? Pt[tid + 64 * kCW * e] : 0.0;
-        }
+        for (int e = 0; e < NE; ++e) pk[e] = Pk[tid + 64 * kCW * e];
 #pragma unroll
-        for (int e = 0; e < NE; ++e) {
-            sk[tid + 64 * kCW * e] = pk[e];
-            st[tid + 64 * kCW * e] = pt[e];
-        }
+        for (int e = 0; e < NX; ++e)
+            pt[e] = upx ? Pt[(xc + e * (64 * kCW / HR)) * kCT + xr] : 0.0;
+#pragma unroll
+        for (int e = 0; e < NE; ++e) sk[tid + 64 * kCW * e] = pk[e];
+#pragma unroll
+        for (int e = 0; e < NX; ++e) st[tid + 64 * kCW * e] = pt[e];
         __syncthreads();
+        double pv[kCT / 4];
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            if (J0 + h <= I) ad[h] = block_product(sk, sk, I, J0 + h, g, q);
-            if (upx) ax[h] = block_product(st, sk, I, J0 + h, g, q);
+        for (int h = 0; h < UW; ++h) {
+            if ((xw && !upx) || (h == 2 && !w3)) break;
+            double qv[kCT / 4];
+#pragma unroll
+            for (int k4 = 0; k4 < kCT / 4; ++k4) qv[k4] = sk[(4 * k4 + g) * kCT + 16 * block_col(h) + q];
+            if (h == 0 || (h == 2 && wave == 7)) {
+                const double *P = (xw ? st + g * HR : sk + g * kCT) + 16 * block_row(h) + q;
+                const int ps = 4 * (xw ? HR : kCT);
+#pragma unroll
+                for (int k4 = 0; k4 < kCT / 4; ++k4) pv[k4] = P[k4 * ps];
+            }
+            au[h] = xt_d4c{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int k4 = 0; k4 < kCT / 4; ++k4)
+                au[h] = __builtin_amdgcn_mfma_f64_16x16x4f64(qv[k4], pv[k4], au[h], 0, 0, 0);
         }
         __syncthreads();
     }
 #pragma unroll
-    for (int e = 0; e < NE; ++e) {
-        sA[lane][wave + kCW * e] = dv[e];
-        sX[lane][wave + kCW * e] = xv[e];
-    }
+    for (int e = 0; e < NE; ++e) sA[lane][wave + kCW * e] = dv[e];
+#pragma unroll
+    for (int e = 0; e < NX; ++e) sX[xr][xc + e * (64 * kCW / HR)] = xv[e];
     if (tid == 0) sbad = 0;
     __syncthreads();
     if (Wp) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
+        for (int h = 0; h < UW; ++h) {
+            if ((xw && !upx) || (h == 2 && !w3)) break;
+            double (*Cm)[kCT + 1] = xw ? sX : sA;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int c = 16 * (J0 + h) + g + 4 * i;
-                if (J0 + h <= I) sA[16 * I + q][c] -= ad[h][i];
-                if (upx) sX[16 * I + q][c] -= ax[h][i];
-            }
+            for (int i = 0; i < 4; ++i)
+                Cm[16 * block_row(h) + q][16 * block_col(h) + g + 4 * i] -= au[h][i];
+        }
         __syncthreads();
     }
     // rank-16 update of block (Ib, J) of the tile (or of the row tile) by step s's columns
@@ -807,67 +850,66 @@ chol_step_kernel(int b, int nt, int k, CholSides cs) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) Cm[16 * Ib + g + 4 * i][16 * J + q] -= a4[i];
     };
-    // four 16-column steps: the 16 x 16 diagonal block by wave 0 in registers while the other
-    // waves finish the step before (the rank-16 updates past the next 16 columns); the rows
-    // below it (and the row tile's) by forward substitution, four lanes a row; the rank-16
-    // update of the next 16 columns on the matrix cores
+    // four 16-column steps: the inverse factor of the 16 x 16 diagonal block by wave 0 in
+    // registers while the other waves finish the step before (the rank-16 updates past the
+    // next 16 columns); then on the matrix cores the rows below it (and the row tile's) by
+    // that inverse and the rank-16 update of the next 16 columns
     for (int s = 0; s < 4; ++s) {
         const int c0 = 16 * s;
         if (wave == 0) {
-            const int bad = chol16(sA, c0, lane, rdiag, Ls, colb);
+            const int bad = chol16_inverse(sA, c0, lane, sL);
             if (tid == 0 && bad && !sbad) sbad = c0 + bad;
         } else if (s > 0) {
-            // blocks (Ib, J) of the tile with s < J <= Ib, then (0..3, J) of the row tile
-            const int nj = 3 - s, n1 = nj * (nj + 1) / 2, n2 = 4 * nj;
+            // blocks (Ib, J) of the tile with s < J <= Ib, then (0..1, J) of the row tile
+            const int nj = 3 - s, n1 = nj * (nj + 1) / 2, n2 = 2 * nj;
             for (int u = wave - 1; u < n1 + n2; u += kCW - 1) {
                 if (u < n1) {
                     const int J = u < nj ? s + 1 : s + 2, Ib = u < nj ? s + 1 + u : 3;
                     rank16(sA, Ib, J, c0 - 16);
                 } else {
-                    rank16(sX, (u - n1) & 3, s + 1 + ((u - n1) >> 2), c0 - 16);
+                    rank16(sX, (u - n1) & 1, s + 1 + ((u - n1) >> 1), c0 - 16);
                 }
             }
         }
         __syncthreads();
-        // x L_s^T = a for the rows below the block in the tile, then the row tile's rows
-        const int nd = kCT - c0 - 16, rw = tid >> 2, h = tid & 3;
-        double *row = nullptr;
-        if (rw < nd) row = &sA[c0 + 16 + rw][c0 + 4 * h];
-        else if (rw < nd + kCT) row = &sX[rw - nd][c0 + 4 * h];
-        if (row) {
-            double x[4], l[16][4];
+        // the rows below the block in the tile and the row tile's: x = a L_s^-T
+        {
+            const int n1 = 3 - s;
+            if (wave < n1 + 2) {
+                double (*Cm)[kCT + 1] = wave < n1 ? sA : sX;
+                const int r0 = wave < n1 ? c0 + 16 + 16 * wave : 16 * (wave - n1);
+                double pa[4], qb[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) x[e] = row[e];
-#pragma unroll
-            for (int j = 0; j < 15; ++j)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) l[j][e] = Ls[j][4 * h + e];
-#pragma unroll
-            for (int j = 0; j < 16; ++j) {
-                const double c = x[j & 3] * rdiag[j];
-                x[j & 3] = h == (j >> 2) ? c : x[j & 3];
-                const double cq = quad_bcast(c, j >> 2);
-                if (j < 15) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) x[e] = fma(-cq, l[j][e], x[e]);
+                for (int k4 = 0; k4 < 4; ++k4) {
+                    pa[k4] = Cm[r0 + q][c0 + 4 * k4 + g];
+                    qb[k4] = 4 * k4 + g <= q ? sL[4 * k4 + g][q] : 0.0;
                 }
-            }
+                xt_d4c a4 = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-            for (int e = 0; e < 4; ++e) row[e] = x[e];
+                for (int k4 = 0; k4 < 4; ++k4)
+                    a4 = __builtin_amdgcn_mfma_f64_16x16x4f64(pa[k4], qb[k4], a4, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) Cm[r0 + g + 4 * i][c0 + q] = a4[i];
+            }
         }
         __syncthreads();
-        if (s < 3) {   // the next 16 columns: blocks (s + 1..3, s + 1), the row tile's (0..3, s + 1)
+        if (s < 3) {   // the next 16 columns: blocks (s + 1..3, s + 1), the row tile's (0..1, s + 1)
             const int n1 = 3 - s;
             if (wave < n1) rank16(sA, s + 1 + wave, s + 1, c0);
-            else if (wave < n1 + 4) rank16(sX, wave - n1, s + 1, c0);
+            else if (wave < n1 + 2) rank16(sX, wave - n1, s + 1, c0);
             __syncthreads();
         }
     }
-    if (t == 0 && tid == 0 && sbad) S.info[0] = k * kCT + sbad;
+    if (id == 0 && tid == 0 && sbad) S.info[0] = k * kCT + sbad;
     double *wt = S.W + TS * t;
-    for (int e = tid; e < kCT * kCT; e += 64 * kCW) {
-        const int c = e >> 6, r = e & 63;
-        wt[e] = t > 0 ? sX[r][c] : sX[c][r];
+    if (t > 0) {
+        for (int e = tid; e < HR * kCT; e += 64 * kCW) {
+            const int c = e / HR, r = e & (HR - 1);
+            wt[c * kCT + hr + r] = sX[r][c];
+        }
+    } else {                           // row r of the solved identity: column r of D_kk
+        for (int e = tid; e < HR * kCT; e += 64 * kCW)
+            wt[hr * kCT + e] = sX[e >> 6][e & 63];
     }
 }
 
