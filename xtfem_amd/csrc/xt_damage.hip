@@ -21,8 +21,9 @@
 // step are taken, without a change of any result: what depends on the damage alone (3
 // divisions, kept until it changes), the divisions by 3 (div3) and the root of the yield
 // test (its square against the largest double whose root is at most sig_f; the root itself
-// only where the corrector or the end asks for it); in the corrector 18 of 30 divisions share a
-// reciprocal (quotients) and 8 are by 3.  345600 points, 2560 time points: 11.9 -> 9.7 ms,
+// only where the corrector or the end asks for it); in the corrector 20 of 34 divisions have a
+// reciprocal at hand (quotients), 8 are by 3 and 2 are of constants (a block of 630 elements
+// that damages, 688 points: 0.69 -> 0.48 ms).  345600 points, 2560 time points: 11.9 -> 9.7 ms,
 // with the displacements written a time point ahead 8.8; 5400 waves on 1024 SIMDs leave
 // 12 % of it to the last round.
 //
@@ -75,11 +76,12 @@ static __device__ inline bool ordinary(double v) {   // 2^-100 .. 2^100
     return e > -100 && e < 100 && !__builtin_amdgcn_class(v, 0x267);
 }
 // x[i] / den, r = 1 / den correctly rounded
-static __device__ inline void quotients(double (&x)[6], double den, double r, bool ord_den) {
-    double y[6];
+template <int N>
+static __device__ inline void quotients(double (&x)[N], double den, double r, bool ord_den) {
+    double y[N];
     int lo = 0, hi = 0;
     bool inf = false;
-    for (int i = 0; i < 6; ++i) {
+    for (int i = 0; i < N; ++i) {
         const int e = __builtin_amdgcn_frexp_exp(x[i]);   // (0 for 0, infinities and NaNs)
         lo = min(lo, e);
         hi = max(hi, e);
@@ -90,8 +92,8 @@ static __device__ inline void quotients(double (&x)[6], double den, double r, bo
     }
     const bool odd = !ord_den || inf || lo < -900 || hi > 900;
     if (__builtin_amdgcn_ballot_w64(odd))
-        for (int i = 0; i < 6; ++i) y[i] = odd ? x[i] / den : y[i];
-    for (int i = 0; i < 6; ++i) x[i] = y[i];
+        for (int i = 0; i < N; ++i) y[i] = odd ? x[i] / den : y[i];
+    for (int i = 0; i < N; ++i) x[i] = y[i];
 }
 // 1.5 and 3 times the squares of a deviator, summed in the reference's order
 static __device__ inline double equivalent2(const double (&t)[6]) {
@@ -112,9 +114,10 @@ damage_kernel(int ngp, int nn, int nip, const int *__restrict__ nodes,
               double *__restrict__ sig_back, double *__restrict__ pp, double *__restrict__ dd,
               double *__restrict__ wsv, double *__restrict__ del_po_v,
               double *__restrict__ sig_d_v, const DamageParams dp, const double sigf2,
-              const double r2s) {
+              const double r2s, const double rs) {
     __shared__ double xch[2][64][4];  // [parity][lane][disp of the lane's node, padded]
-    // what only the corrector reads, out of the registers: c4, gamma, p, ws, del_po, G, Kb, nu, E
+    // what only the corrector reads, out of the registers: c4, gamma, p, ws, del_po, G, Kb,
+    // (1 + nu) / 2 E and nu / 2 E
     __shared__ double rare[9][64];
     const int lane = threadIdx.x;
     const int ii = blockIdx.x * 64 + lane;
@@ -157,8 +160,8 @@ damage_kernel(int ngp, int nn, int nip, const int *__restrict__ nodes,
     const double b = 2.0 * (4.0 - 5.0 * nui) / (15.0 * (1.0 - nui));
     rare[5][lane] = ymi / (2.0 * (1.0 + nui));
     rare[6][lane] = ymi / (3.0 * (1.0 - 2.0 * nui));
-    rare[7][lane] = nui;
-    rare[8][lane] = ymi;
+    rare[7][lane] = (1.0 + nui) / (2.0 * ymi);
+    rare[8][lane] = nui / (2.0 * ymi);
     const double coef = ymi / ((1. + nui) * (1. - 2. * nui));
     const double dl = coef * nui;
     const double dg = coef * (1.0 - nui);
@@ -263,7 +266,9 @@ damage_kernel(int ngp, int nn, int nip, const int *__restrict__ nodes,
         const double tr_sigs = -trq;
         const double del_p = (qeq - XT_SIGF) / gamma;
         rare[2][lane] += del_p;
-        const double c5 = 1.0 + gamma * del_p / XT_SIGF;
+        double c5q[1] = {gamma * del_p};
+        quotients(c5q, XT_SIGF, 2.0 * r2s, ordinary(XT_SIGF));
+        const double c5 = 1.0 + c5q[0];
         double dvs[6];
         for (int i = 0; i < 6; ++i) dvs[i] = -dq[i];
         quotients(dvs, c5, 1.0 / c5, ordinary(c5));
@@ -289,18 +294,20 @@ damage_kernel(int ngp, int nn, int nip, const int *__restrict__ nodes,
                 if (se[i] < 0.0) sn[i] = se[i];
                 else sp[i] = se[i];
             }
-            const double nui = rare[7][lane], ymi = rare[8][lane];
+            const double y1 = rare[7][lane], y2 = rare[8][lane];
             const double hr = (1.0 - d) / (1.0 - XT_H * d);
-            const double Yp = (1.0 + nui) / (2.0 * ymi) *
+            const double Yp = y1 *
                               (sp[0] * sp[0] + sp[1] * sp[1] + sp[2] * sp[2] +
                                XT_H * hr * hr * (sn[0] * sn[0] + sn[1] * sn[1] + sn[2] * sn[2]));
             double trt = 0.0;
             for (int i = 0; i < 3; ++i) trt += se[i];
             double Yn;
-            if (trt >= 0.0) Yn = nui / (2.0 * ymi) * trt * trt;
-            else Yn = nui / (2.0 * ymi) * XT_H * hr * hr * trt * trt;
+            if (trt >= 0.0) Yn = y2 * trt * trt;
+            else Yn = y2 * XT_H * hr * hr * trt * trt;
             // (Y/S)^s: s = 0.5 as the correctly rounded sqrt (the reference's value)
-            d += (dp.sexp == 0.5 ? sqrt((Yp - Yn) / XT_S) : pow((Yp - Yn) / XT_S, dp.sexp)) * del_p;
+            double ys[1] = {Yp - Yn};
+            quotients(ys, XT_S, rs, ordinary(XT_S));
+            d += (dp.sexp == 0.5 ? sqrt(ys[0]) : pow(ys[0], dp.sexp)) * del_p;
         } else {
             d = 0.0;
         }
@@ -387,7 +394,7 @@ extern "C" int xt_damage_device_params(int ne, int nn, int nip, const int *nodes
     hipLaunchKernelGGL(damage_kernel, dim3(ceil_div(ngp, 64)), dim3(64), 0,
                        (hipStream_t)stream, ngp, nn, nip, nodes, Nx, Ny, Nz, Nt, sol, ym, nu,
                        eps_old, eps_pl, sig_eff, sig_back, p, D, ws, del_po, sig_d, dp,
-                       largest_square(dp.sigf), 1.0 / (2.0 * dp.sigf));
+                       largest_square(dp.sigf), 1.0 / (2.0 * dp.sigf), 1.0 / dp.S);
     if (prof)   // state 31 FP64 read + written, 24 derivatives + 8 node ids, Nt, 24 disp gathers per step
         prof_end(XT_PROF_DAMAGE, (hipStream_t)stream,
                  (double)ngp * (31 * 16 + 24 * 8 + 8 * 4) + 8.0 * 6 * nip + 8.0 * 18 * nn, 0.0);
