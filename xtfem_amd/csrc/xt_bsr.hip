@@ -21,9 +21,9 @@
 // Work mapping of the slices: one lane per (node row, load case r), or SPL lanes with the
 // entries split between them.  The lane accumulates the 3 rows x 6 temporal columns of
 // K X and M X for its node in registers (72 FMA per block), then applies the 6x6
-// temporal matrices of its load case in registers and stores its outputs once.  A wave
-// covers 64 / (LPN SPL) nodes of one slice (LPN = load cases rounded up to a power of
-// two), so loop bounds are wave-uniform.
+// temporal matrices of its load case in registers and stores its outputs once.  With W
+// lanes a node a slice's 64 slots fill W whole waves for any W, so loop bounds are
+// wave-uniform without lanes left over.
 //
 // Storage ("node groups", kron_group_kernel, several load cases on enough nodes): kG
 // consecutive nodes share the sorted union of their neighbours; the blocks stand
@@ -55,6 +55,7 @@ struct BsrPlan {
     // group's nodes it couples to), its blocks from gblk[s] + b on (nodes ascending); gkmap,
     // gmmap as kmap, mmap.
     int ngroups = 0;
+    long long ngnbr = 0;    // neighbours of all groups
     DevBuf gptr, gblk, gnbr, gval32, gval64, gkmap, gmmap;
     // Staged form: the distinct column nodes of each slice (its neighbour set, sorted),
     // unode[ubase[s] .. ubase[s] + ulen[s]), and for every stored block the position of
@@ -264,6 +265,7 @@ int bsr_build(int p, const int *krp, const int *kci, const double *kv, const int
     if (P.nk) XT_TRY(P.gkmap.upload(gkmap.data(), sizeof(int) * P.nk));
     if (P.nm) XT_TRY(P.gmmap.upload(gmmap.data(), sizeof(int) * P.nm));
     P.ngroups = ngroups;
+    P.ngnbr = gptr[ngroups];
     XT_TRY(P.gptr.upload(gptr.data(), sizeof(int) * gptr.size()));
     XT_TRY(P.gblk.upload(gblk.data(), sizeof(int) * gblk.size()));
     XT_TRY(P.gnbr.upload(gnbr.data(), sizeof(int) * gnbr.size()));
@@ -322,26 +324,33 @@ __device__ __forceinline__ long long xcd_block(long long b, long long grid) {
     return (b % 8) * per + b / 8;
 }
 
-// LPN: lanes per node (power of two >= load cases in this launch, <= 64); UNR: entries
-// per pass (loads in flight)
-template <typename T, int LPN, int UNR>
+// W: lanes per node, from the load cases of this launch on (R: past its last one, <= 64 of
+// them), inv = ceil(2^31 / W); UNR: entries per pass (loads in flight).  Bound by the vector
+// cache, whose load instructions cost the same for idle lanes, so W is the cases themselves
+// and not the power of two above them.  W = power of two / cases, us:
+//   4879 nodes, FP64  9 cases 29 / 20, 12: 30 / 24, 17: 57 / 37, 28: 59 / 57
+//  13237 nodes, FP32  5 cases 21 / 19, 9: 40 / 28, 12: 41 / 33, 17: 77 / 47, 28: 79 / 71
+// One lane below a power of two is the exception (slice_lanes).
+template <typename T, int UNR>
 __global__ void __launch_bounds__(256)
 kron_bsr3_kernel(int nslices, const int *__restrict__ slot_node,
                  const int *__restrict__ slice_base, const int *__restrict__ slice_len,
-                 const int *__restrict__ bcol, const T *__restrict__ bval, int R, int r0,
-                 int c, const T *__restrict__ tmat, T alpha, T beta, const T *__restrict__ x,
-                 T *__restrict__ y) {
+                 const int *__restrict__ bcol, const T *__restrict__ bval, int W,
+                 unsigned inv, int R, int r0, int c, const T *__restrict__ tmat, T alpha,
+                 T beta, const T *__restrict__ x, T *__restrict__ y) {
     using V2 = typename Vec2<T>::type;
-    constexpr int NPW = 64 / LPN;
+    // Lane f of the slice's 64 W: slot f / W, case f % W.  The quotients by inv are exact
+    // below 2^31 / W for any W, below 2^31 for a power of two; with W not one, 2^25 waves
+    // would need vectors of more than the card's memory.  The wave stays a vector value: with
+    // s and its loop in scalar registers FP64 took 2 to 4% more.
     const int lane = threadIdx.x & 63;
-    const long long blk = xcd_block(blockIdx.x, gridDim.x);
-    const long long wave = blk * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    const long long slot = wave * NPW + lane / LPN;
-    const int s = (int)(slot / kSlice);
+    const int wave = (int)xcd_block(blockIdx.x, gridDim.x) * (int)(blockDim.x >> 6) +
+                     (int)(threadIdx.x >> 6);
+    const int s = (int)__umulhi(2u * (unsigned)wave, inv);
     if (s >= nslices) return;
-    const int k = (int)(slot - (long long)s * kSlice);
-    const int r = r0 + (lane % LPN);
-    const int node = slot_node[slot];
+    const int f = (wave - s * W) * 64 + lane, k = (int)__umulhi(2u * (unsigned)f, inv);
+    const int r = r0 + (f - k * W);
+    const int node = slot_node[s * kSlice + k];
     const bool act = node >= 0 && r < R;
     const int L = slice_len[s];
     const long long b0 = slice_base[s];
@@ -1025,23 +1034,59 @@ static int stage_cols(const BsrPlan &P, int c) {
     return 0;
 }
 
+// Lanes per node of the slice kernel: the cases, except that
+// - up to one wave a CU nothing shares its vector cache, and a power of two's loads touch
+//   fewer lines each (power of two / cases, us, FP64: 5 cases on 455 nodes 12.1 / 12.8, 17 there
+//   12.2 / 12.5; past 256 waves 9 on 1155 nodes 13.8 / 12.8, 17 there 16.7 / 14.8);
+// - a count one below a power of two gets an idle lane: a node's lanes then neither straddle
+//   waves nor shift against the cache lines from node to node (cases / cases + 1, us, FP64:
+//   3 on 23735 nodes 38 / 35, 7 there 74 / 65, 15 on 4879 nodes 32.7 / 32.0; FP32: 15 there
+//   19.0 / 17.8, 31 33.1 / 30.9, but 3 on 32513 nodes 23 / 25).  Other odd counts lose by it
+//   as often as they win (5 on 23735 nodes 53 / 61, 13 on 13237 69 / 67).
+template <typename T>
+static int slice_lanes(int R, int nslices) {
+    int up = 1;
+    while (up < R) up <<= 1;
+    if ((long long)nslices * up <= 256) return up;
+    return R + 1 == up && R > (sizeof(T) == 4 ? 3 : 1) ? up : R;
+}
+
 // The group kernel from enough work on: a wave takes 24 (64 lanes a group) to 36 us (16) for
 // its first group, a chain of loads, whatever the number of groups (a group's neighbours
 // shared by the four waves of a workgroup: 13 to 18 us, but slower at every size from 4879
-// nodes on in FP64 and 13237 in FP32, and no better than slices below).  lanes: of the slice
-// kernel, nodes times cases rounded up to a power of two (3 for 3 cases).  Slices / groups, us:
-//   FP64  lanes 78000 (9 cases) 29 / 36, 87000 (42) 33 / 28, 122000 (2) 55 / 77, 130000 (4) 50 / 61,
-//         156000 (17) 58 / 38, 183000 (3) 85 / 77, 190000 (5) 60 / 57, 212000 (9) 74 / 50
-//   FP32  lanes 156000 (32) 33 / 33, 190000 (8) 39 / 47, 212000 (9) 40 / 44, 244000 (4) 50 / 52,
-//         260000 (8) 50 / 49, 312000 (42) 58 / 45, 380000 (9) 66 / 55
+// nodes on in FP64 and 13237 in FP32, and no better than slices below).  The slices' time
+// grows with nodes times cases (work, in thousands below); above 8 cases the groups' with
+// their lanes, close to a power of two, hence the share of it that the cases fill.
+// Slices / groups, us, at work (cases):
+//   FP64  137 (3) 66 / 66, 207 (3) 106 / 90, 163 (4) 71 / 83, 183 (4) 73 / 69, 165 (6) 70 / 62,
+//         139 (8) 59 / 60, 136 (9) 62 / 45, 157 (9) 67 / 67, 106 (12) 42 / 48, 142 (16) 60 / 50,
+//         83 (20) 36 / 36, 128 (20) 48 / 38, 91 (28) 37 / 27, 79 (36) 33 / 36, 117 (36) 47 / 37,
+//         150 (36) 60 / 65, 104 (40) 40 / 34
+//   FP32  276 (4) 63 / 61, 345 (5) 80 / 62, 245 (6) 50 / 61, 274 (6) 64 / 51, 327 (8) 61 / 62,
+//         247 (9) 53 / 68, 368 (9) 75 / 77, 181 (12) 38 / 39, 249 (14) 49 / 42, 242 (16) 48 / 40,
+//         257 (17) 51 / 51, 153 (24) 33 / 33, 179 (28) 38 / 31, 133 (32) 30 / 31,
+//         290 (36) 59 / 50, 320 (36) 61 / 72, 373 (42) 72 / 72
+// Far above these the slices' time goes with stored blocks times cases, the groups' with their
+// neighbours, 9 (four nodes across a mesh) to 13.5 a node, times the lanes for the cases: share
+// is where they meet.  On thick meshes few cases stay with the slices at any size (FP64: 2
+// cases on 115351 nodes 146 / 208, 3 there 210 / 214, but 161 / 127 on 95793 nodes 3 across;
+// FP32: 4 there 95 / 118, 6 on 52521 nodes 65 / 76, 9 there 95 / 112, 9 on 61004 nodes 4
+// across 110 / 91, 17 on 29791 nodes 95 / 98).
 static bool group_form(const BsrPlan &P, int R, bool f32) {
     const int k = tune_knob(XT_TUNE_SPMM_GROUP);
     if (R < 2 || k == 1) return false;
     if (k == 2) return true;
-    int lpn = 1;
-    while (lpn < R) lpn <<= 1;
-    const long long lanes = (long long)P.nn * (R == 3 ? 3 : lpn);
-    return lanes >= (f32 ? (R > 16 ? 200000 : 250000) : R > 8 ? 100000 : 180000);
+    const int chunks = ceil_div(R, 32), per = ceil_div(R, chunks);
+    const double share = f32 ? (per <= 8 ? 13 : per <= 16 ? 25 : 36) * chunks : R <= 4 ? 8 : 0;
+    if ((double)R * P.nblocks <= share * P.ngnbr) return false;
+    int up = 1;
+    while (up < R) up <<= 1;
+    const long long work = (long long)P.nn * R;
+    if (R <= 8) return work >= (f32 ? 270000 : R > 4 ? 140000 : 180000);
+    const long long filled = work * R / up;
+    if (R <= 16) return filled >= (f32 ? 200000 : 85000);
+    if (R <= 32) return filled >= (f32 ? 155000 : 55000);
+    return filled >= (f32 ? 160000 : 62000);
 }
 
 template <typename T>
@@ -1117,23 +1162,18 @@ int bsr_apply(const BsrPlan &P, int R, const T *tmat, double alpha, double beta,
     }
     for (int r0 = 0; r0 < R; r0 += 64) {
         const int Rc = std::min(64, R - r0);
-        int lpn = 1;
-        while (lpn < Rc) lpn <<= 1;
         const long long slots = (long long)P.nslices * kSlice;
-        const long long waves = slots * lpn / 64;
+        const int W = slice_lanes<T>(Rc, P.nslices);
+        const long long waves = (long long)P.nslices * W;
+        const unsigned inv = (0x80000000u + W - 1) / W;
         const int wk = tune_knob(XT_TUNE_SPMM_WPB);
         const int wpb = wk ? wk : (waves >= 4 * 1024 ? 4 : 1);
         const int grid = (int)(((waves + wpb - 1) / wpb + 7) / 8 * 8);
         const int unr = spmm_unr<T>(R);
-#define XT_BSR_LAUNCH(N, U)                                                                   \
-    hipLaunchKernelGGL((kron_bsr3_kernel<T, N, U>), dim3(grid), dim3(64 * wpb), 0, s,         \
-                       P.nslices, P.slot_node.as<int>(), P.slice_base.as<int>(),              \
-                       P.slice_len.as<int>(), P.bcol.as<int>(), bv, R, r0, c, tmat, (T)alpha, \
-                       (T)beta, x, y)
-#define XT_BSR_UNR(N)                                                                         \
-    if (unr == 2) XT_BSR_LAUNCH(N, 2);                                                        \
-    else if (unr == 8) XT_BSR_LAUNCH(N, 8);                                                   \
-    else XT_BSR_LAUNCH(N, 4)
+#define XT_BSR_LAUNCH(U)                                                                      \
+    hipLaunchKernelGGL((kron_bsr3_kernel<T, U>), dim3(grid), dim3(64 * wpb), 0, s, P.nslices,  \
+                       P.slot_node.as<int>(), P.slice_base.as<int>(), P.slice_len.as<int>(),  \
+                       P.bcol.as<int>(), bv, W, inv, r0 + Rc, r0, c, tmat, (T)alpha, (T)beta, x, y)
 #define XT_BSR_R1(S, U)                                                                       \
     hipLaunchKernelGGL((kron_bsr3_r1_kernel<T, S, U>), dim3(grid1), dim3(64), 0, s, P.nslices, \
                        P.slot_node.as<int>(), P.slice_base.as<int>(), P.slice_len.as<int>(),  \
@@ -1152,17 +1192,14 @@ int bsr_apply(const BsrPlan &P, int R, const T *tmat, double alpha, double beta,
                 else if (unr == 8) XT_BSR_R1(4, 8);
                 else XT_BSR_R1(4, 4);
             }
-        } else switch (lpn) {
-            case 1: XT_BSR_UNR(1); break;
-            case 2: XT_BSR_UNR(2); break;
-            case 4: XT_BSR_UNR(4); break;
-            case 8: XT_BSR_UNR(8); break;
-            case 16: XT_BSR_UNR(16); break;
-            case 32: XT_BSR_UNR(32); break;
-            default: XT_BSR_UNR(64); break;
+        } else if (unr == 2) {
+            XT_BSR_LAUNCH(2);
+        } else if (unr == 8) {
+            XT_BSR_LAUNCH(8);
+        } else {
+            XT_BSR_LAUNCH(4);
         }
 #undef XT_BSR_R1
-#undef XT_BSR_UNR
 #undef XT_BSR_LAUNCH
         if (prof_on(XT_PROF_SPMM)) {
             // 12 values (3x3 K block + diagonal of the M block) + 1 column index per
