@@ -52,13 +52,16 @@ namespace xt {
 
 // The sweeps of one apply are a fixed sequence of launches on fixed buffers for a given
 // column count and precision: captured once into a HIP graph and replayed, they skip the
-// per-launch host overhead.  Keyed on every pointer the launches use, so a
-// refactorization or a grown workspace captures anew.
+// per-launch host overhead.  Keyed on every pointer the launches use and on the factor's
+// layout (a refactorization of a wider band changes kw and rc, and an array that was freed
+// for it can come back at its old address), so a refactorization or a grown workspace
+// captures anew.
 constexpr int kLevels = 4;     // pairing levels of the block recurrences, at most
 constexpr int kMinChain = 3;   // a level is added while its chain keeps this many steps
 constexpr int kKey = 6 + 2 * kLevels;
 struct SweepGraph {
     int c = 0, pi = -1, nl = 0;                          // columns, precision, levels used,
+    int kw = 0, rc = 0;                                  // the factor's layout,
     long long epoch = -1;                                // knob epoch
     const void *key[kKey] = {};
     hipGraphExec_t exec = nullptr;
@@ -1794,7 +1797,7 @@ int band_apply(BandPrec *bp, int R, int q, const T *minv, const T *x, T *y, hipS
         for (SweepGraph &cand : bp->graph)
             if (cand.exec && cand.c == c && cand.pi == pi &&
                 cand.epoch == tune_epoch() &&
-                cand.nl == nlev &&
+                cand.nl == nlev && cand.kw == kw && cand.rc == rc &&
                 std::equal(key, key + kKey, cand.key)) {
                 g = &cand;
                 break;
@@ -1808,12 +1811,12 @@ int band_apply(BandPrec *bp, int R, int q, const T *minv, const T *x, T *y, hipS
                 g->exec = nullptr;
             }
             XT_HIP(hipStreamBeginCapture(bp->cap, hipStreamCaptureModeThreadLocal));
-            const int rc = sweeps(bp->cap);
+            const int status = sweeps(bp->cap);
             hipGraph_t graph = nullptr;
             const hipError_t e = hipStreamEndCapture(bp->cap, &graph);
-            if (rc != XT_OK || e != hipSuccess) {
+            if (status != XT_OK || e != hipSuccess) {
                 if (graph) (void)hipGraphDestroy(graph);
-                if (rc != XT_OK) return rc;
+                if (status != XT_OK) return status;
                 XT_HIP(e);
             }
             const hipError_t ei = hipGraphInstantiate(&g->exec, graph, nullptr, nullptr, 0);
@@ -1824,6 +1827,8 @@ int band_apply(BandPrec *bp, int R, int q, const T *minv, const T *x, T *y, hipS
             g->pi = pi;
             g->epoch = tune_epoch();
             g->nl = nlev;
+            g->kw = kw;
+            g->rc = rc;
             std::copy(key, key + kKey, g->key);
         }
         XT_HIP(hipGraphLaunch(g->exec, s));
