@@ -46,3 +46,34 @@ def test_captured_sweeps_follow_the_band(dev, block):
         W = coupled(K, reach)
         pr.refactor(*on_device(W))
         check(dev, pr, W, (3, 60), reach)
+
+
+def test_scratch_is_kept_from_the_first_refactorization_on(dev):
+    """A factor that is only built holds its matrices and no scratch; a second refactorization
+    takes no more memory than the first.  The scratch is the diagonal and the sub-diagonal
+    blocks in FP64, 16 bytes b^2 a block; memory is counted to half of it."""
+    import torch
+    b, nb = 1024, 24
+    K = strip(nb * b // 12 - 2)
+    small = dev.BandPreconditioner(strip(20))      # (the library's own first allocations)
+    small.refactor(*on_device(strip(20)))
+    torch.cuda.synchronize()
+    Kd = on_device(K)
+
+    def used():
+        torch.cuda.synchronize()
+        free, total = torch.cuda.mem_get_info()
+        return total - free
+
+    scratch = 16 * b * b * nb
+    start = used()
+    pr = dev.BandPreconditioner(K, block=b)
+    assert pr.nblocks == nb
+    built = used()
+    # D and D^T in both precisions; G and H are narrow here (64 of 1024 columns)
+    assert built - start < 24 * b * b * nb + scratch // 2
+    pr.refactor(*Kd)
+    once = used()
+    assert once - built > scratch // 2
+    pr.refactor(*Kd)
+    assert used() - once < scratch // 8

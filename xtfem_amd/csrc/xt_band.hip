@@ -1275,16 +1275,17 @@ static int factor_dev(BandPrec &bp, const int *dia, const int *dja, const double
     DevBuf &L = bp.sL, &E = bp.sE, &Wb = bp.sW, &Km = bp.sK, &info = bp.sinfo;
     struct Release {   // the scratch is freed on every way out unless it is kept
         BandPrec &bp;
+        const bool again;   // a refactorization: the factor was built before this call
         ~Release() {
             DevBuf *b[5] = {&bp.sL, &bp.sE, &bp.sW, &bp.sK, &bp.sinfo};
             size_t sum = 0;
             for (DevBuf *d : b) sum += d->bytes;
-            if (bp.built && bp.keep64 && sum <= kKeepScratch) return;
+            if (again && bp.keep64 && sum <= kKeepScratch) return;
             for (DevBuf *d : b) d->release();
             delete bp.rb;
             bp.rb = nullptr;
         }
-    } release{bp};
+    } release{bp, bp.built};
     struct Band {      // a failed factorization leaves the old factor's layout
         BandPrec &bp;
         const int kw, rc;
