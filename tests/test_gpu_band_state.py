@@ -77,3 +77,24 @@ def test_scratch_is_kept_from_the_first_refactorization_on(dev):
     assert once - built > scratch // 2
     pr.refactor(*Kd)
     assert used() - once < scratch // 8
+
+
+def test_refactorizations_on_streams_that_come_and_go(dev):
+    """Each refactorization on a stream of its own that is destroyed afterwards: what the
+    factor keeps refers to none of them."""
+    import ctypes as C
+    import torch
+    from xtfem_amd._lib import check as ok, lib
+    hip = lib()                      # (its symbols include those of the runtime it links)
+    K = strip(60)
+    pr = dev.BandPreconditioner(K, block=128)
+    for scale in (1.5, 0.7, 1.1):
+        K2 = (K[0], K[1], K[2] * scale)
+        ia, ja, a = on_device(K2)
+        torch.cuda.synchronize()
+        s = C.c_void_p()
+        assert hip.hipStreamCreate(C.byref(s)) == 0
+        ok(lib().xt_prec_refactor_band(pr.h, ia.data_ptr(), ja.data_ptr(), a.data_ptr(), s),
+           "refactor")
+        assert hip.hipStreamDestroy(s) == 0
+        check(dev, pr, K2, (6, 60), 3)

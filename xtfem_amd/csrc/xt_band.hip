@@ -1280,7 +1280,11 @@ static int factor_dev(BandPrec &bp, const int *dia, const int *dja, const double
             DevBuf *b[5] = {&bp.sL, &bp.sE, &bp.sW, &bp.sK, &bp.sinfo};
             size_t sum = 0;
             for (DevBuf *d : b) sum += d->bytes;
-            if (again && bp.keep64 && sum <= kKeepScratch) return;
+            if (again && bp.keep64 && sum <= kKeepScratch) {
+                // (the caller's stream may be gone by the next call)
+                if (bp.rb && bp.rb->h) (void)rocblas_set_stream(bp.rb->h, nullptr);
+                return;
+            }
             for (DevBuf *d : b) d->release();
             delete bp.rb;
             bp.rb = nullptr;
