@@ -1095,9 +1095,10 @@ int bsr_apply(const BsrPlan &P, int R, const T *tmat, double alpha, double beta,
     const T *bv = f32 ? (const T *)P.bval32.ptr : (const T *)P.bval64.ptr;
     const int c = 6 * R;
     // staged kernel: only when the tuning knob asks for it (2; measured slower than the
-    // lane-per-case kernel on the structured meshes here at 32 load cases)
-    const int lk = tune_knob(XT_TUNE_SPMM_LDS);
-    const int cc = (lk != 2 || R < 2) ? 0 : stage_cols<T>(P, c);
+    // lane-per-case kernel on the structured meshes here at 32 load cases) and the groups
+    // are not asked for as well
+    const int lk = tune_knob(XT_TUNE_SPMM_LDS), gk = tune_knob(XT_TUNE_SPMM_GROUP);
+    const int cc = (lk != 2 || gk == 2 || R < 2) ? 0 : stage_cols<T>(P, c);
     if (cc) {
         const int nch = c / cc;
         const int grid = (int)(((long long)P.nslices * nch + 7) / 8 * 8);
