@@ -259,6 +259,10 @@ int xt_prec_create_band_seg(int p, const int *rowptr, const int *colidx, const d
  * 0 for ILUT): ngroup, and when non-NULL the first DOF of each run and the end
  * (goff [ngroup+1]) and each run's block size (gblock [ngroup]). */
 int xt_prec_band_groups(xt_prec pr, int *ngroup, int *goff, int *gblock);
+/* Bytes of the matrices of K's banded factor that an apply in one precision streams, summed
+ * over its runs: D_i and D_i^T as stored (whole b x b blocks) and G_i, H_i (b x the band
+ * rounded up to 64), without the pairing products (0 for ILUT). */
+int xt_prec_band_bytes(xt_prec pr, int fp32, long long *bytes);
 /* Number of shifted factors of a preconditioner and (when shifts != NULL) their shifts. */
 int xt_prec_shifts(xt_prec pr, int *nshift, double *shifts);
 /* Refactor a banded-factor preconditioner with new values of K (1-based CSR in device

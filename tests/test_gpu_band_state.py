@@ -98,3 +98,38 @@ def test_refactorizations_on_streams_that_come_and_go(dev):
            "refactor")
         assert hip.hipStreamDestroy(s) == 0
         check(dev, pr, K2, (6, 60), 3)
+
+
+@pytest.mark.parametrize("block,fp32", [(768, False), (64, True)])
+def test_work_is_counted_on_the_band(dev, block, fp32):
+    """Algorithmic bytes and flops of an apply without pairing levels against those of its
+    launches (bytes within 2 %: the launches read the middle block's vector once for both
+    chains and a chain's own vectors twice where its rows are split), and the bytes of the
+    matrices: blocks of 768 rows with a band of 64, and blocks all band."""
+    import ctypes as C
+    import torch
+    from xtfem_amd import tune
+    from xtfem_amd._lib import check as ok, lib
+    nb, c, kw = 9, 32, 64
+    pr = dev.BandPreconditioner(strip(nb * block // 12 - 2), block=block)
+    assert pr.nblocks == nb
+    sv, dt = (4, torch.float32) if fp32 else (8, torch.float64)
+    assert pr.matrix_bytes(fp32) == sv * (2 * nb * block * block + 2 * (nb - 1) * block * kw)
+    x = torch.ones(pr.p * c, device="cuda", dtype=dt)
+    y = torch.empty_like(x)
+    kind = tune.XT_PROF_BAND if fp32 else tune.XT_PROF_BAND64
+    v = [C.c_double() for _ in range(5)]
+    n = C.c_longlong()
+    tune.set_knob("band_pair", 1)
+    try:
+        ok(lib().xt_prof_enable(1 << kind))
+        pr.apply(None, x, y, c, q=1, fp32=fp32)
+        ok(lib().xt_prof_read(kind, C.addressof(v[0]), C.addressof(n), C.addressof(v[1]),
+                              C.addressof(v[2])))
+        ok(lib().xt_prof_read_alg(kind, C.addressof(v[3]), C.addressof(v[4])))
+    finally:
+        ok(lib().xt_prof_enable(0))
+        tune.set_knob("band_pair", 0)
+    _, byts, flops, alg_bytes, alg_flops = (u.value for u in v)
+    assert alg_flops == pytest.approx(flops, rel=1e-9)
+    assert alg_bytes == pytest.approx(byts, rel=0.02)

@@ -1575,6 +1575,11 @@ void band_dims(const BandPrec *bp, int *b, int *nb, int *bw) {
 
 bool band_has_fp64(const BandPrec *bp) { return bp->keep64; }
 
+long long band_bytes(const BandPrec *bp, bool f32) {
+    const long long b = bp->b, n = bp->nb;
+    return (f32 ? 4 : 8) * (2 * b * b * n + 2 * b * bp->kw * (n - 1));
+}
+
 // x into the sweeps' workspace w (rows in the factor's order, ld columns): the temporal mix
 // with minv (NULL: none) of the active cases a < Ra (case cols[a], NULL: a), slot a's q
 // columns at a q; the rows past p zero.  One thread per row and slot.  Q: the q that is
@@ -1840,12 +1845,13 @@ int band_apply(BandPrec *bp, int R, int q, const T *minv, const T *x, T *y, hipS
     } else {
         XT_TRY(sweeps(s));
         // algorithmic work of the apply: the unpaired block recurrences, each factor block
-        // read once (D_i, D_i^T as triangles, G_i, H_i), each vector block read and written
-        // once per product (plus the read of the block it is subtracted from)
-        const double tri = (double)b * (b + 1) / 2, full = (double)b * b, vb = (double)b * c;
+        // read once (D_i, D_i^T as triangles, G_i, H_i: b x kw), each vector block read and
+        // written once per product (plus the read of the block it is subtracted from)
+        const double tri = (double)b * (b + 1) / 2, gh = (double)b * kw, vb = (double)b * c;
+        const double vg = (double)kw * c + 2.0 * vb;
         prof_alg(band_kind<T>(),
-                 sizeof(T) * (2.0 * (nb * tri + (nb - 1) * full) + 2.0 * (2.0 * nb + 3.0 * (nb - 1)) * vb),
-                 2.0 * (2.0 * nb * tri * c + 2.0 * (nb - 1) * full * c));
+                 sizeof(T) * (2.0 * (nb * tri + (nb - 1) * gh) + 2.0 * (2.0 * nb * vb + (nb - 1) * vg)),
+                 2.0 * (2.0 * nb * tri * c + 2.0 * (nb - 1) * gh * c));
     }
     XT_HIP(hipGetLastError());
 #define XT_STORE(Q)                                                                            \

@@ -265,6 +265,7 @@ int band_build(int p, const int *ia, const int *ja, const double *a, int block, 
 bool band_has_fp64(const BandPrec *bp);
 void band_delete(BandPrec *bp);
 void band_dims(const BandPrec *bp, int *b, int *nb, int *bw);
+long long band_bytes(const BandPrec *bp, bool f32);
 int band_refactor(BandPrec *bp, const int *dia, const int *dja, const double *da,
                   hipStream_t s, int first_row = 0);
 // Ra >= 0 with dcols (device, R entries, the Ra active cases first): the sweeps run on the

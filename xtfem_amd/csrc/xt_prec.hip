@@ -875,6 +875,13 @@ int xt_prec_band_groups(xt_prec pr, int *ngroup, int *goff, int *gblock) {
     return XT_OK;
 }
 
+int xt_prec_band_bytes(xt_prec pr, int fp32, long long *bytes) {
+    XT_ARG(pr && bytes, "prec_band_bytes arguments");
+    *bytes = pr->band ? band_bytes(pr->band, fp32 != 0) : 0;
+    for (const BandPrec *g : pr->groups) *bytes += band_bytes(g, fp32 != 0);
+    return XT_OK;
+}
+
 int xt_prec_shifts(xt_prec pr, int *nshift, double *shifts) {
     XT_ARG(pr, "prec");
     if (nshift) *nshift = (int)pr->shifts.size();

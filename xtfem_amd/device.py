@@ -239,13 +239,11 @@ class BandPreconditioner(IlutPreconditioner):
 
     def matrix_bytes(self, fp32):
         """Bytes of the four block-matrix sets one apply streams (D, D^T halves counted
-        as stored: whole b x b blocks; summed over the runs of a grouped factor)."""
-        sv = 4 if fp32 else 8
-        tot = 0
-        for g, b in enumerate(self.group_blocks):
-            nb = -(-int(self.group_offsets[g + 1] - self.group_offsets[g]) // int(b))
-            tot += sv * int(b) * int(b) * (2 * nb + 2 * (nb - 1))
-        return tot
+        as stored: whole b x b blocks; G and H: b rows by the band; summed over the runs of
+        a grouped factor)."""
+        n = C.c_longlong(0)
+        check(lib().xt_prec_band_bytes(self.h, int(fp32), C.addressof(n)), "prec_band_bytes")
+        return n.value
 
 
 def dominant_temporal_mode(A, B):
