@@ -45,6 +45,7 @@
 #include <algorithm>
 #include <cstring>
 #include <new>
+#include <type_traits>
 
 #include "xt_common.h"
 
@@ -184,6 +185,11 @@ __device__ __forceinline__ long long xcd_tile() {
 // bytes a lane, 128 contiguous bytes a row; column tiles go in pairs, lane t taking
 // columns 2 t and 2 t + 1 of the 32.  Output layout of the 4 accumulators per lane: f32
 // row 4 g + i, f64 row g + 4 i.
+// FP32 with few columns (CT = 1): a sum of its own for each step of a chunk, and the waves'
+// partial tiles added to one another and to the old value in FP64.  One FP32 chain a wave and
+// FP32 sums of the waves had 1.2 times the error of a sum over 256 threads and a tree (the
+// largest of y, mean of 72 factors, 6 columns; thermal ones 1.3 to 1.9); so it is 0.92, for 2
+// of 105 us an apply (768-row thermal blocks).  All sums in FP64 from the waves on: 0.80, 4 us.
 // nseg = 2: one item whose product is A[0] V[0] + A[1] V[1], half the waves each.
 // Consecutive tiles are the column tiles of one row tile, so one XCD's L2 serves its A.
 template <typename T, int RT, int CT, int KW, int PF>
@@ -195,6 +201,8 @@ band_prod_kernel(Items<T> it, int rows, int lda, int kdim, int tri, int ld, int 
     typedef T avec __attribute__((ext_vector_type(AV)));
     typedef T vpair __attribute__((ext_vector_type(2)));
     constexpr int CP = CT / 2;                      // column-tile pairs
+    constexpr int NA = sizeof(T) == 4 && CT == 1 ? 4 : 1;   // sums a tile, one per step of a chunk
+    typedef std::conditional_t<NA == 4, double, T> sum_t;   // what they are added in
     __shared__ T red[KW][RT * CT][4][64];
     const int ntx = rows / (16 * RT), nty = ld / (16 * CT);
     const long long tile = xcd_tile();
@@ -231,11 +239,13 @@ band_prod_kernel(Items<T> it, int rows, int lda, int kdim, int tri, int ld, int 
         const int u = wave + h * KW;
         if (sub && u < NU) old[h] = *out_at(u);
     }
-    acc_t acc[RT][CT];
+    acc_t acc[RT][CT][NA];
 #pragma unroll
     for (int i = 0; i < RT; ++i)
 #pragma unroll
-        for (int j = 0; j < CT; ++j) acc[i][j] = acc_t{T(0), T(0), T(0), T(0)};
+        for (int j = 0; j < CT; ++j)
+#pragma unroll
+            for (int s = 0; s < NA; ++s) acc[i][j][s] = acc_t{T(0), T(0), T(0), T(0)};
     T a[PF][RT][4], v[PF][CT][4];
     auto load = [&](int j, int ch) {
         const size_t ko = (size_t)16 * ch;
@@ -264,7 +274,8 @@ band_prod_kernel(Items<T> it, int rows, int lda, int kdim, int tri, int ld, int 
 #pragma unroll
             for (int i = 0; i < RT; ++i)
 #pragma unroll
-                for (int c = 0; c < CT; ++c) acc[i][c] = M::step(a[j][i][s], v[j][c][s], acc[i][c]);
+                for (int c = 0; c < CT; ++c)
+                    acc[i][c][s % NA] = M::step(a[j][i][s], v[j][c][s], acc[i][c][s % NA]);
     };
     if (n > 0) {
 #pragma unroll
@@ -294,20 +305,29 @@ band_prod_kernel(Items<T> it, int rows, int lda, int kdim, int tri, int ld, int 
 #pragma unroll
         for (int c = 0; c < CT; ++c)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) red[wave][i * CT + c][e][lane] = acc[i][c][e];
+            for (int e = 0; e < 4; ++e) {
+                T sum[NA];
+#pragma unroll
+                for (int s = 0; s < NA; ++s) sum[s] = acc[i][c][s][e];
+#pragma unroll
+                for (int d = NA / 2; d > 0; d /= 2)
+#pragma unroll
+                    for (int s = 0; s < d; ++s) sum[s] += sum[s + d];
+                red[wave][i * CT + c][e][lane] = sum[0];
+            }
     __syncthreads();
 #pragma unroll
     for (int h = 0; h < UW; ++h) {
         const int u = wave + h * KW;
         if (u >= NU) break;
-        T sum = red[0][u >> 2][u & 3][lane];
+        sum_t sum = red[0][u >> 2][u & 3][lane];
 #pragma unroll
         for (int w = 1; w < KW; ++w) sum += red[w][u >> 2][u & 3][lane];
         T *o = out_at(u);
-        *o = sub ? old[h] - sum : sum;
+        *o = (T)(sub ? old[h] - sum : sum);
         if (it.dup && z == it.dupz) {
             const long long at = o - (O + (size_t)it.dup0 * ld);
-            if (at >= 0) it.dup[at] = sum;
+            if (at >= 0) it.dup[at] = (T)sum;
         }
     }
 }
