@@ -28,11 +28,14 @@
 // Storage ("node groups", kron_group_kernel, several load cases on enough nodes): kG
 // consecutive nodes share the sorted union of their neighbours; the blocks stand
 // neighbour by neighbour (only the couplings that exist), so a wave whose lanes are
-// columns reads each neighbour's rows of X once for all nodes of the group.
+// columns reads each neighbour's rows of X once for all nodes of the group.  The values of a
+// precision are copied from the slices by the first apply that takes the groups, and kept
+// up to date from then on: a program with one load case never holds them.
 //
 // The path is for q = 6 temporal functions (three quadratic temporal nodes, each with a
 // sine enrichment: 2*nnte, main3d.f90:172).
 #include <algorithm>
+#include <mutex>
 #include <vector>
 
 #include "xt_common.h"
@@ -52,11 +55,14 @@ struct BsrPlan {
     DevBuf kmap, mmap;      // value position in bval of every CSR entry of K and of M
     long long nk = 0, nm = 0;
     // Group form: neighbours gptr[s] .. gptr[s + 1] - 1 of group s as (node, 16 b + mask of the
-    // group's nodes it couples to), its blocks from gblk[s] + b on (nodes ascending); gkmap,
-    // gmmap as kmap, mmap.
+    // group's nodes it couples to), its blocks from gblk[s] + b on (nodes ascending); gof: group
+    // block of each stored block, -1 for padding.  Values ([nreal][12]) by group_values, gmutex
+    // held: applies of several threads may be the first.
     int ngroups = 0;
     long long ngnbr = 0;    // neighbours of all groups
-    DevBuf gptr, gblk, gnbr, gval32, gval64, gkmap, gmmap;
+    DevBuf gptr, gblk, gnbr, gof, gval32, gval64;
+    bool no_gval[2] = {};   // no memory for the FP64 [0], FP32 [1] values: slices instead
+    std::mutex gmutex;
     // Staged form: the distinct column nodes of each slice (its neighbour set, sorted),
     // unode[ubase[s] .. ubase[s] + ulen[s]), and for every stored block the position of
     // its column node in that list (uint16), so a workgroup can stage the slice's rows
@@ -69,10 +75,6 @@ static constexpr int kSlice = 64;
 static constexpr int kG = 4;   // nodes of a group
 static constexpr int kTS = 73;   // LDS stride of a case's temporal matrices (odd)
 
-__global__ void __launch_bounds__(256)
-bsr_scatter_kernel(long long n, const int *__restrict__ map, const int *__restrict__ gmap,
-                   const double *__restrict__ v, double *__restrict__ b64,
-                   float *__restrict__ b32, double *__restrict__ g64, float *__restrict__ g32);
 __global__ void __launch_bounds__(256) bsr_zero_kernel(long long n, double *d, float *f) {
     const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
     if (i < n) {
@@ -82,8 +84,8 @@ __global__ void __launch_bounds__(256) bsr_zero_kernel(long long n, double *d, f
 }
 int bsr_set_values(BsrPlan &P, const double *kv, const double *mv, hipStream_t s);
 
-// Build the node-slice and node-group forms (kv, mv: the CSR values on the device); returns
-// XT_E_UNSUPPORTED if K/M are not 3x3-blocked with diagonal M blocks.
+// Build the node-slice form and the node groups' lists (kv, mv: the CSR values on the
+// device); returns XT_E_UNSUPPORTED if K/M are not 3x3-blocked with diagonal M blocks.
 int bsr_build(int p, const int *krp, const int *kci, const double *kv, const int *mrp,
               const int *mci, const double *mv, BsrPlan &P) {
     if (p % 3) return XT_E_UNSUPPORTED;
@@ -134,8 +136,8 @@ int bsr_build(int p, const int *krp, const int *kci, const double *kv, const int
     }
     if (nb * 12 > 0x7fffffffLL) return XT_E_UNSUPPORTED;
     std::vector<int> bcol(nb);
-    std::vector<int> pos(nn, -1), gat(nn, 0);  // entry and group block of column node b in the row
-    std::vector<int> kmap(krp[p]), mmap(mrp[p]), gkmap(krp[p]), gmmap(mrp[p]);
+    std::vector<int> pos(nn, -1);   // entry of column node b in the row
+    std::vector<int> kmap(krp[p]), mmap(mrp[p]), gof(nb, -1);
     // groups: merge the kG sorted neighbour lists; gpos: block of each of row a's neighbours,
     // from cfirst[a] on
     const int ngroups = ceil_div(nn, kG);
@@ -199,14 +201,14 @@ int bsr_build(int p, const int *krp, const int *kci, const double *kv, const int
             } else {
                 for (int e = 0; e < (int)c.size(); ++e) pos[c[e]] = e;
             }
-            for (int e = 0; e < (int)c.size(); ++e) gat[c[e]] = gpos[cfirst[a] + e];
+            for (int e = 0; e < (int)c.size(); ++e)
+                gof[(long long)base[s] + (long long)pos[c[e]] * kSlice + k] = gpos[cfirst[a] + e];
             for (int d = 0; d < 3; ++d) {
                 const int i = 3 * a + d;
                 for (int e = krp[i]; e < krp[i + 1]; ++e) {
                     const int b = kci[e] / 3, cd = kci[e] % 3;
                     const long long idx = (long long)base[s] + (long long)pos[b] * kSlice + k;
                     kmap[e] = (int)(idx * 12 + d * 3 + cd);
-                    gkmap[e] = gat[b] * 12 + d * 3 + cd;
                     if (klast[kci[e]] >= krp[i]) kmap[klast[kci[e]]] = -1;   // the last one stands
                     klast[kci[e]] = e;
                 }
@@ -214,7 +216,6 @@ int bsr_build(int p, const int *krp, const int *kci, const double *kv, const int
                     const int b = mci[e] / 3;
                     const long long idx = (long long)base[s] + (long long)pos[b] * kSlice + k;
                     mmap[e] = (int)(idx * 12 + 9 + d);
-                    gmmap[e] = gat[b] * 12 + 9 + d;
                     if (mlast[mci[e]] >= mrp[i]) mmap[mlast[mci[e]]] = -1;
                     mlast[mci[e]] = e;
                 }
@@ -262,23 +263,18 @@ int bsr_build(int p, const int *krp, const int *kci, const double *kv, const int
     P.nm = mrp[p];
     if (P.nk) XT_TRY(P.kmap.upload(kmap.data(), sizeof(int) * P.nk));
     if (P.nm) XT_TRY(P.mmap.upload(mmap.data(), sizeof(int) * P.nm));
-    if (P.nk) XT_TRY(P.gkmap.upload(gkmap.data(), sizeof(int) * P.nk));
-    if (P.nm) XT_TRY(P.gmmap.upload(gmmap.data(), sizeof(int) * P.nm));
+    XT_TRY(P.gof.upload(gof.data(), sizeof(int) * nb));
     P.ngroups = ngroups;
     P.ngnbr = gptr[ngroups];
     XT_TRY(P.gptr.upload(gptr.data(), sizeof(int) * gptr.size()));
     XT_TRY(P.gblk.upload(gblk.data(), sizeof(int) * gblk.size()));
     XT_TRY(P.gnbr.upload(gnbr.data(), sizeof(int) * gnbr.size()));
     // the values, from the CSR values already on the device
-    const long long nv = nb * 12, ng = ((long long)gblk[ngroups] + 1) * 12;
+    const long long nv = nb * 12;
     XT_TRY(P.bval64.reserve(sizeof(double) * nv));
     XT_TRY(P.bval32.reserve(sizeof(float) * nv));
-    XT_TRY(P.gval64.reserve(sizeof(double) * ng));
-    XT_TRY(P.gval32.reserve(sizeof(float) * ng));
     hipLaunchKernelGGL(bsr_zero_kernel, dim3(ceil_div(nv, 256)), dim3(256), 0, 0, nv,
                        P.bval64.as<double>(), P.bval32.as<float>());
-    hipLaunchKernelGGL(bsr_zero_kernel, dim3(ceil_div(ng, 256)), dim3(256), 0, 0, ng,
-                       P.gval64.as<double>(), P.gval32.as<float>());
     XT_HIP(hipGetLastError());
     XT_TRY(bsr_set_values(P, kv, mv, 0));
     XT_HIP(hipDeviceSynchronize());
@@ -978,33 +974,81 @@ kron_bsr3_r1_kernel(int nslices, const int *__restrict__ slot_node,
     }
 }
 
-// K and M values (CSR entries in the order the plan was built from) into the node blocks of
-// both forms, FP64 and FP32.
+// K and M values (CSR entries in the order the plan was built from) into the node blocks,
+// FP64 and FP32.
 __global__ void __launch_bounds__(256)
-bsr_scatter_kernel(long long n, const int *__restrict__ map, const int *__restrict__ gmap,
-                   const double *__restrict__ v, double *__restrict__ b64,
-                   float *__restrict__ b32, double *__restrict__ g64, float *__restrict__ g32) {
+bsr_scatter_kernel(long long n, const int *__restrict__ map, const double *__restrict__ v,
+                   double *__restrict__ b64, float *__restrict__ b32) {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const int t = map[i], u = gmap[i];
+    const int t = map[i];
     if (t < 0) return;   // an entry that a later one of the row replaces
     const double w = v[i];
     b64[t] = w;
     b32[t] = (float)w;
-    g64[u] = w;
-    g32[u] = (float)w;
+}
+
+// The slices' blocks to the groups, a 16-byte piece a lane (PPB a block; n pieces).
+template <int PPB>
+__global__ void __launch_bounds__(256)
+bsr_group_kernel(long long n, const int *__restrict__ gof, const F4 *__restrict__ b,
+                 F4 *__restrict__ g) {
+    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int blk = (int)(i / PPB), u = gof[blk];
+    if (u >= 0) g[(long long)u * PPB + (i - (long long)blk * PPB)] = b[i];
+}
+template <typename T>
+static int copy_groups(const BsrPlan &P, const DevBuf &b, const DevBuf &g, hipStream_t s) {
+    constexpr int PPB = 12 * sizeof(T) / 16;
+    const long long n = P.nblocks * PPB;
+    hipLaunchKernelGGL(bsr_group_kernel<PPB>, dim3(ceil_div(n, 256)), dim3(256), 0, s, n,
+                       P.gof.as<int>(), b.as<F4>(), g.as<F4>());
+    XT_HIP(hipGetLastError());
+    return XT_OK;
 }
 
 int bsr_set_values(BsrPlan &P, const double *kv, const double *mv, hipStream_t s) {
     if (P.nk)
         hipLaunchKernelGGL(bsr_scatter_kernel, dim3(ceil_div(P.nk, 256)), dim3(256), 0, s, P.nk,
-                           P.kmap.as<int>(), P.gkmap.as<int>(), kv, P.bval64.as<double>(),
-                           P.bval32.as<float>(), P.gval64.as<double>(), P.gval32.as<float>());
+                           P.kmap.as<int>(), kv, P.bval64.as<double>(), P.bval32.as<float>());
     if (P.nm)
         hipLaunchKernelGGL(bsr_scatter_kernel, dim3(ceil_div(P.nm, 256)), dim3(256), 0, s, P.nm,
-                           P.mmap.as<int>(), P.gmmap.as<int>(), mv, P.bval64.as<double>(),
-                           P.bval32.as<float>(), P.gval64.as<double>(), P.gval32.as<float>());
+                           P.mmap.as<int>(), mv, P.bval64.as<double>(), P.bval32.as<float>());
     XT_HIP(hipGetLastError());
+    std::lock_guard<std::mutex> lock(P.gmutex);
+    if (P.gval64.ptr) XT_TRY(copy_groups<double>(P, P.bval64, P.gval64, s));
+    if (P.gval32.ptr) XT_TRY(copy_groups<float>(P, P.bval32, P.gval32, s));
+    return XT_OK;
+}
+
+// The groups' values in T (NULL: the slices are to be taken), copied by the first caller and
+// complete when it returns, whatever streams the next ones use.  A graph capture allocates
+// nothing, so an operator's first apply there takes the slices, as does one without memory
+// for a second copy.
+template <typename T>
+static int group_values(BsrPlan &P, hipStream_t s, const T **out) {
+    const bool f32 = sizeof(T) == 4;
+    DevBuf &g = f32 ? P.gval32 : P.gval64;
+    std::lock_guard<std::mutex> lock(P.gmutex);
+    if (!g.ptr && !P.no_gval[f32]) {
+        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+        XT_HIP(hipStreamIsCapturing(s, &capturing));
+        if (capturing == hipStreamCaptureStatusNone) {
+            if (g.reserve(sizeof(T) * 12 * (size_t)P.nreal) != XT_OK) {
+                (void)hipGetLastError();   // (not an error of this call)
+                P.no_gval[f32] = true;
+            } else {
+                int rc = copy_groups<T>(P, f32 ? P.bval32 : P.bval64, g, s);
+                if (rc == XT_OK && hipStreamSynchronize(s) != hipSuccess) rc = XT_E_HIP;
+                if (rc != XT_OK) {
+                    g.release();
+                    return rc;
+                }
+            }
+        }
+    }
+    *out = g.as<T>();
     return XT_OK;
 }
 
@@ -1090,7 +1134,7 @@ static bool group_form(const BsrPlan &P, int R, bool f32) {
 }
 
 template <typename T>
-int bsr_apply(const BsrPlan &P, int R, const T *tmat, double alpha, double beta, const T *x,
+int bsr_apply(BsrPlan &P, int R, const T *tmat, double alpha, double beta, const T *x,
               T *y, bool f32, hipStream_t s) {
     const T *bv = f32 ? (const T *)P.bval32.ptr : (const T *)P.bval64.ptr;
     const int c = 6 * R;
@@ -1129,10 +1173,11 @@ int bsr_apply(const BsrPlan &P, int R, const T *tmat, double alpha, double beta,
         XT_HIP(hipGetLastError());
         return XT_OK;
     }
-    if (group_form(P, R, f32)) {
+    const T *gv = nullptr;
+    if (group_form(P, R, f32)) XT_TRY(group_values<T>(P, s, &gv));
+    if (gv) {
         // cases split evenly over launches' second dimension, at most 32 a wave
         const int nchunk = ceil_div(R, 32), per = ceil_div(R, nchunk);
-        const T *gv = f32 ? (const T *)P.gval32.ptr : (const T *)P.gval64.ptr;
         if (prof_on(XT_PROF_SPMM)) prof_begin(XT_PROF_SPMM, s);
 #define XT_GROUP(LPG)                                                                          \
     {                                                                                          \
@@ -1216,9 +1261,9 @@ int bsr_apply(const BsrPlan &P, int R, const T *tmat, double alpha, double beta,
     }
     return XT_OK;
 }
-template int bsr_apply<float>(const BsrPlan &, int, const float *, double, double, const float *,
+template int bsr_apply<float>(BsrPlan &, int, const float *, double, double, const float *,
                               float *, bool, hipStream_t);
-template int bsr_apply<double>(const BsrPlan &, int, const double *, double, double,
+template int bsr_apply<double>(BsrPlan &, int, const double *, double, double,
                                const double *, double *, bool, hipStream_t);
 
 }  // namespace xt

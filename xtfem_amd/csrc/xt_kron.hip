@@ -321,7 +321,7 @@ struct BsrPlan;
 int bsr_build(int p, const int *krp, const int *kci, const double *kv, const int *mrp,
               const int *mci, const double *mv, BsrPlan &P);
 template <typename T>
-int bsr_apply(const BsrPlan &P, int R, const T *tmat, double alpha, double beta, const T *x,
+int bsr_apply(BsrPlan &P, int R, const T *tmat, double alpha, double beta, const T *x,
               T *y, bool f32, hipStream_t s);
 BsrPlan *bsr_new();
 void bsr_delete(BsrPlan *);
