@@ -544,9 +544,9 @@ int xt_graphs_enable(int on);
  *                         the columns)                                      1, 2
  *   XT_TUNE_SPMM_GROUP    node-block SpMM, several load cases: the kernel that reads each
  *                         neighbour's rows of X once for a group of four nodes never 1,
- *                         always 2 (built-in: from about 60000 to 300000 nodes times
- *                         cases on, by precision and cases); where it runs, UNR, WPB and LDS
- *                         have no effect                                    1, 2
+ *                         always 2 (built-in: from about 68000 to 280000 nodes times
+ *                         cases on, by precision, cases and the pattern); where it runs, UNR,
+ *                         WPB and LDS have no effect                        1, 2
  * XT_E_ARG for a value a knob does not take. */
 #define XT_TUNE_SPMM_UNR 0
 #define XT_TUNE_SPMM_WPB 1

@@ -1099,38 +1099,33 @@ static int slice_lanes(int R, int nslices) {
 // its first group, a chain of loads, whatever the number of groups (a group's neighbours
 // shared by the four waves of a workgroup: 13 to 18 us, but slower at every size from 4879
 // nodes on in FP64 and 13237 in FP32, and no better than slices below).  The slices' time
-// grows with nodes times cases (work, in thousands below); above 8 cases the groups' with
-// their lanes, close to a power of two, hence the share of it that the cases fill.
-// Slices / groups, us, at work (cases):
-//   FP64  137 (3) 66 / 66, 207 (3) 106 / 90, 163 (4) 71 / 83, 183 (4) 73 / 69, 165 (6) 70 / 62,
-//         139 (8) 59 / 60, 136 (9) 62 / 45, 157 (9) 67 / 67, 106 (12) 42 / 48, 142 (16) 60 / 50,
-//         83 (20) 36 / 36, 128 (20) 48 / 38, 91 (28) 37 / 27, 79 (36) 33 / 36, 117 (36) 47 / 37,
-//         150 (36) 60 / 65, 104 (40) 40 / 34
-//   FP32  276 (4) 63 / 61, 345 (5) 80 / 62, 245 (6) 50 / 61, 274 (6) 64 / 51, 327 (8) 61 / 62,
-//         247 (9) 53 / 68, 368 (9) 75 / 77, 181 (12) 38 / 39, 249 (14) 49 / 42, 242 (16) 48 / 40,
-//         257 (17) 51 / 51, 153 (24) 33 / 33, 179 (28) 38 / 31, 133 (32) 30 / 31,
-//         290 (36) 59 / 50, 320 (36) 61 / 72, 373 (42) 72 / 72
-// Far above these the slices' time goes with stored blocks times cases, the groups' with their
-// neighbours, 9 (four nodes across a mesh) to 13.5 a node, times the lanes for the cases: share
-// is where they meet.  On thick meshes few cases stay with the slices at any size (FP64: 2
-// cases on 115351 nodes 146 / 208, 3 there 210 / 214, but 161 / 127 on 95793 nodes 3 across;
-// FP32: 4 there 95 / 118, 6 on 52521 nodes 65 / 76, 9 there 95 / 112, 9 on 61004 nodes 4
-// across 110 / 91, 17 on 29791 nodes 95 / 98).
+// grows with nodes times cases, the groups' with their neighbours, 26 a group (3 x 3 nodes in
+// the section) to 51 (40 x 9), so the line lies in nodes times cases at 45 a group (work, in
+// thousands below; a section 5 nodes across).  Slices / groups, us, at work (cases):
+//   FP64  197 (4) 79 / 102, 275 (4) 125 / 117, 281 (4) 79 / 84, 340 (4) 77 / 72, 95 (8) 36 / 41,
+//         134 (8) 55 / 55, 232 (8) 55 / 41, 267 (8) 104 / 109, 395 (8) 142 / 130, 106 (9) 42 / 45,
+//         151 (9) 63 / 62, 184 (9) 42 / 33, 95 (16) 35 / 34, 132 (16) 53 / 45, 59 (20) 24 / 27,
+//         83 (20) 35 / 35, 118 (20) 45 / 36, 106 (36) 40 / 36, 123 (36) 31 / 23
+//   FP32  267 (8) 58 / 59, 327 (8) 36 / 32, 395 (8) 77 / 75, 200 (12) 40 / 52, 284 (12) 58 / 54,
+//         166 (20) 34 / 40, 236 (20) 45 / 41, 166 (28) 33 / 31, 232 (28) 45 / 38, 213 (36) 42 / 41,
+//         298 (36) 58 / 68, 425 (36) 77 / 74
+// The groups' time goes in rounds of the waves that the card holds (16 lanes a group: 32768
+// nodes in FP64, 49152 in FP32), so just above one they lose up to 15 % (FP64, 6 cases on 33900
+// nodes: 79 / 90).  In FP32 the stored blocks times cases have to outweigh the neighbours times
+// the lanes as well (share; 4 cases on 99972 nodes 82 / 103, 36 on 8400 59 / 68).  Over 2480
+// operators (40 to 800 thousand nodes times cases, 2 to 64 cases, eight sections) the choice
+// takes 1.005 times the better kernel's time, 1.32 at most (FP64, 14 cases on 3900 nodes).
 static bool group_form(const BsrPlan &P, int R, bool f32) {
     const int k = tune_knob(XT_TUNE_SPMM_GROUP);
     if (R < 2 || k == 1) return false;
     if (k == 2) return true;
+    if (R < (f32 ? 5 : 3)) return false;
     const int chunks = ceil_div(R, 32), per = ceil_div(R, chunks);
-    const double share = f32 ? (per <= 8 ? 13 : per <= 16 ? 25 : 36) * chunks : R <= 4 ? 8 : 0;
+    const double share = f32 ? (per <= 8 ? 15 : per <= 16 ? 28 : 40) * chunks : 0;
     if ((double)R * P.nblocks <= share * P.ngnbr) return false;
-    int up = 1;
-    while (up < R) up <<= 1;
-    const long long work = (long long)P.nn * R;
-    if (R <= 8) return work >= (f32 ? 270000 : R > 4 ? 140000 : 180000);
-    const long long filled = work * R / up;
-    if (R <= 16) return filled >= (f32 ? 200000 : 85000);
-    if (R <= 32) return filled >= (f32 ? 155000 : 55000);
-    return filled >= (f32 ? 160000 : 62000);
+    const double work = (double)P.nn * R * 45 * P.ngroups / P.ngnbr;
+    if (f32) return work >= (R <= 16 ? 280000 : 200000);
+    return work >= (R <= 4 ? 270000 : R <= 16 ? 115000 : 68000);
 }
 
 template <typename T>
