@@ -432,6 +432,25 @@ static int run_tri(const Tri &tri, const T *vals, const T *dinv, int c, const T 
 constexpr long long kOneWgWork = 4LL << 20;
 // ... and keep the solution vector in LDS when it fits this many bytes.
 constexpr size_t kOneWgLds = 128 * 1024;
+// Whether both sweeps in a workgroup for each two columns (trsv_sf_kernel) beat the kernels
+// above, by estimates in us of what each is bound by (rl: mean entries of a factor row):
+//   two columns a workgroup  its rows, 0.1 for both sweeps, or its levels, 0.2 + 0.006 rl
+//                            (512 columns at a time)
+//   one workgroup            a barrier a level and its longest row, 0.45 + 0.11 rl, and every
+//                            entry and column, 0.45 ns
+//   a launch a level         3.7 + 0.1 rl
+// Two columns / the others, us, 6 columns: 4000 rows, 80 levels of 1 entry a row 404 / 65, 800
+// levels 405 / 410, 7950 levels of 34 entries 3150 / 34500; 300 rows, 40 levels 36 / 25, 86
+// levels 37 / 43; 975 rows, 529 levels of 17 entries 149 / 1105.  Over 1106 factors and column
+// counts the choice takes 1.004 times the better one's time (1.36 by levels per row alone).
+static bool two_columns_pay(const xt_prec_s &pr, int c) {
+    const double p = pr.p, nnz = (double)(pr.L.m.nnz + pr.U.m.nnz), rl = nnz / (2 * p);
+    const double levels = (double)(pr.L.lev_ptr.size() + pr.U.lev_ptr.size()) - 2;
+    const double sf = std::max(6 + 0.1 * p, levels * (0.2 + 0.006 * rl)) * ceil_div(c, 512);
+    const bool one = (nnz + 2 * p) * c <= kOneWgWork;
+    return sf <= (one ? levels * (0.45 + 0.11 * rl) + 0.45e-3 * (nnz + 2 * p) * c
+                      : levels * (3.7 + 0.1 * rl));
+}
 // ILUT sweeps Y = (LU)^-1 X Minv_r^T.  stage: p*q*R elements of device memory for the
 // temporal mix (used only when minv is given); timed: per-launch HIP-event timing when
 // enabled (it creates events, so the allocation-free entry point passes false).
@@ -447,13 +466,12 @@ static int ilut_apply(xt_prec pr, int R, int q, const T *minv, const T *x, T *y,
     const T *lv = f32 ? (const T *)pr->L.m.val32.ptr : (const T *)pr->L.m.val64.ptr;
     const T *uv = f32 ? (const T *)pr->U.m.val32.ptr : (const T *)pr->U.m.val64.ptr;
     const T *dv = f32 ? (const T *)pr->dinv32.ptr : (const T *)pr->dinv64.ptr;
-    // Factors with slots and levels of 100 rows at most (mean of both sweeps): both sweeps of
-    // two columns in one workgroup (0.3 us a level, 0.04 a row; 512 columns at a time).
-    // Others of little work: one workgroup with a barrier per level (2.5 us); else one launch
-    // per level over the whole device (4 us).
+    // Factors with slots: both sweeps of two columns in one workgroup where that pays.  Others
+    // of little work: one workgroup with a barrier per level; else one launch per level over
+    // the whole device.
     const long long work = (pr->L.m.nnz + pr->U.m.nnz + 2LL * pr->p) * c;
-    const long long levels = (long long)pr->L.lev_ptr.size() + pr->U.lev_ptr.size() - 2;
-    const bool slots = pr->L.slot_ci.ptr && pr->U.slot_ci.ptr && 50 * levels >= pr->p && c <= 4096;
+    const bool slots = pr->L.slot_ci.ptr && pr->U.slot_ci.ptr && c <= 4096 &&
+                       two_columns_pay(*pr, c);
     if (slots || work <= kOneWgWork) {
         const bool prof = timed && prof_on(XT_PROF_TRSV);
         if (prof) prof_begin(XT_PROF_TRSV, s);
