@@ -172,8 +172,10 @@ static int launch_kron(const DevCSR *S, int p, int q, int R, const T *tmat, doub
         A.v[t] = fp32 ? (const T *)S[t].val32.ptr : (const T *)S[t].val64.ptr;
     }
     const int c = q * R;
-    // (80000: 9455 rows with 9 columns equal, with 12 slower, by the figures at the kernel)
-    const int split = (long long)p * c <= 80000 && c <= 32 ? 8 : 1;
+    // (80000: 9455 rows with 9 columns equal, with 12 slower, by the figures at the kernel.  Past
+    // 16 columns a workgroup of 8 lanes holds one row and idles in part: 3355 rows, 18 columns
+    // FP64 10.9 / 8.2 us with one lane; 1845 rows 8.2 / 8.2)
+    const int split = (long long)p * c <= (c <= 16 ? 80000 : 50000) && c <= 32 ? 8 : 1;
     const int tile = (256 / split / q) * q;  // whole right-hand sides per tile
     for (int col0 = 0; col0 < c; col0 += tile) {
         const int ct = (c - col0) < tile ? (c - col0) : tile;
