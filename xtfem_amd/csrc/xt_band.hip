@@ -185,14 +185,14 @@ __device__ __forceinline__ long long xcd_tile() {
 // bytes a lane, 128 contiguous bytes a row; column tiles go in pairs, lane t taking
 // columns 2 t and 2 t + 1 of the 32.  Output layout of the 4 accumulators per lane: f32
 // row 4 g + i, f64 row g + 4 i.
-// FP32 with few columns (CT = 1): a sum of its own for each step of a chunk, and the waves'
+// FP32 with up to 16 columns (NA = 4): a sum of its own for each step of a chunk, and the waves'
 // partial tiles added to one another and to the old value in FP64.  One FP32 chain a wave and
 // FP32 sums of the waves had 1.2 times the error of a sum over 256 threads and a tree (the
 // largest of y, mean of 72 factors, 6 columns; thermal ones 1.3 to 1.9); so it is 0.92, for 2
 // of 105 us an apply (768-row thermal blocks).  All sums in FP64 from the waves on: 0.80, 4 us.
 // nseg = 2: one item whose product is A[0] V[0] + A[1] V[1], half the waves each.
 // Consecutive tiles are the column tiles of one row tile, so one XCD's L2 serves its A.
-template <typename T, int RT, int CT, int KW, int PF>
+template <typename T, int RT, int CT, int KW, int PF, int NA>
 __global__ void __launch_bounds__(64 * KW)
 band_prod_kernel(Items<T> it, int rows, int lda, int kdim, int tri, int ld, int sub, int nseg) {
     using M = Mfma<T>;
@@ -201,8 +201,7 @@ band_prod_kernel(Items<T> it, int rows, int lda, int kdim, int tri, int ld, int 
     typedef T avec __attribute__((ext_vector_type(AV)));
     typedef T vpair __attribute__((ext_vector_type(2)));
     constexpr int CP = CT / 2;                      // column-tile pairs
-    constexpr int NA = sizeof(T) == 4 && CT == 1 ? 4 : 1;   // sums a tile, one per step of a chunk
-    typedef std::conditional_t<NA == 4, double, T> sum_t;   // what they are added in
+    typedef std::conditional_t<NA == 4, double, T> sum_t;   // what the waves' sums are added in
     __shared__ T red[KW][RT * CT][4][64];
     const int ntx = rows / (16 * RT), nty = ld / (16 * CT);
     const long long tile = xcd_tile();
@@ -457,17 +456,18 @@ static int launch_prod(const Items<T> &it, int rows, int lda, int kdim, int tri,
     auto grid = [&](int tr, int tc) {
         return dim3((unsigned)(ceil_div((long long)(rows / tr) * ceil_div(ld, tc) * it.n, 8) * 8));
     };
-#define XT_PROD(RT, CT, KW, PF)                                                              \
-    hipLaunchKernelGGL((band_prod_kernel<T, RT, CT, KW, PF>), grid(16 * RT, 16 * CT),         \
+    constexpr int few = sizeof(T) == 4 ? 4 : 1;   // sums a tile with up to 16 columns
+#define XT_PROD(RT, CT, KW, PF, NA)                                                          \
+    hipLaunchKernelGGL((band_prod_kernel<T, RT, CT, KW, PF, NA>), grid(16 * RT, 16 * CT),     \
                        dim3(64 * KW), 0, s, it, rows, lda, kdim, tri, ld, (int)sub, nseg)
     if (ld == 16) {
         // few columns: the matrix is streamed once; two row tiles share V's loads where
         // that leaves enough workgroups (4.3 TB/s in the passes over 92 768-row blocks)
         const int sk = tune_knob(XT_TUNE_BAND_SMALLC);
         const bool rt2 = sk == 2 || (sk != 1 && (long long)rows / 32 * it.n >= 512);
-        if (rt2 && rows % 32 == 0) XT_PROD(2, 1, 4, 4);
-        else if (tune_knob(XT_TUNE_BAND_CHAIN_FEW) == 2) XT_PROD(1, 1, 4, 4);
-        else XT_PROD(1, 1, 8, 2);
+        if (rt2 && rows % 32 == 0) XT_PROD(2, 1, 4, 4, few);
+        else if (tune_knob(XT_TUNE_BAND_CHAIN_FEW) == 2) XT_PROD(1, 1, 4, 4, few);
+        else XT_PROD(1, 1, 8, 2, few);
     } else if (const long long tiles = (long long)(rows / 64) * ceil_div(ld, 64) * it.n;
                rows % 64 == 0 && nseg == 1 && tiles >= kBatchedTiles) {
         const int tk = tune_knob(XT_TUNE_BAND_TILE);
@@ -505,12 +505,12 @@ static int launch_prod(const Items<T> &it, int rows, int lda, int kdim, int tri,
             }
         const bool one = (long long)(rows / (16 * rt)) * (ld / (16 * ct)) * it.n <= 256;
         // (a workgroup alone on its CU: 8 waves, two a SIMD, hide more of the loads)
-        if (rt == 2 && ct == 3 && one) XT_PROD(2, 3, 8, 2);
-        else if (rt == 2 && ct == 3) XT_PROD(2, 3, 4, 2);
-        else if (rt == 2) XT_PROD(2, 2, 4, 2);
-        else if (ct == 3) XT_PROD(1, 3, 4, 3);
-        else if (ct == 2) XT_PROD(1, 2, 4, 3);
-        else XT_PROD(1, 1, 4, 4);
+        if (rt == 2 && ct == 3 && one) XT_PROD(2, 3, 8, 2, 1);
+        else if (rt == 2 && ct == 3) XT_PROD(2, 3, 4, 2, 1);
+        else if (rt == 2) XT_PROD(2, 2, 4, 2, 1);
+        else if (ct == 3) XT_PROD(1, 3, 4, 3, 1);
+        else if (ct == 2) XT_PROD(1, 2, 4, 3, 1);
+        else XT_PROD(1, 1, 4, 4, 1);
     }
 #undef XT_PROD
     if (prof) {
