@@ -1602,12 +1602,11 @@ long long band_bytes(const BandPrec *bp, bool f32) {
 
 // x into the sweeps' workspace w (rows in the factor's order, ld columns): the temporal mix
 // with minv (NULL: none) of the active cases a < Ra (case cols[a], NULL: a), slot a's q
-// columns at a q; the rows past p zero.  One thread per row and slot.  Q: the q that is
-// unrolled, 0 for any.  The sums run
-// in the order of temporal_mix.
+// columns at a q; the rows past p zero.  n rows and slots from row first on, one thread each.
+// Q: the q that is unrolled, 0 for any.  The sums run in the order of temporal_mix.
 template <typename T, int Q>
 __global__ void __launch_bounds__(256)
-band_load_kernel(unsigned n, int p, int split, int total, int R, int q, int Ra,
+band_load_kernel(unsigned n, int first, int p, int split, int total, int R, int q, int Ra,
                  const int *__restrict__ cols, int ld, const T *__restrict__ minv,
                  const T *__restrict__ x, T *__restrict__ w) {
     constexpr int LM = Q ? 256 * Q : 1;
@@ -1619,10 +1618,10 @@ band_load_kernel(unsigned n, int p, int split, int total, int R, int q, int Ra,
     }
     const unsigned idx = blockIdx.x * 256u + threadIdx.x;
     if (idx >= n) return;
-    const unsigned row = idx / (unsigned)Ra;
-    const int a = (int)(idx - row * (unsigned)Ra);
+    const unsigned slot_row = idx / (unsigned)Ra;
+    const int row = first + (int)slot_row, a = (int)(idx - slot_row * (unsigned)Ra);
     T *o = w + (size_t)row * ld + a * q;
-    const int dof = (int)row < split ? (int)row : split + total - 1 - (int)row;
+    const int dof = row < split ? row : split + total - 1 - row;
     if (dof >= p) {
         for (int j = 0; j < q; ++j) o[j] = T(0);
         return;
@@ -1656,17 +1655,17 @@ band_load_kernel(unsigned n, int p, int split, int total, int R, int q, int Ra,
 }
 
 // The workspace's columns back to y: slot a's to case cols[a], zero for the cases listed
-// from Ra on (inactive).  One thread per DOF and case.
+// from Ra on (inactive).  n DOFs and cases from DOF first on, one thread each.
 template <typename T, int Q>
 __global__ void __launch_bounds__(256)
-band_store_kernel(unsigned n, int split, int total, int R, int q, int Ra,
+band_store_kernel(unsigned n, int first, int split, int total, int R, int q, int Ra,
                   const int *__restrict__ cols, int ld, const T *__restrict__ w,
                   T *__restrict__ y) {
     const unsigned idx = blockIdx.x * 256u + threadIdx.x;
     if (idx >= n) return;
-    const unsigned dof = idx / (unsigned)R;
-    const int a = (int)(idx - dof * (unsigned)R);
-    const int row = (int)dof < split ? (int)dof : split + total - 1 - (int)dof;
+    const unsigned case_dof = idx / (unsigned)R;
+    const int dof = first + (int)case_dof, a = (int)(idx - case_dof * (unsigned)R);
+    const int row = dof < split ? dof : split + total - 1 - dof;
     T *o = y + ((size_t)dof * R + (cols ? cols[a] : a)) * q;
     const T *v = w + (size_t)row * ld + a * q;
     if (Q) {
@@ -1709,15 +1708,21 @@ int band_apply(BandPrec *bp, int R, int q, const T *minv, const T *x, T *y, hipS
     XT_TRY(bp->w2.reserve(es * (size_t)(nb + 1) * b * pad_cols(q * R)));
     T *w1 = bp->w1.as<T>(), *w2 = bp->w2.as<T>();
     const int total = nb * b, split = (nt + 1) * b;
-    const long long nload = (long long)total * Ra, nstore = (long long)bp->p * R;
-    XT_ARG(nload < (1LL << 32) - 256 && nstore < (1LL << 32) - 256, "band_apply: too many columns");
+    // (a launch holds fewer than 2^32 threads: more rows and cases take several)
+    auto in_launches = [](int rows, int cases, auto launch) {
+        const int most = std::max(1, (int)((1LL << 31) / cases));
+        for (int first = 0; first < rows; first += most)
+            launch(first, (long long)std::min(most, rows - first) * cases);
+    };
+    in_launches(total, Ra, [&](int first, long long n) {
 #define XT_LOAD(Q)                                                                             \
-    hipLaunchKernelGGL((band_load_kernel<T, Q>), dim3(ceil_div(nload, 256)), dim3(256), 0, s,   \
-                       (unsigned)nload, bp->p, split, total, R, q, Ra, dcols, ld, minv, x, w1)
-    if (q == 6) XT_LOAD(6);
-    else if (q == 3) XT_LOAD(3);
-    else XT_LOAD(0);
+    hipLaunchKernelGGL((band_load_kernel<T, Q>), dim3(ceil_div(n, 256)), dim3(256), 0, s,       \
+                       (unsigned)n, first, bp->p, split, total, R, q, Ra, dcols, ld, minv, x, w1)
+        if (q == 6) XT_LOAD(6);
+        else if (q == 3) XT_LOAD(3);
+        else XT_LOAD(0);
 #undef XT_LOAD
+    });
     XT_HIP(hipGetLastError());
     const long long bb = (long long)b * b, bk = (long long)b * kw, bc = (long long)b * ld;
     const T *Dl = bp->Dl[pi].as<T>(), *Du = bp->Du[pi].as<T>();
@@ -1874,13 +1879,15 @@ int band_apply(BandPrec *bp, int R, int q, const T *minv, const T *x, T *y, hipS
                  2.0 * (2.0 * nb * tri * c + 2.0 * (nb - 1) * gh * c));
     }
     XT_HIP(hipGetLastError());
+    in_launches(bp->p, R, [&](int first, long long n) {
 #define XT_STORE(Q)                                                                            \
-    hipLaunchKernelGGL((band_store_kernel<T, Q>), dim3(ceil_div(nstore, 256)), dim3(256), 0, s, \
-                       (unsigned)nstore, split, total, R, q, Ra, dcols, ld, (const T *)w1, y)
-    if (q == 6) XT_STORE(6);
-    else if (q == 3) XT_STORE(3);
-    else XT_STORE(0);
+    hipLaunchKernelGGL((band_store_kernel<T, Q>), dim3(ceil_div(n, 256)), dim3(256), 0, s,      \
+                       (unsigned)n, first, split, total, R, q, Ra, dcols, ld, (const T *)w1, y)
+        if (q == 6) XT_STORE(6);
+        else if (q == 3) XT_STORE(3);
+        else XT_STORE(0);
 #undef XT_STORE
+    });
     XT_HIP(hipGetLastError());
     return XT_OK;
 }
