@@ -133,3 +133,18 @@ def test_work_is_counted_on_the_band(dev, block, fp32):
     _, byts, flops, alg_bytes, alg_flops = (u.value for u in v)
     assert alg_flops == pytest.approx(flops, rel=1e-9)
     assert alg_bytes == pytest.approx(byts, rel=0.02)
+
+
+@pytest.mark.parametrize("row", [5, 300, 640, 700, 1271, 1280])
+def test_indefinite_row_is_named(dev, row):
+    """An uncoupled row with a negative diagonal (0-based; blocks of 128, the middle block
+    from 640 on) is named in K's order, whichever end its elimination starts from."""
+    from xtfem_amd.api import XtError
+    ia, ja, a = strip(106)
+    p = len(ia) - 1
+    assert p == 1284
+    rows = np.repeat(np.arange(p), np.diff(ia))
+    hit = (rows == row) | (ja - 1 == row)
+    a = np.where(hit, np.where(rows == ja - 1, -1.0, 0.0), a)
+    with pytest.raises(XtError, match=rf"code -3.*elimination of row {row}\)"):
+        dev.BandPreconditioner((ia, ja, a), block=128)

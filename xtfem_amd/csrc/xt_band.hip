@@ -923,7 +923,7 @@ chol_step_kernel(int b, int nt, int k, CholSides cs) {
             __syncthreads();
         }
     }
-    if (id == 0 && tid == 0 && sbad) S.info[0] = k * kCT + sbad;
+    if (id == 0 && tid == 0 && sbad && !S.info[0]) S.info[0] = k * kCT + sbad;   // (the first)
     double *wt = S.W + TS * t;
     if (t > 0) {
         for (int e = tid; e < HR * kCT; e += 64 * kCW) {
@@ -1428,11 +1428,15 @@ static int factor_dev(BandPrec &bp, const int *dia, const int *dja, const double
     std::vector<int> hinfo(nb + 1);
     XT_HIP(hipMemcpyAsync(hinfo.data(), ip, sizeof(int) * nb, hipMemcpyDeviceToHost, s));
     XT_HIP(hipStreamSynchronize(s));
-    for (int i = ft; i < nb; ++i)
-        if (hinfo[i] != 0) {
-            set_error("K is not positive definite (block %d, minor %d)", i, hinfo[i]);
+    for (int e = ft; e < nb; ++e) {   // the chains, then the middle block
+        const int i = e < nt ? e : e + 1 < nb ? e + 1 : nt;
+        if (hinfo[i] != 0) {   // (the bottom chain's rows run backwards)
+            const int r = i * b + hinfo[i] - 1;
+            set_error("K is not positive definite (elimination of row %d)",
+                      i <= nt ? r : (nt + 1 + nb) * b - 1 - r);
             return XT_E_SINGULAR;
         }
+    }
     // nothing can fail numerically from here on: the new blocks go into the factor's own
     // arrays (a full factorization's into new ones where those are missing or too small,
     // allocated before anything is overwritten); an apply still running on another stream
