@@ -33,3 +33,29 @@ def test_more_rows_and_cases_than_a_launch_holds():
         assert (y[r:r + 4096] == first[r:r + 4096, None]).all()
     del x, y
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("cases", [1, 7])
+def test_few_cases_take_one_launch_each_way(cases):
+    """The nodes of a captured apply on 12012 rows: a launch each way and those of the sweeps,
+    not one for every row."""
+    import ctypes as C
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+    from xtfem_amd import device
+    from xtfem_amd._lib import check, lib
+    hip = lib()                           # (its symbols include those of the runtime it links)
+    pr = device.BandPreconditioner(strip(1000), block=512)
+    x = torch.ones((pr.p, cases), device="cuda", dtype=torch.float64)
+    y = torch.empty_like(x)
+    pr.apply(None, x, y, cases, q=1)      # (sizes the workspace)
+    torch.cuda.synchronize()
+    s, graph, n = C.c_void_p(), C.c_void_p(), C.c_size_t(0)
+    assert hip.hipStreamCreate(C.byref(s)) == 0
+    assert hip.hipStreamBeginCapture(s, 1) == 0            # thread-local
+    check(lib().xt_prec_apply(pr.h, cases, 1, None, x.data_ptr(), y.data_ptr(), 0, s))
+    assert hip.hipStreamEndCapture(s, C.byref(graph)) == 0
+    assert hip.hipGraphGetNodes(graph, None, C.byref(n)) == 0
+    assert hip.hipGraphDestroy(graph) == 0 and hip.hipStreamDestroy(s) == 0
+    assert 4 <= n.value < 100

@@ -1714,9 +1714,9 @@ int band_apply(BandPrec *bp, int R, int q, const T *minv, const T *x, T *y, hipS
     const int total = nb * b, split = (nt + 1) * b;
     // (a launch holds fewer than 2^32 threads: more rows and cases take several)
     auto in_launches = [](int rows, int cases, auto launch) {
-        const int most = std::max(1, (int)((1LL << 31) / cases));
-        for (int first = 0; first < rows; first += most)
-            launch(first, (long long)std::min(most, rows - first) * cases);
+        const long long most = std::max(1LL, (1LL << 31) / cases);   // rows of a launch
+        for (long long first = 0; first < rows; first += most)
+            launch((int)first, std::min(most, rows - first) * cases);
     };
     in_launches(total, Ra, [&](int first, long long n) {
 #define XT_LOAD(Q)                                                                             \
