@@ -1224,12 +1224,12 @@ def main():
         fp32_only = True      # FP64 shifted factors of the panel would not fit beside the rest
     else:
         prob = Problem(*(args.grid or [100, 46, 4]), args.notch, R, args.cases_kind)
+        fp32_only = False
     if args.spmm_only:
         from xtfem_amd import device
         op = device.KronOperator([prob.Kb, prob.Mb], q=6)
         print(json.dumps(dict(workload=prob.describe(), kron_spmm=spmm_legs(op, prob.p))))
         return
-        fp32_only = False
     t_asm = time.perf_counter() - t0
     op, pr, sinfo = setup_solver(prob, args, fp32_only)
     print(f"# setup: p={prob.p} assembly {t_asm:.1f}s, {sinfo}", file=sys.stderr, flush=True)
