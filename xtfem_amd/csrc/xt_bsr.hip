@@ -26,11 +26,19 @@
 // wave-uniform without lanes left over.
 //
 // Storage ("node groups", kron_group_kernel, several load cases on enough nodes): kG
-// consecutive nodes share the sorted union of their neighbours; the blocks stand
-// neighbour by neighbour (only the couplings that exist), so a wave whose lanes are
-// columns reads each neighbour's rows of X once for all nodes of the group.  The values of a
-// precision are copied from the slices by the first apply that takes the groups, and kept
-// up to date from then on: a program with one load case never holds them.
+// consecutive nodes share the union of their neighbours; the blocks stand neighbour by
+// neighbour (only the couplings that exist), so a wave whose lanes are columns reads each
+// neighbour's rows of X once for all nodes of the group.  The order is far nodes, near ones
+// (within a third of the way to the lowest neighbour), the group's own, each ascending: the
+// kernel adds product by product (the slices a block's three together), and with the large
+// diagonal block before half of the products the sums rounded more often than the slices'.
+// Error in the 2-norm, random X, against more bits: slices 1.12e-7 (FP32) and 2.1e-16 (FP64),
+// groups in sorted order 1.37e-7 and 2.6e-16, in this order 8.1e-8 and 1.5e-16.
+// Time of 145323 nodes, 32 cases, FP64: sorted 685 us, so 697, own nodes last and the others
+// sorted 722 (FP32 389, 391, 395); 23735 nodes 117, 121, 118 (80, 80, 80); a block's three
+// products summed before they are added (error as the slices') 715 (430) and 142 (93).
+// The values of a precision are copied from the slices by the first apply that takes the
+// groups, and kept up to date from then on: a program with one load case never holds them.
 //
 // The path is for q = 6 temporal functions (three quadratic temporal nodes, each with a
 // sine enrichment: 2*nnte, main3d.f90:172).
@@ -138,33 +146,49 @@ int bsr_build(int p, const int *krp, const int *kci, const double *kv, const int
     std::vector<int> bcol(nb);
     std::vector<int> pos(nn, -1);   // entry of column node b in the row
     std::vector<int> kmap(krp[p]), mmap(mrp[p]), gof(nb, -1);
-    // groups: merge the kG sorted neighbour lists; gpos: block of each of row a's neighbours,
-    // from cfirst[a] on
+    // groups: merge the kG sorted neighbour lists, then far, near and own nodes; gpos: block of
+    // each of row a's neighbours, from cfirst[a] on
     const int ngroups = ceil_div(nn, kG);
     std::vector<int> gptr(ngroups + 1, 0), gblk(ngroups + 1, 0), gnbr;
     std::vector<int> cfirst(nn + 1, 0);
     for (int a = 0; a < nn; ++a) cfirst[a + 1] = cfirst[a] + (int)cols[a].size();
     std::vector<int> gpos(cfirst[nn]);
     {
+        struct Neighbour {
+            int m, mask, at[kG];   // column node, coupled nodes of the group, their entries
+        };
+        std::vector<Neighbour> u;
         int blk = 0;
         for (int s = 0; s < ngroups; ++s) {
             const int a0 = s * kG, na = std::min(kG, nn - a0);
-            int at[kG] = {};
-            gblk[s] = blk;
+            Neighbour n{};
+            u.clear();
             for (;;) {
-                int m = nn;
+                n.m = nn;
                 for (int i = 0; i < na; ++i)
-                    if (at[i] < (int)cols[a0 + i].size()) m = std::min(m, cols[a0 + i][at[i]]);
-                if (m == nn) break;
-                int e = (blk - gblk[s]) << 4;
+                    if (n.at[i] < (int)cols[a0 + i].size())
+                        n.m = std::min(n.m, cols[a0 + i][n.at[i]]);
+                if (n.m == nn) break;
+                n.mask = 0;
                 for (int i = 0; i < na; ++i)
-                    if (at[i] < (int)cols[a0 + i].size() && cols[a0 + i][at[i]] == m) {
-                        gpos[cfirst[a0 + i] + at[i]++] = blk++;
-                        e |= 1 << i;
-                    }
-                gnbr.push_back(m);
-                gnbr.push_back(e);
+                    if (n.at[i] < (int)cols[a0 + i].size() && cols[a0 + i][n.at[i]] == n.m)
+                        n.mask |= 1 << i;
+                u.push_back(n);
+                for (int i = 0; i < na; ++i) n.at[i] += n.mask >> i & 1;
             }
+            gblk[s] = blk;
+            const int third = std::max(a0 - u[0].m, 0) / 3;
+            auto kind = [&](int m) {
+                return m >= a0 && m < a0 + na ? 2 : m >= a0 - third && m < a0 + na + third ? 1 : 0;
+            };
+            for (int k = 0; k < 3; ++k)
+                for (const Neighbour &v : u) {
+                    if (kind(v.m) != k) continue;
+                    gnbr.push_back(v.m);
+                    gnbr.push_back((blk - gblk[s]) << 4 | v.mask);
+                    for (int i = 0; i < na; ++i)
+                        if (v.mask >> i & 1) gpos[cfirst[a0 + i] + v.at[i]] = blk++;
+                }
             gptr[s + 1] = (int)(gnbr.size() / 2);
         }
         gblk[ngroups] = blk;
@@ -605,7 +629,7 @@ static __device__ inline void block_row(float kv, const float (&x)[3][3], float 
 // cache), 687 here.  Block values through scalar loads, a column or three a lane: 1460,
 // 1160 (a dependent scalar load a block); by LDS reads of 16 bytes at one address: 880;
 // one neighbour ahead, one group a wave: 760.  What is left: the rows of X reach a CU at 9 TB/s over
-// all CUs with half of them missing the L2 (the vector cache waits on about 80 lines of 128
+// all CUs with 60 % of them missing the L2 (the vector cache waits on about 80 lines of 128
 // bytes at 600 cycles each), and the clock sinks to 1.7 - 1.9 GHz.  Groups taken in strips of
 // the section rather than in order halve the misses for 10 % of the time, but need the
 // section's width, which the pattern does not give.
