@@ -1070,8 +1070,7 @@ def cpu_damage_sample(ne_s=1000, nip=2560):
 
 
 # rocprofv3 --pmc summaries (FETCH_SIZE / WRITE_SIZE per launch, calibrated on a plain
-# copy), per workload; none is committed for the current kernels (the counter runs
-# crashed in the profiler's initialisation on this image), so traffic reads null
+# copy), per workload
 PMC_SUMMARY = {"panel": os.path.join(ROOT, "profiles", "band_sweep_panel_32cases_pmc.md"),
                "plate": os.path.join(ROOT, "profiles", "band_sweep_notched_plate_32cases_pmc.md")}
 

@@ -34,9 +34,10 @@
 // diagonal block before half of the products the sums rounded more often than the slices'.
 // Error in the 2-norm, random X, against more bits: slices 1.12e-7 (FP32) and 2.1e-16 (FP64),
 // groups in sorted order 1.37e-7 and 2.6e-16, in this order 8.1e-8 and 1.5e-16.
-// Time of 145323 nodes, 32 cases, FP64: sorted 685 us, so 697, own nodes last and the others
-// sorted 722 (FP32 389, 391, 395); 23735 nodes 117, 121, 118 (80, 80, 80); a block's three
-// products summed before they are added (error as the slices') 715 (430) and 142 (93).
+// Time of 145323 nodes, 32 cases, FP64: sorted 685 us, so 697 (5 % more of the reads miss the
+// L2), own nodes last and the others sorted 722 (FP32 389, 391, 395); 23735 nodes 117, 121,
+// 118 (80, 80, 80); a block's three products summed before they are added (error as the
+// slices') 715 (430) and 142 (93).
 // The values of a precision are copied from the slices by the first apply that takes the
 // groups, and kept up to date from then on: a program with one load case never holds them.
 //
@@ -626,13 +627,13 @@ static __device__ inline void block_row(float kv, const float (&x)[3][3], float 
 //
 // 145323 nodes (241 x 201 x 3), 32 cases, FP64: 1704 us by the slice kernel (every lane loads
 // its node's block and its neighbours' rows: 15 loads an entry through the CU's vector
-// cache), 687 here.  Block values through scalar loads, a column or three a lane: 1460,
-// 1160 (a dependent scalar load a block); by LDS reads of 16 bytes at one address: 880;
-// one neighbour ahead, one group a wave: 760.  What is left: the rows of X reach a CU at 9 TB/s over
-// all CUs with 60 % of them missing the L2 (the vector cache waits on about 80 lines of 128
-// bytes at 600 cycles each), and the clock sinks to 1.7 - 1.9 GHz.  Groups taken in strips of
-// the section rather than in order halve the misses for 10 % of the time, but need the
-// section's width, which the pattern does not give.
+// cache), 687 here (699 since each group's own nodes come last).  Block values through scalar
+// loads, a column or three a lane: 1460, 1160 (a dependent scalar load a block); by LDS reads
+// of 16 bytes at one address: 880; one neighbour ahead, one group a wave: 760.  What is left:
+// the rows of X reach a CU at 8.8 TB/s over all CUs with 63 % of them missing the L2 (the
+// vector cache waits on about 80 lines of 128 bytes at 660 cycles each), and the clock sinks
+// to 1.7 - 1.9 GHz.  Groups taken in strips of the section rather than in order halve the
+// misses for 10 % of the time, but need the section's width, which the pattern does not give.
 template <typename T, int LPG>
 struct GroupGeom {
     static constexpr int CH = LPG >= 48 ? 6 : 3;              // neighbours of a chunk
